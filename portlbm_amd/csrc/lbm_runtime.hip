@@ -19,6 +19,7 @@
 
 #include "lbm_device.hpp"
 #include "lbm_error.hpp"
+#include "lbm_march.hpp"
 #include "lbm_setup.hpp"
 
 using namespace lbm_dev;
@@ -70,6 +71,9 @@ struct lbm_ctx
     size_t elem;          // bytes per stored population
     void *lat[2] = {nullptr, nullptr};
     int cur = 0;          // index of the source lattice
+    int uy_cur = 0;       // half of uycol that the next step reads
+    int cus = 0;
+    bool march = false;   // nptl / lptl: several steps per launch (k_march)
     int8_t *phase = nullptr;
     uint16_t *code = nullptr;
     double *res = nullptr;    // 4 * D: rho, jx, jy, |j|
@@ -1587,9 +1591,8 @@ struct Impl
         p.jx = c->res + c->D;
         p.jy = c->res + 2 * size_t(c->D);
         p.jabs = c->res + 3 * size_t(c->D);
-        const int parity = int(c->iteration & 1u);
-        p.uy_in = c->uycol + size_t(parity) * c->V;
-        p.uy_out = c->uycol + size_t(1 - parity) * c->V;
+        p.uy_in = c->uycol + size_t(c->uy_cur) * c->V;
+        p.uy_out = c->uycol + size_t(1 - c->uy_cur) * c->V;
         p.omega = host_omega(c->desc.storage, c->desc.relaxation_time);
         p.ref_in = c->ref[c->ref_cur];
         p.ref_out = c->ref_switch ? c->ref[1 - c->ref_cur] : p.ref_in;
@@ -1755,8 +1758,24 @@ struct Impl
         LBM_HIP_TRY(hipGetLastError());
         if (c->two_lattice)
             c->cur ^= 1;
+        c->uy_cur ^= 1;
         c->iteration++;
         end_reference(c);
+        return LBM_OK;
+    }
+
+    // n time steps in one launch (march_steps says how many may go together)
+    static int march(lbm_ctx *c, uint32_t n, bool macros)
+    {
+        MarchParams m{};
+        m.p = params(c, macros);
+        for (uint32_t k = 0; k < n; ++k)
+            m.sr[k] = c->desc.rounding == LBM_ROUND_STOCHASTIC ? (step_seed(c->iteration + k) | 1u) : 0u;
+        march_launch(L, S, n, m, c->cus, c->stream);
+        LBM_HIP_TRY(hipGetLastError());
+        c->cur ^= 1;
+        c->uy_cur ^= 1;
+        c->iteration += n;
         return LBM_OK;
     }
 
@@ -1790,6 +1809,7 @@ struct Impl
             LBM_HIP_TRY(hipGetLastError());
             if (c->two_lattice)
                 c->cur ^= 1;
+            c->uy_cur ^= 1;
             c->iteration++;
             end_reference(c);
             return LBM_OK;
@@ -1903,13 +1923,15 @@ struct VTable
     int (*equilibrium)(lbm_ctx *, const double *, const double *, const double *);
     int (*reduce)(lbm_ctx *, int, double *);
     int (*split)(lbm_ctx *, int, double *);
+    int (*march)(lbm_ctx *, uint32_t, bool);
 };
 
 template <int L, int S>
 static VTable make_vtable()
 {
     return VTable{&Impl<L, S>::step, &Impl<L, S>::init, &Impl<L, S>::decode, &Impl<L, S>::encode,
-                  &Impl<L, S>::equilibrium, &Impl<L, S>::reduce, &Impl<L, S>::split};
+                  &Impl<L, S>::equilibrium, &Impl<L, S>::reduce, &Impl<L, S>::split,
+                  &Impl<L, S>::march};
 }
 
 template <int L>
@@ -1982,6 +2004,8 @@ int lbm_device_name(char *buf, size_t len)
     buf[n] = '\0';
     return LBM_OK;
 }
+
+static uint64_t march_min_nodes(size_t elem) { return elem == 8 ? 300000u : (elem == 4 ? 1200000u : 6000000u); }
 
 static int validate_desc(const lbm_desc *d)
 {
@@ -2157,6 +2181,7 @@ int lbm_create(const lbm_desc *desc, lbm_ctx **out)
     // 1024, 3844 tiles, 154 / 174).
     size_t side_bytes = 0;
     int cus = 0;
+    bool march = false;   // nptl / lptl: several steps per launch (k_march)
     {
         int dev = 0;
         CREATE_TRY(hipGetDevice(&dev));
@@ -2202,6 +2227,10 @@ int lbm_create(const lbm_desc *desc, lbm_ctx **out)
         else
             c->tile_staged = false;  // the block kernels with the reference's refresh
     }
+    c->cus = cus;
+    // nptl and lptl go through the lattice once for up to four steps when it
+    // is large enough to fill the chip with marching waves
+    c->march = c->two_lattice && uint64_t(c->Hx - 2u) * (c->Vx - 2u) >= march_min_nodes(c->elem);
     CREATE_TRY(hipMalloc(&c->lat[0], lat_bytes + std::max<size_t>(64, side_bytes)));
     if (c->two_lattice)
         CREATE_TRY(hipMalloc(&c->lat[1], lat_bytes + 64));
@@ -2283,6 +2312,7 @@ int lbm_init_populations(lbm_ctx *c)
     if (!c->phase_set)
         return fail(LBM_ERR_STATE, "lbm_init_populations: lbm_set_phase must come first");
     c->cur = 0;
+    c->uy_cur = 0;
     c->side_valid = false;
     if (int rc = reset_reference(c))
         return rc;
@@ -2325,6 +2355,45 @@ int lbm_get_node_codes(lbm_ctx *c, uint16_t *codes, size_t n)
     return LBM_OK;
 }
 
+// How many of the next `left` steps go into one launch: none past the next
+// step whose results are written, none across a change of the 16-bit forms'
+// rho_ref (that step runs alone).
+static uint32_t fused_steps(const lbm_ctx *c, uint32_t left, uint32_t frame_interval)
+{
+    if (!c->march)
+        return 1;
+    uint32_t n = left;
+    if (frame_interval)
+        n = std::min(n, uint32_t(frame_interval - c->iteration % frame_interval));
+    if (c->ref[0])
+    {
+        const uint32_t at = uint32_t(c->iteration % kRefInterval);
+        n = at == 0u && c->iteration ? 1u : std::min(n, kRefInterval - at);
+    }
+    // 4, 4, ..., and a remainder of one or two shared with the four before it
+    return n <= kMarchMaxSteps ? n : (n < 2u * kMarchMaxSteps - 1u ? 3u : kMarchMaxSteps);
+}
+
+// The next launch of a run: how many steps, and what its last one writes.
+struct Chunk
+{
+    uint32_t steps;
+    bool frame, macros;
+};
+
+static Chunk next_chunk(const lbm_ctx *c, uint32_t left, uint32_t frame_interval)
+{
+    const uint32_t n = fused_steps(c, left, frame_interval);
+    const uint64_t last = c->iteration + n - 1u;
+    const bool frame = frame_interval ? (last % frame_interval == frame_interval - 1u) : false;
+    return Chunk{n, frame, frame || n == left};
+}
+
+static int run_chunk(lbm_ctx *c, const VTable &vt, const Chunk &k)
+{
+    return k.steps > 1u ? vt.march(c, k.steps, k.macros) : vt.step(c, k.macros);
+}
+
 int lbm_run(lbm_ctx *c, uint32_t steps, uint32_t frame_interval)
 {
     if (!c)
@@ -2333,13 +2402,12 @@ int lbm_run(lbm_ctx *c, uint32_t steps, uint32_t frame_interval)
         return fail(LBM_ERR_STATE, "lbm_run: call lbm_init_populations first");
     const VTable vt = vtable(c);
     LBM_HIP_TRY(hipEventRecord(c->ev0, c->stream));
-    for (uint32_t i = 0; i < steps; ++i)
+    for (uint32_t left = steps; left;)
     {
-        const uint64_t it = c->iteration;
-        const bool frame = frame_interval ? (it % frame_interval == frame_interval - 1u) : false;
-        const bool macros = frame || i + 1u == steps;
-        if (int rc = vt.step(c, macros))
+        const Chunk k = next_chunk(c, left, frame_interval);
+        if (int rc = run_chunk(c, vt, k))
             return rc;
+        left -= k.steps;
     }
     LBM_HIP_TRY(hipEventRecord(c->ev1, c->stream));
     LBM_HIP_TRY(hipEventSynchronize(c->ev1));
@@ -2366,20 +2434,19 @@ int lbm_run_frames(lbm_ctx *c, uint32_t steps, uint32_t frame_interval)
     const VTable vt = vtable(c);
     uint64_t last_frame = ~0ull;
     LBM_HIP_TRY(hipEventRecord(c->ev0, c->stream));
-    for (uint32_t i = 0; i < steps; ++i)
+    for (uint32_t left = steps; left;)
     {
-        const uint64_t it = c->iteration;
-        const bool frame = frame_interval ? (it % frame_interval == frame_interval - 1u) : false;
-        const bool macros = frame || i + 1u == steps;
-        if (macros && c->copy_pending)
+        const Chunk k = next_chunk(c, left, frame_interval);
+        if (k.macros && c->copy_pending)
         {
             // the results must not change under the copy still reading them
             LBM_HIP_TRY(hipStreamWaitEvent(c->stream, c->ev_copied, 0));
             c->copy_pending = false;
         }
-        if (int rc = vt.step(c, macros))
+        if (int rc = run_chunk(c, vt, k))
             return rc;
-        if (frame)
+        left -= k.steps;
+        if (k.frame)
         {
             LBM_HIP_TRY(hipEventRecord(c->ev_frame, c->stream));
             LBM_HIP_TRY(hipStreamWaitEvent(c->copy_stream, c->ev_frame, 0));
@@ -2387,7 +2454,7 @@ int lbm_run_frames(lbm_ctx *c, uint32_t steps, uint32_t frame_interval)
                                        c->copy_stream));
             LBM_HIP_TRY(hipEventRecord(c->ev_copied, c->copy_stream));
             c->copy_pending = true;
-            last_frame = it;
+            last_frame = c->iteration - 1u;
         }
     }
     LBM_HIP_TRY(hipEventRecord(c->ev1, c->stream));
@@ -2552,8 +2619,14 @@ int lbm_get_state(lbm_ctx *c, void *buf, size_t bytes)
     LBM_HIP_TRY(hipStreamSynchronize(c->stream));
     for (uint32_t l = 0; l < lattices; ++l, off += lat_bytes)
         LBM_HIP_TRY(hipMemcpy(out + off, c->lat[l], lat_bytes, hipMemcpyDeviceToHost));
-    LBM_HIP_TRY(hipMemcpy(out + off, c->uycol, 2ull * c->V * sizeof(double), hipMemcpyDeviceToHost));
-    off += 2ull * c->V * sizeof(double);
+    // outlet history: the half that the next step reads at the place of the
+    // iteration's parity
+    const size_t half = size_t(c->V) * sizeof(double);
+    const size_t at = (c->iteration & 1u) ? half : 0u;
+    LBM_HIP_TRY(hipMemcpy(out + off + at, c->uycol + size_t(c->uy_cur) * c->V, half, hipMemcpyDeviceToHost));
+    LBM_HIP_TRY(hipMemcpy(out + off + (half - at), c->uycol + size_t(1 - c->uy_cur) * c->V, half,
+                          hipMemcpyDeviceToHost));
+    off += 2u * half;
     LBM_HIP_TRY(hipMemcpy(out + off, c->res, 4ull * c->D * sizeof(double), hipMemcpyDeviceToHost));
     off += 4ull * c->D * sizeof(double);
     if (c->ref_len)
@@ -2596,6 +2669,7 @@ int lbm_set_state(lbm_ctx *c, const void *buf, size_t bytes)
     c->iteration = iteration;
     c->frame_iteration = ~0ull;
     c->cur = int(cur);
+    c->uy_cur = int(iteration & 1u);
     c->snap_valid = false;
     c->side_valid = false;
     return LBM_OK;
