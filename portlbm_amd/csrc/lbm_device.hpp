@@ -465,6 +465,45 @@ __device__ __forceinline__ void collide(C f[9], C omega, C &rho, C &jx, C &jy, C
         f[d] = -omega * (f[d] - feq[d]) + f[d];
 }
 
+// collide<C, kPromote, kFull> where every population is finite: the terms that
+// kFull keeps (x + 0 f) change nothing then.  A population that is not makes
+// the density infinite or NaN, and the wave takes the full sums.
+template <class C, bool kPromote, bool kFull>
+__device__ __forceinline__ void collide_node(C f[9], C omega, C &rho, C &jx, C &jy, C &usq)
+{
+    using A = std::conditional_t<kPromote, double, C>;
+    rho = f[0];
+#pragma unroll
+    for (int d = 1; d < 9; ++d)
+        rho += f[d];
+    if constexpr (kFull)
+    {
+        if (__builtin_expect(__any(!__builtin_isfinite(rho)), 0))
+        {
+            collide<C, kPromote, true>(f, omega, rho, jx, jy, usq);
+            return;
+        }
+    }
+    jx = ((((-f[0] + f[2]) - f[3]) + f[5]) - f[6]) + f[8];
+    jy = ((((-f[0] - f[1]) - f[2]) + f[6]) + f[7]) + f[8];
+    usq = jx * jx + jy * jy;
+    const A s = A(1.5) * A(usq);
+    C feq[9];
+#pragma unroll
+    for (int d = 0; d < 4; ++d)
+    {
+        const C cu = c_dot<C, false>(d, jx, jy);
+        const C t = C(3) * cu;
+        const A q = A(4.5) * A(cu) * A(cu);
+        feq[d] = C(A(weight<C>(d)) * (A(rho + t) + q - s));
+        feq[8 - d] = C(A(weight<C>(8 - d)) * (A(rho - t) + q - s));
+    }
+    feq[4] = C(A(weight<C>(4)) * (A(rho) - s));
+#pragma unroll
+    for (int d = 0; d < 9; ++d)
+        f[d] = -omega * (f[d] - feq[d]) + f[d];
+}
+
 // In the stream layout every store instruction of a wave writes whole
 // contiguous segments, and the populations are written with non-temporal
 // stores: nothing reads them again within the step, so they should not

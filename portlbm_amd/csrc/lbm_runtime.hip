@@ -15,6 +15,7 @@
 #include <cstdio>
 #include <cstring>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "lbm_device.hpp"
@@ -73,7 +74,9 @@ struct lbm_ctx
     int cur = 0;          // index of the source lattice
     int uy_cur = 0;       // half of uycol that the next step reads
     int cus = 0;
-    bool march = false;   // nptl / lptl: several steps per launch (k_march)
+    uint32_t fuse_steps = 1;  // steps per launch, at most
+    bool fuse_in_tiles = false;  // by k_tile_steps on regions of fuse_tile, else by k_march
+    TileShape fuse_tile = TileShape::k32x32;
     int8_t *phase = nullptr;
     uint16_t *code = nullptr;
     double *res = nullptr;    // 4 * D: rho, jx, jy, |j|
@@ -87,9 +90,14 @@ struct lbm_ctx
     hipStream_t stream = nullptr;
     // asynchronous frame copies (lbm_run_frames; created on first use)
     hipStream_t copy_stream = nullptr;
-    hipEvent_t ev_frame = nullptr, ev_copied = nullptr;
+    hipEvent_t ev_frame = nullptr, ev_copied[2] = {nullptr, nullptr};
     double *frame_host = nullptr;  // pinned, 4 * D
-    bool copy_pending = false;     // a copy of the results may still be reading them
+    // Frames write two result arrays in turn, so that the steps to the next
+    // frame need not wait for the copy of the last one; c->res is the latest.
+    double *res_other = nullptr;   // allocated by the first lbm_run_frames; none if memory ran out
+    bool res_other_valid = false;  // its nodes that are not fluid hold what c->res holds
+    int res_half = 0;              // which of the two c->res is
+    bool copy_pending[2] = {false, false};  // a copy may still be reading it
     uint64_t frame_iteration = ~0ull;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     uint64_t iteration = 0;
@@ -1448,6 +1456,20 @@ __global__ void k_copy16(const uint4 *__restrict__ a, uint4 *__restrict__ b, siz
         b[i] = a[i];
 }
 
+// A frame to pinned host memory.  As a kernel the copy follows the frame step
+// and releases the next one through queue packets alone; through the copy
+// engine a 512 x 128 lattice with a frame every 10 steps took 126 us per
+// frame, with this kernel 63 (2 MB: 37 us at the link's 57 GB/s).  A few
+// blocks fill the link: 16 / 64 / 256 / 1024 of them gave 3.14 / 3.32 / 3.26 /
+// 3.26 ms for 50 frames of 512 x 128 and 123 / 125 / 136 / 140 ms for 50 of
+// 4096 x 1024 (copy engine: 124).
+constexpr uint32_t FRAME_COPY_BLOCKS = 16;
+__global__ __launch_bounds__(256) void k_copy_frame(const uint4 *__restrict__ a, uint4 *__restrict__ b, size_t n)
+{
+    for (size_t i = size_t(blockIdx.x) * 256u + threadIdx.x; i < n; i += size_t(gridDim.x) * 256u)
+        b[i] = a[i];
+}
+
 // ---------------------------------------------------------------------------
 // split step (the reference's debug kernels, nptl_kernels.hpp:48-295): one
 // launch per pass over every physical place, the populations between passes
@@ -1764,14 +1786,17 @@ struct Impl
         return LBM_OK;
     }
 
-    // n time steps in one launch (march_steps says how many may go together)
-    static int march(lbm_ctx *c, uint32_t n, bool macros)
+    // n time steps in one launch (fused_steps says how many may go together)
+    static int fused(lbm_ctx *c, uint32_t n, bool macros)
     {
         MarchParams m{};
         m.p = params(c, macros);
         for (uint32_t k = 0; k < n; ++k)
             m.sr[k] = c->desc.rounding == LBM_ROUND_STOCHASTIC ? (step_seed(c->iteration + k) | 1u) : 0u;
-        march_launch(L, S, n, m, c->cus, c->stream);
+        if (c->fuse_in_tiles)
+            tile_launch(L, S, n, c->fuse_tile, m, c->stream);
+        else
+            march_launch(L, S, n, m, c->cus, c->stream);
         LBM_HIP_TRY(hipGetLastError());
         c->cur ^= 1;
         c->uy_cur ^= 1;
@@ -1923,7 +1948,7 @@ struct VTable
     int (*equilibrium)(lbm_ctx *, const double *, const double *, const double *);
     int (*reduce)(lbm_ctx *, int, double *);
     int (*split)(lbm_ctx *, int, double *);
-    int (*march)(lbm_ctx *, uint32_t, bool);
+    int (*fused)(lbm_ctx *, uint32_t, bool);
 };
 
 template <int L, int S>
@@ -1931,7 +1956,7 @@ static VTable make_vtable()
 {
     return VTable{&Impl<L, S>::step, &Impl<L, S>::init, &Impl<L, S>::decode, &Impl<L, S>::encode,
                   &Impl<L, S>::equilibrium, &Impl<L, S>::reduce, &Impl<L, S>::split,
-                  &Impl<L, S>::march};
+                  &Impl<L, S>::fused};
 }
 
 template <int L>
@@ -2005,7 +2030,30 @@ int lbm_device_name(char *buf, size_t len)
     return LBM_OK;
 }
 
-static uint64_t march_min_nodes(size_t elem) { return elem == 8 ? 300000u : (elem == 4 ? 1200000u : 6000000u); }
+// How nptl and lptl put several steps into one launch.  Small lattices are
+// bound by the launch itself and then by the latency of a step: blocks hold a
+// region of nodes in LDS for several steps (k_tile_steps), the region small
+// enough that every compute unit gets one.  Large lattices are bound by HBM:
+// marching waves read each row once (k_march).  us per step on porous
+// channels (FP64 stream / FP32 stream / FP16 collision), one step per launch,
+// then the shapes around the choice:
+//   256 x 64     3.8 / 3.6 / 4.6     16x16 T 5: 1.25 / 1.23 / 1.45    32x16 T 6: 1.42 / 1.30 / 1.44
+//   512 x 128    4.5 / 3.8 / 5.0     32x32 T 6: 2.12 / 1.75 / 1.73    16x16 T 5: 2.41 / 2.04 / 1.99
+//   1024 x 256   10.2 / 6.1 / 6.3    32x32 T 5: 4.69 / 3.73 / 3.65    32x16 T 4: 4.38 / 3.82 / 3.90
+//   2048 x 512   29.5 / 16.1 / 16.3  32x16 T 4: 12.6 / 10.7 / 11.1    march:     14.6 / 13.0 / 20.3
+//   4096 x 1024  112 / 55.8 / 48.9   32x16 T 4: 59.0 / 42.9 / 38.7    march:     45.4 / 32.7 / 37.5
+static void plan_fusion(lbm_ctx *c)
+{
+    const uint64_t nodes = uint64_t(c->Hx - 2u) * (c->Vx - 2u);
+    if (nodes >= (c->elem == 8 ? 1500000u : (c->elem == 4 ? 2000000u : 3500000u)))
+    {
+        c->fuse_steps = kMarchMaxSteps;
+        return;
+    }
+    c->fuse_in_tiles = true;
+    c->fuse_tile = nodes <= 36000u ? TileShape::k16x16 : (nodes <= 500000u ? TileShape::k32x32 : TileShape::k32x16);
+    c->fuse_steps = nodes <= 36000u ? 5u : (nodes <= 130000u ? 6u : (nodes <= 500000u ? 5u : 4u));
+}
 
 static int validate_desc(const lbm_desc *d)
 {
@@ -2065,6 +2113,7 @@ void lbm_destroy(lbm_ctx *c)
     (void)hipFree(c->phase);
     (void)hipFree(c->code);
     (void)hipFree(c->res);
+    (void)hipFree(c->res_other);
     (void)hipFree(c->uycol);
     (void)hipFree(c->snap);
     (void)hipFree(c->pass);
@@ -2085,8 +2134,9 @@ void lbm_destroy(lbm_ctx *c)
     }
     if (c->ev_frame)
         (void)hipEventDestroy(c->ev_frame);
-    if (c->ev_copied)
-        (void)hipEventDestroy(c->ev_copied);
+    for (hipEvent_t e : c->ev_copied)
+        if (e)
+            (void)hipEventDestroy(e);
     if (c->frame_host)
         (void)hipHostFree(c->frame_host);
     if (c->stream)
@@ -2181,7 +2231,9 @@ int lbm_create(const lbm_desc *desc, lbm_ctx **out)
     // 1024, 3844 tiles, 154 / 174).
     size_t side_bytes = 0;
     int cus = 0;
-    bool march = false;   // nptl / lptl: several steps per launch (k_march)
+    uint32_t fuse_steps = 1;  // steps per launch, at most
+    bool fuse_in_tiles = false;  // by k_tile_steps on regions of fuse_tile, else by k_march
+    TileShape fuse_tile = TileShape::k32x32;
     {
         int dev = 0;
         CREATE_TRY(hipGetDevice(&dev));
@@ -2228,9 +2280,8 @@ int lbm_create(const lbm_desc *desc, lbm_ctx **out)
             c->tile_staged = false;  // the block kernels with the reference's refresh
     }
     c->cus = cus;
-    // nptl and lptl go through the lattice once for up to four steps when it
-    // is large enough to fill the chip with marching waves
-    c->march = c->two_lattice && uint64_t(c->Hx - 2u) * (c->Vx - 2u) >= march_min_nodes(c->elem);
+    if (c->two_lattice)
+        plan_fusion(c);
     CREATE_TRY(hipMalloc(&c->lat[0], lat_bytes + std::max<size_t>(64, side_bytes)));
     if (c->two_lattice)
         CREATE_TRY(hipMalloc(&c->lat[1], lat_bytes + 64));
@@ -2276,6 +2327,7 @@ int lbm_set_phase(lbm_ctx *c, const int8_t *phase, size_t n)
     LBM_HIP_TRY(hipStreamSynchronize(c->stream));
     c->phase_set = true;
     c->initialized = false;
+    c->res_other_valid = false;
     return LBM_OK;
 }
 
@@ -2360,7 +2412,7 @@ int lbm_get_node_codes(lbm_ctx *c, uint16_t *codes, size_t n)
 // rho_ref (that step runs alone).
 static uint32_t fused_steps(const lbm_ctx *c, uint32_t left, uint32_t frame_interval)
 {
-    if (!c->march)
+    if (c->fuse_steps < 2u)
         return 1;
     uint32_t n = left;
     if (frame_interval)
@@ -2370,8 +2422,9 @@ static uint32_t fused_steps(const lbm_ctx *c, uint32_t left, uint32_t frame_inte
         const uint32_t at = uint32_t(c->iteration % kRefInterval);
         n = at == 0u && c->iteration ? 1u : std::min(n, kRefInterval - at);
     }
-    // 4, 4, ..., and a remainder of one or two shared with the four before it
-    return n <= kMarchMaxSteps ? n : (n < 2u * kMarchMaxSteps - 1u ? 3u : kMarchMaxSteps);
+    // as few launches as there can be, of nearly the same length
+    const uint32_t launches = (n + c->fuse_steps - 1u) / c->fuse_steps;
+    return (n + launches - 1u) / launches;
 }
 
 // The next launch of a run: how many steps, and what its last one writes.
@@ -2391,7 +2444,7 @@ static Chunk next_chunk(const lbm_ctx *c, uint32_t left, uint32_t frame_interval
 
 static int run_chunk(lbm_ctx *c, const VTable &vt, const Chunk &k)
 {
-    return k.steps > 1u ? vt.march(c, k.steps, k.macros) : vt.step(c, k.macros);
+    return k.steps > 1u ? vt.fused(c, k.steps, k.macros) : vt.step(c, k.macros);
 }
 
 int lbm_run(lbm_ctx *c, uint32_t steps, uint32_t frame_interval)
@@ -2427,21 +2480,38 @@ int lbm_run_frames(lbm_ctx *c, uint32_t steps, uint32_t frame_interval)
     {
         LBM_HIP_TRY(hipStreamCreateWithFlags(&c->copy_stream, hipStreamNonBlocking));
         LBM_HIP_TRY(hipEventCreateWithFlags(&c->ev_frame, hipEventDisableTiming));
-        LBM_HIP_TRY(hipEventCreateWithFlags(&c->ev_copied, hipEventDisableTiming));
+        for (hipEvent_t &e : c->ev_copied)
+            LBM_HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+        if (hipMalloc(&c->res_other, 4ull * std::max(1u, c->D) * sizeof(double)) != hipSuccess)
+        {
+            (void)hipGetLastError();
+            c->res_other = nullptr;  // frames then wait for each other's copies
+        }
         LBM_HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&c->frame_host),
                                   4ull * std::max(1u, c->D) * sizeof(double), hipHostMallocDefault));
     }
     const VTable vt = vtable(c);
     uint64_t last_frame = ~0ull;
+    if (c->res_other && !c->res_other_valid)
+    {
+        LBM_HIP_TRY(hipMemcpyAsync(c->res_other, c->res, 4ull * c->D * sizeof(double), hipMemcpyDeviceToDevice,
+                                   c->stream));
+        c->res_other_valid = true;
+    }
     LBM_HIP_TRY(hipEventRecord(c->ev0, c->stream));
     for (uint32_t left = steps; left;)
     {
         const Chunk k = next_chunk(c, left, frame_interval);
-        if (k.macros && c->copy_pending)
+        if (k.frame && c->res_other)
+        {
+            std::swap(c->res, c->res_other);
+            c->res_half ^= 1;
+        }
+        if (k.macros && c->copy_pending[c->res_half])
         {
             // the results must not change under the copy still reading them
-            LBM_HIP_TRY(hipStreamWaitEvent(c->stream, c->ev_copied, 0));
-            c->copy_pending = false;
+            LBM_HIP_TRY(hipStreamWaitEvent(c->stream, c->ev_copied[c->res_half], 0));
+            c->copy_pending[c->res_half] = false;
         }
         if (int rc = run_chunk(c, vt, k))
             return rc;
@@ -2450,17 +2520,20 @@ int lbm_run_frames(lbm_ctx *c, uint32_t steps, uint32_t frame_interval)
         {
             LBM_HIP_TRY(hipEventRecord(c->ev_frame, c->stream));
             LBM_HIP_TRY(hipStreamWaitEvent(c->copy_stream, c->ev_frame, 0));
-            LBM_HIP_TRY(hipMemcpyAsync(c->frame_host, c->res, 4ull * c->D * sizeof(double), hipMemcpyDeviceToHost,
-                                       c->copy_stream));
-            LBM_HIP_TRY(hipEventRecord(c->ev_copied, c->copy_stream));
-            c->copy_pending = true;
+            const size_t n = 2ull * c->D;  // 16-byte vectors
+            hipLaunchKernelGGL(k_copy_frame, dim3(uint32_t(std::min<size_t>((n + 255) / 256, FRAME_COPY_BLOCKS))),
+                               dim3(256), 0, c->copy_stream, reinterpret_cast<const uint4 *>(c->res),
+                               reinterpret_cast<uint4 *>(c->frame_host), n);
+            LBM_HIP_TRY(hipGetLastError());
+            LBM_HIP_TRY(hipEventRecord(c->ev_copied[c->res_half], c->copy_stream));
+            c->copy_pending[c->res_half] = true;
             last_frame = c->iteration - 1u;
         }
     }
     LBM_HIP_TRY(hipEventRecord(c->ev1, c->stream));
     LBM_HIP_TRY(hipEventSynchronize(c->ev1));
     LBM_HIP_TRY(hipStreamSynchronize(c->copy_stream));
-    c->copy_pending = false;
+    c->copy_pending[0] = c->copy_pending[1] = false;
     if (last_frame != ~0ull)
         c->frame_iteration = last_frame;
     float ms = 0.f;
@@ -2670,6 +2743,7 @@ int lbm_set_state(lbm_ctx *c, const void *buf, size_t bytes)
     c->frame_iteration = ~0ull;
     c->cur = int(cur);
     c->uy_cur = int(iteration & 1u);
+    c->res_other_valid = false;
     c->snap_valid = false;
     c->side_valid = false;
     return LBM_OK;

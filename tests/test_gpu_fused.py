@@ -40,28 +40,41 @@ def check(doc, steps, frame_interval=0):
         assert same(one.macros(), many.macros())
 
 
-# inner extents: a whole number of strips and ragged ones (a strip is 56, 112
-# or 224 columns in FP64, FP32 and 16-bit storage)
-SIZES = {"f64": [(1120, 300), (3001, 103), (57, 5400)], "f32": [(2240, 560), (1999, 613)],
-         "f16-shifted": [(3001, 2003)], "bf16-shifted": [(3001, 2003)]}
+# Inner extents.  Marching waves own strips of 56, 112 or 224 columns (FP64,
+# FP32, 16-bit): whole strips, ragged ones, one strip and a half.
+MARCHED = {"f64": [(2240, 700), (3001, 503), (85, 17700)], "f32": [(2240, 901), (1999, 1013)],
+           "f16-shifted": [(3001, 1171)], "bf16-shifted": [(2688, 1310)]}
+# Small lattices: less than a region, each shape's whole and ragged numbers of them.
+TILED = [(4, 9), (30, 12), (61, 37), (256, 64), (257, 131), (500, 250), (1031, 301), (1030, 800)]
 
 
 @pytest.mark.parametrize("storage,rounding", STORAGES)
 @pytest.mark.parametrize("layout", ["collision", "stream", "bundle"])
-def test_fused_steps_equal_single_steps(layout, storage, rounding):
-    for k, (h, v) in enumerate(SIZES[storage]):
+def test_marched_steps_equal_single_steps(layout, storage, rounding):
+    for k, (h, v) in enumerate(MARCHED[storage]):
         scenario = ["porous-circles", "walls", "circle"][k]
         check(document("nptl" if k != 1 else "lptl", layout, storage, rounding, h, v, scenario), 23)
 
 
+@pytest.mark.parametrize("storage,rounding", STORAGES)
+@pytest.mark.parametrize("layout", ["collision", "stream", "bundle"])
+def test_tiled_steps_equal_single_steps(layout, storage, rounding):
+    for k, (h, v) in enumerate(TILED):
+        scenario = ["Hagen-Poiseuille", "walls", "porous", "porous-circles"][k % 4]
+        check(document("lptl" if k % 2 else "nptl", layout, storage, rounding, h, v, scenario, 64 if h < 64 else 256),
+              29 + k)
+
+
+@pytest.mark.parametrize("size", [(2011, 801), (1031, 301), (300, 100)])
 @pytest.mark.parametrize("steps", [1, 2, 3, 4, 5, 6, 7, 8])
-def test_every_remainder(steps):
-    check(document("nptl", "stream", "f64", "nearest", 1031, 301, "porous-circles"), steps)
+def test_every_remainder(steps, size):
+    check(document("nptl", "stream", "f64", "nearest", *size, "porous-circles"), steps)
 
 
+@pytest.mark.parametrize("size", [(2011, 801), (300, 100)])
 @pytest.mark.parametrize("interval", [1, 3, 10])
-def test_frames_end_a_launch(interval):
-    doc = document("lptl", "collision", "f64", "nearest", 1031, 301, "porous-circles")
+def test_frames_end_a_launch(interval, size):
+    doc = document("lptl", "collision", "f64", "nearest", *size, "porous-circles")
     check(doc, 21, interval)
     phase = pa.build_phase(doc)
     with pa.Lattice(pa.desc_from_settings(doc), phase) as a, pa.Lattice(pa.desc_from_settings(doc), phase) as b:
@@ -72,14 +85,16 @@ def test_frames_end_a_launch(interval):
         assert same(fields, b.macros())
 
 
-def test_reference_change_between_launches():
+@pytest.mark.parametrize("size", [(3001, 1171), (300, 100)])
+def test_reference_change_between_launches(size):
     """16-bit storage changes its column reference at step 128."""
-    check(document("nptl", "stream", "f16-shifted", "nearest", 3001, 2003, "porous-circles"), 134)
+    check(document("nptl", "stream", "f16-shifted", "nearest", *size, "porous-circles"), 134)
 
 
-def test_state_after_fused_steps():
+@pytest.mark.parametrize("size", [(2011, 801), (300, 100)])
+def test_state_after_fused_steps(size):
     """A state taken after an odd number of launches continues elsewhere."""
-    doc = document("nptl", "bundle", "f64", "nearest", 1031, 301, "porous-circles")
+    doc = document("nptl", "bundle", "f64", "nearest", *size, "porous-circles")
     phase = pa.build_phase(doc)
     with pa.Lattice(pa.desc_from_settings(doc), phase) as a, pa.Lattice(pa.desc_from_settings(doc), phase) as b:
         a.run(12)
@@ -92,14 +107,16 @@ def test_state_after_fused_steps():
         assert same(a.macros(), b.macros())
 
 
-def test_diverging_flow_keeps_its_infinities():
+@pytest.mark.parametrize("size", [(2011, 801), (300, 100)])
+@pytest.mark.parametrize("storage", ["f64", "f32"])
+def test_diverging_flow_keeps_its_infinities(storage, size):
     """Populations that are not finite take the full sums, as the one-step kernels do."""
-    doc = document("nptl", "stream", "f64", "nearest", 1031, 301, "porous-circles", tau=0.503)
+    doc = document("nptl", "stream", storage, "nearest", *size, "porous-circles", tau=0.503)
     phase = pa.build_phase(doc)
     with pa.Lattice(pa.desc_from_settings(doc), phase) as one, pa.Lattice(pa.desc_from_settings(doc), phase) as many:
         f = one.populations()
         f[::7919] = np.inf
-        f[::15838] = 1e300
+        f[::15838] = 1e300 if storage == "f64" else 1e30
         for lattice in (one, many):
             lattice.set_populations(f)
         for _ in range(8):
