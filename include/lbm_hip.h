@@ -22,8 +22,9 @@
  *     npol/npol.hpp:180-201, nsol/nsol.hpp:184-205
  *     (EmplaceBounceBackKernel, OutletUpdateKernel, StreamCollideKernel and
  *      the buffer-copy kernels of every algorithm are fused into one launch
- *      per step; the one-lattice schemes with tiles wider than 64 nodes, and
- *      npol's FP64 collision layout, add the buffer refresh: two launches)
+ *      for up to six steps; in place, the one-lattice schemes take one step
+ *      per launch, and with tiles wider than 64 nodes, or in npol's FP64
+ *      collision layout, add the buffer refresh: two launches)
  *   SYCLAlgorithm::copy_macroscopic_observables_to_cpu   lbm_get_macros
  *     include/lbm/execution/sycl_algorithm.hpp:90-104
  *   the same copies enqueued after each frame step       lbm_run_frames /
@@ -86,13 +87,19 @@ enum lbm_storage {
  * every step near a steady state.  No counterpart in the reference. */
 enum lbm_rounding { LBM_ROUND_NEAREST = 0, LBM_ROUND_STOCHASTIC = 1 };
 
-/* Step kernel of npol/nsol lattices whose tiles are at most 64 nodes wide.
+/* Step kernels of npol/nsol.
+ * Auto, first choice: round-to-nearest lattices whose second copy takes at
+ * most 1/64 of the device's memory, and gets it, run the unexpanded lattice
+ * through lptl's kernels, several steps per launch; lbm_get_populations then
+ * returns the rest state at buffer nodes.  Everything else works in place on
+ * one lattice, by one of the kernels below.
+ * The in-place kernels of lattices whose tiles are at most 64 nodes wide.
  * Sweep: one wave walks each tile, the tile-edge copies in side arrays (no
  * refresh launches); block: one work-group per tile with the reference's
  * buffer refresh before each step; staged (tiles at least 8 nodes wide;
  * narrower ones run the automatic choice): one work-group per tile walks it
  * a chunk of rows at a time through LDS, with the sweep's side arrays.
- * Auto: in the FP64 and FP32 collision layout the staged
+ * Auto, in place: in the FP64 and FP32 collision layout the staged
  * kernel on lattices of at least half a tile (FP64) or one tile (FP32) per
  * compute unit; else the sweep when the lattice has at least two tiles per
  * compute unit and the layout is not npol's FP64 collision layout; else the

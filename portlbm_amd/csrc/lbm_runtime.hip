@@ -106,6 +106,11 @@ struct lbm_ctx
     bool snap_valid = false;
     double last_ms = 0.0;
     double feq_in[9], feq_out[9];
+    // npol / nsol that need not stay in place (see plan_compact): the work is
+    // done by this context on the unexpanded lattice; the outer one converts
+    // what callers hand over and receive in the expanded order.
+    lbm_ctx *inner = nullptr;
+    std::vector<int8_t> outer_phase;  // the expanded node types, as set
     // 16-bit forms: rho_ref per unexpanded column (Hx + 64 floats, the tail
     // 1), two tables used in turn; a step that changes the reference reads
     // with ref[ref_cur] and writes with ref[1 - ref_cur]
@@ -1991,6 +1996,74 @@ static size_t storage_bytes(int s)
     }
 }
 
+// npol and nsol keep one lattice and work in place, tile by tile, each step
+// behind the exchange of tile edges: two to three times the time of a
+// two-lattice step, and of one step only.  Their fields are the two-lattice
+// algorithms' (every pull reads the previous step), so where a second lattice
+// is cheap -- at most 1/64 of the device's memory -- the automatic choice
+// drops the buffer rows and columns and runs the unexpanded lattice through
+// lptl's kernels, several steps per launch (us per step, FP64 npol stream on
+// 4096 x 1024: 142 in place, 46 so).  Larger lattices and explicit
+// lbm_desc.tile_kernel choices stay in place; so does stochastic rounding,
+// whose random bits are drawn from a node's place in the expanded lattice.
+static bool plan_compact(const lbm_ctx *c)
+{
+    if (!c->buffered || c->desc.tile_kernel != LBM_TILE_AUTO || c->desc.rounding == LBM_ROUND_STOCHASTIC)
+        return false;
+    size_t free_bytes = 0, total = 0;
+    if (hipMemGetInfo(&free_bytes, &total) != hipSuccess)
+        return false;
+    return 9ull * (c->H + 127u) * c->V * c->elem <= total / 64u;
+}
+
+// Expanded coordinate of unexpanded u on an axis of `last` + 1 nodes (map_axis on the host).
+static uint32_t expanded_of(uint32_t u, uint32_t last, uint32_t sub)
+{
+    return u == 0u ? 0u : (u == last ? last + (last - 2u) / sub : u + (u - 1u) / sub);
+}
+
+// Calls f(unexpanded node, expanded node, count) for runs of nodes that are
+// consecutive in both orders, over the whole unexpanded lattice.
+template <class F>
+static void for_runs(const lbm_ctx *c, F f)
+{
+    for (uint32_t y = 0; y < c->V; ++y)
+    {
+        const size_t row = size_t(expanded_of(y, c->V - 1u, c->sub_v)) * c->Hx;
+        // a tile's nodes; the ghosts adjoin the first and the last one
+        for (uint32_t x = 0, n; x < c->H; x += n)
+        {
+            n = x ? c->sub_h : c->sub_h + 1u;
+            if (n >= c->H - 1u - x)
+                n = c->H - x;
+            f(size_t(y) * c->H + x, row + expanded_of(x, c->H - 1u, c->sub_h), size_t(n));
+        }
+    }
+}
+
+// Index of population d of node n in a layout's flat order over `total` nodes.
+static size_t flat_index(int layout, size_t n, uint32_t d, size_t total)
+{
+    return layout == LBM_LAYOUT_COLLISION ? 9u * n + d
+                                          : (layout == LBM_LAYOUT_STREAM ? total * d + n : 3u * (d / 3u) * total + d % 3u + 3u * n);
+}
+
+// For a context that works on an inner one: f(bytes into the inner lattice,
+// bytes into the expanded placement that states are kept in, bytes) over the
+// lattice's nodes.
+template <class F>
+static void for_placed_runs(const lbm_ctx *c, F f)
+{
+    const lbm_ctx *in = c->inner;
+    const size_t el = c->elem;
+    const size_t K = c->desc.layout == LBM_LAYOUT_COLLISION ? 9 : (c->desc.layout == LBM_LAYOUT_BUNDLE ? 3 : 1);
+    for (size_t a = 0; a < 9 / K; ++a)  // arrays of K populations per node
+        for_runs(c, [&](size_t u, size_t e, size_t k) {
+            const size_t pu = in->X0 + u % c->H + u / c->H * in->P, pe = c->X0 + e % c->Hx + e / c->Hx * c->P;
+            f((a * K * in->Sd + K * pu) * el, (a * K * c->Sd + K * pe) * el, k * K * el);
+        });
+}
+
 // ---------------------------------------------------------------------------
 // C ABI
 // ---------------------------------------------------------------------------
@@ -2103,6 +2176,7 @@ void lbm_destroy(lbm_ctx *c)
 {
     if (!c)
         return;
+    lbm_destroy(c->inner);
     // both streams drained before anything they may still read or write is freed
     if (c->stream)
         (void)hipStreamSynchronize(c->stream);
@@ -2195,6 +2269,26 @@ int lbm_create(const lbm_desc *desc, lbm_ctx **out)
     host_equilibrium(desc->storage, desc->inlet_velocity_x, desc->inlet_velocity_y, desc->inlet_density, c->feq_in);
     host_equilibrium(desc->storage, desc->outlet_velocity_x, desc->outlet_velocity_y, desc->outlet_density,
                      c->feq_out);
+
+    if (plan_compact(c))
+    {
+        lbm_desc d = *desc;
+        d.algorithm = LBM_ALG_LPTL;
+        d.expanded_horizontal_nodes = d.horizontal_nodes;
+        d.expanded_vertical_nodes = d.vertical_nodes;
+        d.work_group_size = 256;
+        if (lbm_create(&d, &c->inner) == LBM_OK)
+        {
+            c->inner->outlet_active = c->outlet_active;
+            if (c->inner->ref_len)
+                c->ref_len = std::max(c->Hx, c->H) + 64u;
+            c->outer_phase.assign(c->N, int8_t(-1));
+            *out = c;
+            return LBM_OK;
+        }
+        (void)hipGetLastError();
+        c->inner = nullptr;  // no memory for two lattices: in place
+    }
 
     auto cleanup = [&](int rc) {
         lbm_destroy(c);
@@ -2323,6 +2417,15 @@ int lbm_set_phase(lbm_ctx *c, const int8_t *phase, size_t n)
         return fail(LBM_ERR_INVALID_ARGUMENT, "lbm_set_phase: null argument");
     if (n != c->N)
         return fail(LBM_ERR_INVALID_ARGUMENT, "lbm_set_phase: node_count must equal the expanded node count");
+    if (c->inner)
+    {
+        std::vector<int8_t> own(size_t(c->H) * c->V);
+        for_runs(c, [&](size_t u, size_t e, size_t k) { std::copy_n(phase + e, k, own.begin() + u); });
+        if (int rc = lbm_set_phase(c->inner, own.data(), own.size()))
+            return rc;
+        std::copy_n(phase, n, c->outer_phase.begin());
+        return LBM_OK;
+    }
     LBM_HIP_TRY(hipMemcpyAsync(c->phase, phase, n, hipMemcpyHostToDevice, c->stream));
     LBM_HIP_TRY(hipStreamSynchronize(c->stream));
     c->phase_set = true;
@@ -2337,6 +2440,11 @@ int lbm_get_phase(lbm_ctx *c, int8_t *phase, size_t n)
         return fail(LBM_ERR_INVALID_ARGUMENT, "lbm_get_phase: null argument");
     if (n != c->N)
         return fail(LBM_ERR_INVALID_ARGUMENT, "lbm_get_phase: node_count must equal the expanded node count");
+    if (c->inner)
+    {
+        std::copy(c->outer_phase.begin(), c->outer_phase.end(), phase);
+        return LBM_OK;
+    }
     LBM_HIP_TRY(hipMemcpyAsync(phase, c->phase, n, hipMemcpyDeviceToHost, c->stream));
     LBM_HIP_TRY(hipStreamSynchronize(c->stream));
     return LBM_OK;
@@ -2361,6 +2469,8 @@ int lbm_init_populations(lbm_ctx *c)
 {
     if (!c)
         return fail(LBM_ERR_INVALID_ARGUMENT, "lbm_init_populations: null context");
+    if (c->inner)
+        return lbm_init_populations(c->inner);
     if (!c->phase_set)
         return fail(LBM_ERR_STATE, "lbm_init_populations: lbm_set_phase must come first");
     c->cur = 0;
@@ -2388,6 +2498,17 @@ int lbm_get_node_codes(lbm_ctx *c, uint16_t *codes, size_t n)
 {
     if (!c || !codes)
         return fail(LBM_ERR_INVALID_ARGUMENT, "lbm_get_node_codes: null argument");
+    if (c->inner)
+    {
+        if (n != c->N)
+            return fail(LBM_ERR_INVALID_ARGUMENT, "lbm_get_node_codes: node_count must equal the expanded node count");
+        std::vector<uint16_t> own(size_t(c->H) * c->V);
+        if (int rc = lbm_get_node_codes(c->inner, own.data(), own.size()))
+            return rc;
+        std::fill_n(codes, n, uint16_t(0));
+        for_runs(c, [&](size_t u, size_t e, size_t k) { std::copy_n(own.begin() + u, k, codes + e); });
+        return LBM_OK;
+    }
     if (!c->initialized)
         return fail(LBM_ERR_STATE, "lbm_get_node_codes: call lbm_init_populations first");
     if (n != c->N)
@@ -2451,6 +2572,8 @@ int lbm_run(lbm_ctx *c, uint32_t steps, uint32_t frame_interval)
 {
     if (!c)
         return fail(LBM_ERR_INVALID_ARGUMENT, "lbm_run: null context");
+    if (c->inner)
+        return lbm_run(c->inner, steps, frame_interval);
     if (!c->initialized)
         return fail(LBM_ERR_STATE, "lbm_run: call lbm_init_populations first");
     const VTable vt = vtable(c);
@@ -2474,6 +2597,8 @@ int lbm_run_frames(lbm_ctx *c, uint32_t steps, uint32_t frame_interval)
 {
     if (!c)
         return fail(LBM_ERR_INVALID_ARGUMENT, "lbm_run_frames: null context");
+    if (c->inner)
+        return lbm_run_frames(c->inner, steps, frame_interval);
     if (!c->initialized)
         return fail(LBM_ERR_STATE, "lbm_run_frames: call lbm_init_populations first");
     if (!c->copy_stream)
@@ -2546,6 +2671,8 @@ int lbm_get_frame(lbm_ctx *c, double *rho, double *jx, double *jy, double *jabs,
 {
     if (!c)
         return fail(LBM_ERR_INVALID_ARGUMENT, "lbm_get_frame: null context");
+    if (c->inner)
+        return lbm_get_frame(c->inner, rho, jx, jy, jabs, count, iteration);
     if (count != c->D)
         return fail(LBM_ERR_INVALID_ARGUMENT, "lbm_get_frame: count must equal (H-2)*(V-2)");
     if (c->frame_iteration == ~0ull)
@@ -2563,6 +2690,8 @@ int lbm_run_split(lbm_ctx *c, uint32_t steps, lbm_pass_callback cb, void *user)
 {
     if (!c)
         return fail(LBM_ERR_INVALID_ARGUMENT, "lbm_run_split: null context");
+    if (c->inner)
+        return lbm_run_split(c->inner, steps, cb, user);
     if (!c->initialized)
         return fail(LBM_ERR_STATE, "lbm_run_split: call lbm_init_populations first");
     if (!c->pass)
@@ -2593,6 +2722,22 @@ int lbm_get_pass_populations(lbm_ctx *c, double *values, size_t count)
 {
     if (!c || !values)
         return fail(LBM_ERR_INVALID_ARGUMENT, "lbm_get_pass_populations: null argument");
+    if (c->inner)
+    {
+        if (!c->inner->pass)
+            return fail(LBM_ERR_STATE, "lbm_get_pass_populations: no split step has run");
+        if (count != 9ull * c->N)
+            return fail(LBM_ERR_INVALID_ARGUMENT,
+                        "lbm_get_pass_populations: count must be 9 * expanded node count");
+        const size_t M = size_t(c->H) * c->V;
+        std::vector<double> own(9 * M);
+        if (int rc = lbm_get_pass_populations(c->inner, own.data(), own.size()))
+            return rc;
+        std::fill_n(values, count, 0.0);
+        for (uint32_t d = 0; d < 9; ++d)
+            for_runs(c, [&](size_t u, size_t e, size_t k) { std::copy_n(&own[d * M + u], k, values + size_t(d) * c->N + e); });
+        return LBM_OK;
+    }
     if (!c->pass)
         return fail(LBM_ERR_STATE, "lbm_get_pass_populations: no split step has run");
     if (count != 9ull * c->N)
@@ -2627,6 +2772,8 @@ int lbm_get_iteration(lbm_ctx *c, uint64_t *it)
 {
     if (!c || !it)
         return fail(LBM_ERR_INVALID_ARGUMENT, "lbm_get_iteration: null argument");
+    if (c->inner)
+        return lbm_get_iteration(c->inner, it);
     *it = c->iteration;
     return LBM_OK;
 }
@@ -2635,6 +2782,8 @@ int lbm_last_run_ms(lbm_ctx *c, double *ms)
 {
     if (!c || !ms)
         return fail(LBM_ERR_INVALID_ARGUMENT, "lbm_last_run_ms: null argument");
+    if (c->inner)
+        return lbm_last_run_ms(c->inner, ms);
     *ms = c->last_ms;
     return LBM_OK;
 }
@@ -2643,6 +2792,8 @@ int lbm_get_macros(lbm_ctx *c, double *rho, double *jx, double *jy, double *jabs
 {
     if (!c)
         return fail(LBM_ERR_INVALID_ARGUMENT, "lbm_get_macros: null context");
+    if (c->inner)
+        return lbm_get_macros(c->inner, rho, jx, jy, jabs, count);
     if (count != c->D)
         return fail(LBM_ERR_INVALID_ARGUMENT, "lbm_get_macros: count must equal (H-2)*(V-2)");
     double *dst[4] = {rho, jx, jy, jabs};
@@ -2671,15 +2822,91 @@ int lbm_state_size(const lbm_ctx *c, size_t *bytes)
     return LBM_OK;
 }
 
+// What follows the lattices in a state: the outlet history, the half that the
+// next step reads at the place of the iteration's parity; the results; the
+// 16-bit forms' rho_ref table, ref_len columns of it.
+static int get_state_tail(lbm_ctx *c, char *out, uint32_t ref_len)
+{
+    const size_t half = size_t(c->V) * sizeof(double);
+    const size_t at = (c->iteration & 1u) ? half : 0u;
+    LBM_HIP_TRY(hipMemcpy(out + at, c->uycol + size_t(c->uy_cur) * c->V, half, hipMemcpyDeviceToHost));
+    LBM_HIP_TRY(hipMemcpy(out + (half - at), c->uycol + size_t(1 - c->uy_cur) * c->V, half, hipMemcpyDeviceToHost));
+    out += 2u * half;
+    LBM_HIP_TRY(hipMemcpy(out, c->res, 4ull * c->D * sizeof(double), hipMemcpyDeviceToHost));
+    out += 4ull * c->D * sizeof(double);
+    if (ref_len)
+    {
+        std::vector<float> ref(std::max(ref_len, c->ref_len), 1.f);
+        LBM_HIP_TRY(hipMemcpy(ref.data(), c->ref[c->ref_cur], c->ref_len * sizeof(float), hipMemcpyDeviceToHost));
+        std::memcpy(out, ref.data(), ref_len * sizeof(float));
+    }
+    return LBM_OK;
+}
+
+static int set_state_tail(lbm_ctx *c, const char *in, uint32_t ref_len, uint64_t iteration, int cur)
+{
+    LBM_HIP_TRY(hipMemcpy(c->uycol, in, 2ull * c->V * sizeof(double), hipMemcpyHostToDevice));
+    in += 2ull * c->V * sizeof(double);
+    LBM_HIP_TRY(hipMemcpy(c->res, in, 4ull * c->D * sizeof(double), hipMemcpyHostToDevice));
+    in += 4ull * c->D * sizeof(double);
+    c->ref_cur = 0;
+    c->ref_switch = false;
+    if (ref_len)
+    {
+        std::vector<float> ref(std::max(ref_len, c->ref_len), 1.f);
+        std::memcpy(ref.data(), in, ref_len * sizeof(float));
+        LBM_HIP_TRY(hipMemcpy(c->ref[0], ref.data(), c->ref_len * sizeof(float), hipMemcpyHostToDevice));
+    }
+    LBM_HIP_TRY(hipDeviceSynchronize());
+    c->iteration = iteration;
+    c->frame_iteration = ~0ull;
+    c->cur = cur;
+    c->uy_cur = int(iteration & 1u);
+    c->res_other_valid = false;
+    c->snap_valid = false;
+    c->side_valid = false;
+    return LBM_OK;
+}
+
+static int get_inner_state(lbm_ctx *c, char *out)
+{
+    lbm_ctx *in = c->inner;
+    const uint32_t cur = 0, lattices = 1;
+    std::memcpy(out, &in->iteration, 8);
+    std::memcpy(out + 8, &cur, 4);
+    std::memcpy(out + 12, &lattices, 4);
+    const size_t lat_bytes = c->lattice_elems * c->elem;
+    std::memset(out + 16, 0, lat_bytes);
+    std::vector<char> own(in->lattice_elems * in->elem);
+    LBM_HIP_TRY(hipStreamSynchronize(in->stream));
+    LBM_HIP_TRY(hipMemcpy(own.data(), in->lat[in->cur], own.size(), hipMemcpyDeviceToHost));
+    for_placed_runs(c, [&](size_t o, size_t x, size_t n) { std::memcpy(out + 16 + x, own.data() + o, n); });
+    return get_state_tail(in, out + 16 + lat_bytes, c->ref_len);
+}
+
+static int set_inner_state(lbm_ctx *c, const char *buf, uint64_t iteration)
+{
+    lbm_ctx *in = c->inner;
+    std::vector<char> own(in->lattice_elems * in->elem);
+    LBM_HIP_TRY(hipStreamSynchronize(in->stream));
+    LBM_HIP_TRY(hipMemcpy(own.data(), in->lat[0], own.size(), hipMemcpyDeviceToHost));  // padding as it is
+    for_placed_runs(c, [&](size_t o, size_t x, size_t n) { std::memcpy(own.data() + o, buf + 16 + x, n); });
+    for (void *lat : in->lat)
+        LBM_HIP_TRY(hipMemcpy(lat, own.data(), own.size(), hipMemcpyHostToDevice));
+    return set_state_tail(in, buf + 16 + c->lattice_elems * c->elem, c->ref_len, iteration, 0);
+}
+
 int lbm_get_state(lbm_ctx *c, void *buf, size_t bytes)
 {
     if (!c || !buf)
         return fail(LBM_ERR_INVALID_ARGUMENT, "lbm_get_state: null argument");
-    if (!c->initialized)
+    if (!(c->inner ? c->inner : c)->initialized)
         return fail(LBM_ERR_STATE, "lbm_get_state: call lbm_init_populations first");
     if (bytes != state_bytes(c))
         return fail(LBM_ERR_INVALID_ARGUMENT, "lbm_get_state: size must be lbm_state_size()");
     char *out = static_cast<char *>(buf);
+    if (c->inner)
+        return get_inner_state(c, out);
     const uint32_t lattices = c->two_lattice ? 2u : 1u;
     const uint32_t cur = uint32_t(c->cur);
     std::memcpy(out, &c->iteration, 8);
@@ -2692,26 +2919,14 @@ int lbm_get_state(lbm_ctx *c, void *buf, size_t bytes)
     LBM_HIP_TRY(hipStreamSynchronize(c->stream));
     for (uint32_t l = 0; l < lattices; ++l, off += lat_bytes)
         LBM_HIP_TRY(hipMemcpy(out + off, c->lat[l], lat_bytes, hipMemcpyDeviceToHost));
-    // outlet history: the half that the next step reads at the place of the
-    // iteration's parity
-    const size_t half = size_t(c->V) * sizeof(double);
-    const size_t at = (c->iteration & 1u) ? half : 0u;
-    LBM_HIP_TRY(hipMemcpy(out + off + at, c->uycol + size_t(c->uy_cur) * c->V, half, hipMemcpyDeviceToHost));
-    LBM_HIP_TRY(hipMemcpy(out + off + (half - at), c->uycol + size_t(1 - c->uy_cur) * c->V, half,
-                          hipMemcpyDeviceToHost));
-    off += 2u * half;
-    LBM_HIP_TRY(hipMemcpy(out + off, c->res, 4ull * c->D * sizeof(double), hipMemcpyDeviceToHost));
-    off += 4ull * c->D * sizeof(double);
-    if (c->ref_len)
-        LBM_HIP_TRY(hipMemcpy(out + off, c->ref[c->ref_cur], c->ref_len * sizeof(float), hipMemcpyDeviceToHost));
-    return LBM_OK;
+    return get_state_tail(c, out + off, c->ref_len);
 }
 
 int lbm_set_state(lbm_ctx *c, const void *buf, size_t bytes)
 {
     if (!c || !buf)
         return fail(LBM_ERR_INVALID_ARGUMENT, "lbm_set_state: null argument");
-    if (!c->initialized)
+    if (!(c->inner ? c->inner : c)->initialized)
         return fail(LBM_ERR_STATE, "lbm_set_state: call lbm_init_populations first");
     if (bytes != state_bytes(c))
         return fail(LBM_ERR_INVALID_ARGUMENT, "lbm_set_state: size does not match this context");
@@ -2723,6 +2938,8 @@ int lbm_set_state(lbm_ctx *c, const void *buf, size_t bytes)
     std::memcpy(&lattices, in + 12, 4);
     if (lattices != (c->two_lattice ? 2u : 1u) || cur >= lattices)
         return fail(LBM_ERR_INVALID_ARGUMENT, "lbm_set_state: state of another algorithm");
+    if (c->inner)
+        return set_inner_state(c, in, iteration);
     size_t off = 16;
     const size_t lat_bytes = c->lattice_elems * c->elem;
     // pageable source: blocking copies once the context's stream is idle,
@@ -2730,23 +2947,7 @@ int lbm_set_state(lbm_ctx *c, const void *buf, size_t bytes)
     LBM_HIP_TRY(hipStreamSynchronize(c->stream));
     for (uint32_t l = 0; l < lattices; ++l, off += lat_bytes)
         LBM_HIP_TRY(hipMemcpy(c->lat[l], in + off, lat_bytes, hipMemcpyHostToDevice));
-    LBM_HIP_TRY(hipMemcpy(c->uycol, in + off, 2ull * c->V * sizeof(double), hipMemcpyHostToDevice));
-    off += 2ull * c->V * sizeof(double);
-    LBM_HIP_TRY(hipMemcpy(c->res, in + off, 4ull * c->D * sizeof(double), hipMemcpyHostToDevice));
-    off += 4ull * c->D * sizeof(double);
-    c->ref_cur = 0;
-    c->ref_switch = false;
-    if (c->ref_len)
-        LBM_HIP_TRY(hipMemcpy(c->ref[0], in + off, c->ref_len * sizeof(float), hipMemcpyHostToDevice));
-    LBM_HIP_TRY(hipDeviceSynchronize());
-    c->iteration = iteration;
-    c->frame_iteration = ~0ull;
-    c->cur = int(cur);
-    c->uy_cur = int(iteration & 1u);
-    c->res_other_valid = false;
-    c->snap_valid = false;
-    c->side_valid = false;
-    return LBM_OK;
+    return set_state_tail(c, in + off, c->ref_len, iteration, int(cur));
 }
 
 // The population accessors convert between the storage and FP64 through a
@@ -2767,6 +2968,25 @@ int lbm_get_populations(lbm_ctx *c, double *values, size_t count)
         return fail(LBM_ERR_INVALID_ARGUMENT, "lbm_get_populations: null argument");
     if (count != 9ull * c->N)
         return fail(LBM_ERR_INVALID_ARGUMENT, "lbm_get_populations: count must be 9 * expanded node count");
+    if (c->inner)
+    {
+        const size_t M = size_t(c->H) * c->V;
+        std::vector<double> own(9 * M);
+        if (int rc = lbm_get_populations(c->inner, own.data(), own.size()))
+            return rc;
+        // buffer nodes are not kept: the rest state, as after lbm_init_populations
+        static const double w[9] = {1.0 / 36, 1.0 / 9, 1.0 / 36, 1.0 / 9, 4.0 / 9, 1.0 / 9, 1.0 / 36, 1.0 / 9, 1.0 / 36};
+        const int layout = c->desc.layout;
+        for (uint32_t d = 0; d < 9; ++d)
+            for (size_t e = 0; e < c->N; ++e)
+                values[flat_index(layout, e, d, c->N)] = w[d];
+        for (uint32_t d = 0; d < 9; ++d)
+            for_runs(c, [&](size_t u, size_t e, size_t k) {
+                for (size_t i = 0; i < k; ++i)
+                    values[flat_index(layout, e + i, d, c->N)] = own[flat_index(layout, u + i, d, M)];
+            });
+        return LBM_OK;
+    }
     if (int rc = ensure_stage(c))
         return rc;
     const VTable vt = vtable(c);
@@ -2785,6 +3005,22 @@ int lbm_set_populations(lbm_ctx *c, const double *values, size_t count)
 {
     if (!c || !values)
         return fail(LBM_ERR_INVALID_ARGUMENT, "lbm_set_populations: null argument");
+    if (c->inner)
+    {
+        if (!c->inner->initialized)
+            return fail(LBM_ERR_STATE, "lbm_set_populations: call lbm_init_populations first");
+        if (count != 9ull * c->N)
+            return fail(LBM_ERR_INVALID_ARGUMENT, "lbm_set_populations: count must be 9 * expanded node count");
+        const size_t M = size_t(c->H) * c->V;
+        const int layout = c->desc.layout;
+        std::vector<double> own(9 * M);
+        for (uint32_t d = 0; d < 9; ++d)
+            for_runs(c, [&](size_t u, size_t e, size_t k) {
+                for (size_t i = 0; i < k; ++i)
+                    own[flat_index(layout, u + i, d, M)] = values[flat_index(layout, e + i, d, c->N)];
+            });
+        return lbm_set_populations(c->inner, own.data(), own.size());
+    }
     if (!c->initialized)
         return fail(LBM_ERR_STATE, "lbm_set_populations: call lbm_init_populations first");
     if (count != 9ull * c->N)
@@ -2812,6 +3048,8 @@ int lbm_set_equilibrium_field(lbm_ctx *c, const double *rho, const double *jx, c
 {
     if (!c || !rho || !jx || !jy)
         return fail(LBM_ERR_INVALID_ARGUMENT, "lbm_set_equilibrium_field: null argument");
+    if (c->inner)
+        return lbm_set_equilibrium_field(c->inner, rho, jx, jy, count);
     if (!c->initialized)
         return fail(LBM_ERR_STATE, "lbm_set_equilibrium_field: call lbm_init_populations first");
     if (count != c->D)
@@ -2852,6 +3090,8 @@ int lbm_reduce(lbm_ctx *c, double out[6])
 {
     if (!c || !out)
         return fail(LBM_ERR_INVALID_ARGUMENT, "lbm_reduce: null argument");
+    if (c->inner)
+        return lbm_reduce(c->inner, out);
     if (!c->initialized)
         return fail(LBM_ERR_STATE, "lbm_reduce: call lbm_init_populations first");
     return reduce_common(c, 0, out);
@@ -2861,6 +3101,8 @@ int lbm_residual(lbm_ctx *c, double *residual)
 {
     if (!c || !residual)
         return fail(LBM_ERR_INVALID_ARGUMENT, "lbm_residual: null argument");
+    if (c->inner)
+        return lbm_residual(c->inner, residual);
     if (!c->initialized)
         return fail(LBM_ERR_STATE, "lbm_residual: call lbm_init_populations first");
     if (!c->snap)
@@ -2881,6 +3123,8 @@ int lbm_sync(lbm_ctx *c)
 {
     if (!c)
         return fail(LBM_ERR_INVALID_ARGUMENT, "lbm_sync: null context");
+    if (c->inner)
+        return lbm_sync(c->inner);
     LBM_HIP_TRY(hipStreamSynchronize(c->stream));
     return LBM_OK;
 }
