@@ -15,6 +15,7 @@
 
 #include "lbm_device.hpp"
 #include "lbm_error.hpp"
+#include "lbm_march.hpp"
 #include "lbm_setup.hpp"
 
 using namespace lbm_dev;
@@ -31,19 +32,7 @@ namespace
                                  std::string(#expr) + ": " + hipGetErrorString(e_));                \
     } while (0)
 
-constexpr uint32_t kBatchX0 = 15;  // x = 1 starts a 16-node (64 B in FP32) segment
 constexpr int kTileThreads = 256;
-
-struct BatchDom
-{
-    uint64_t lat;   // element offset of the domain's lattice in each arena
-    uint32_t code;  // node offset in the code arena
-    uint32_t res;   // offset in the result arena (4 * D doubles)
-    uint32_t uy;    // offset in the outlet-history arena (2 * V doubles)
-    uint32_t H, V, P, S, D;
-    uint32_t tile_w;
-    double omega, rho_out;
-};
 
 // Set-up geometry of one domain: an unexpanded lattice with its own pitch.
 // The batched 16-bit forms store f_d - w_d (rho_ref = 1 in every column: `ones`).
@@ -273,13 +262,16 @@ struct lbm_batch
     uint32_t persistent_grid = 2048;
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
-    uint64_t iteration = 0;
+    int cur = 0;                 // arena and half of the outlet history that the next launch reads
+    FusePlan fuse;               // persistent and graph runs: several steps per launch
+    BatchPart *d_parts = nullptr;
+    uint32_t nparts = 0;
     bool initialized = false;
     double last_ms = 0.0;
     uint64_t fluid_nodes = 0;
     hipGraphExec_t graph = nullptr;
     uint32_t graph_steps = 0;
-    int graph_parity = -1;
+    int graph_parity = -1, graph_end = 0;
     double *snap = nullptr;      // 2 doubles per node place (residual snapshot, allocated by lbm_batch_init)
     bool snap_valid = false;
     double *scratch = nullptr;   // device address of this GPU's `scratch` (null if the lookup failed)
@@ -358,12 +350,101 @@ int step_dispatch(lbm_batch *b, int parity, bool macros, const BatchTile *tiles,
     }
 }
 
-int run_persistent_steps(lbm_batch *b, uint32_t steps, uint64_t first_iteration)
+// The parts of all domains for the fused launches: a wave's strip and rows,
+// or a block's first node.
+int build_parts(lbm_batch *b, int cus)
+{
+    uint64_t nodes = 0;
+    for (const BatchDom &dm : b->doms)
+        nodes += dm.D;
+    b->fuse = plan_fusion(b->elem, nodes);
+    std::vector<BatchPart> parts;
+    if (b->fuse.tiles)
+    {
+        const uint32_t halo = b->fuse.steps - 1u;
+        const uint32_t w = (b->fuse.shape == TileShape::k16x16 ? 16u : 32u) - 2u * halo;
+        const uint32_t h = (b->fuse.shape == TileShape::k32x32 ? 32u : 16u) - 2u * halo;
+        for (uint32_t d = 0; d < b->doms.size(); ++d)
+            for (uint32_t y = 1; y + 1u < b->doms[d].V; y += h)
+                for (uint32_t x = 1; x + 1u < b->doms[d].H; x += w)
+                    parts.push_back(BatchPart{d, x, y, 0u});
+    }
+    else
+    {
+        // every domain's rows split evenly into segments of at most `rows`,
+        // rows chosen for the whole batch
+        auto waves_of = [&](uint32_t rows, double *mean) {
+            uint64_t waves = 0, visits = 0;
+            for (const BatchDom &dm : b->doms)
+            {
+                const uint32_t inner = dm.V - 2u, strips = march_strips(b->storage, dm.H - 2u);
+                waves += uint64_t(strips) * ((inner + rows - 1u) / rows);
+                visits += uint64_t(strips) * inner;
+            }
+            *mean = double(visits) / double(waves);
+            return waves;
+        };
+        uint32_t best_rows = 8;
+        double best = 0.0;
+        for (uint32_t rows = 8; rows <= 160u; ++rows)
+        {
+            double mean = 0.0;
+            const uint64_t waves = waves_of(rows, &mean);
+            const double cost = march_cost(waves, mean, b->fuse.steps, cus);
+            if (rows == 8u || cost < best)
+            {
+                best = cost;
+                best_rows = rows;
+            }
+        }
+        for (uint32_t d = 0; d < b->doms.size(); ++d)
+        {
+            const uint32_t inner = b->doms[d].V - 2u, strips = march_strips(b->storage, b->doms[d].H - 2u);
+            const uint32_t segs = (inner + best_rows - 1u) / best_rows;
+            for (uint32_t s = 0; s < segs; ++s)
+                for (uint32_t x = 0; x < strips; ++x)
+                    parts.push_back(BatchPart{d, x, 1u + uint32_t(uint64_t(inner) * s / segs),
+                                              1u + uint32_t(uint64_t(inner) * (s + 1u) / segs)});
+        }
+    }
+    b->nparts = uint32_t(parts.size());
+    BATCH_TRY(hipMalloc(&b->d_parts, std::max<size_t>(1, parts.size()) * sizeof(BatchPart)));
+    BATCH_TRY(hipMemcpy(b->d_parts, parts.data(), parts.size() * sizeof(BatchPart), hipMemcpyHostToDevice));
+    return LBM_OK;
+}
+
+// `steps` steps of every domain, several per launch; *cur: the arena read
+// first and, afterwards, the one that holds the last step.
+int run_persistent_steps(lbm_batch *b, uint32_t steps, int *cur)
 {
     const uint32_t grid = std::max(1u, std::min(b->ntiles, b->persistent_grid));
-    for (uint32_t i = 0; i < steps; ++i)
-        if (int rc = step_dispatch(b, int((first_iteration + i) & 1u), i + 1 == steps, b->d_tiles, b->ntiles, grid))
-            return rc;
+    for (uint32_t left = steps; left; *cur ^= 1)
+    {
+        const uint32_t n = first_chunk(b->fuse, left);
+        left -= n;
+        if (n == 1u)
+        {
+            if (int rc = step_dispatch(b, *cur, left == 0u, b->d_tiles, b->ntiles, grid))
+                return rc;
+            continue;
+        }
+        const BatchFused a{b->d_doms,
+                           b->d_parts,
+                           b->arena[*cur],
+                           b->arena[1 - *cur],
+                           b->codes,
+                           b->res,
+                           b->uy,
+                           *cur,
+                           left == 0u ? 1u : 0u,
+                           b->nan_protection ? 1u : 0u,
+                           b->ones};
+        if (b->fuse.tiles)
+            batch_tile_launch(b->storage, n, b->fuse.steps - 1u, b->fuse.shape, a, b->nparts, b->stream);
+        else
+            batch_march_launch(b->storage, n, a, b->nparts, b->stream);
+        BATCH_TRY(hipGetLastError());
+    }
     return LBM_OK;
 }
 
@@ -431,6 +512,7 @@ void lbm_batch_destroy(lbm_batch *b)
     (void)hipFree(b->uy);
     (void)hipFree(b->d_doms);
     (void)hipFree(b->d_tiles);
+    (void)hipFree(b->d_parts);
     (void)hipFree(b->snap);
     (void)hipFree(b->ones);
     if (b->ev0)
@@ -532,6 +614,8 @@ int lbm_batch_create(const lbm_batch_domain *domains, uint32_t count, int32_t st
 #undef CREATE_TRY
     if (int rc = build_tiles(b))
         return cleanup(rc);
+    if (int rc = build_parts(b, cus))
+        return cleanup(rc);
     *out = b;
     return LBM_OK;
 }
@@ -570,7 +654,7 @@ int lbm_batch_init(lbm_batch *b)
     // set-up, so that lbm_batch_residuals_noalloc never allocates
     if (!b->snap)
         BATCH_TRY(hipMalloc(&b->snap, 2ull * b->code_nodes * sizeof(double)));
-    b->iteration = 0;
+    b->cur = 0;
     b->initialized = true;
     b->snap_valid = false;
     return LBM_OK;
@@ -586,14 +670,15 @@ int lbm_batch_run(lbm_batch *b, uint32_t steps, int32_t mode)
         return lbm_set_error(LBM_ERR_INVALID_ARGUMENT, "lbm_batch_run: unknown mode");
     if (steps == 0)
         return LBM_OK;
-    const int parity0 = int(b->iteration & 1u);
+    const int parity0 = b->cur;
     if (mode == LBM_BATCH_GRAPH && (b->graph_steps != steps || b->graph_parity != parity0))
     {
         // capture the persistent launches of the whole run once per (steps, parity)
         drop_graph(b);
         hipGraph_t g = nullptr;
         BATCH_TRY(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
-        int rc = run_persistent_steps(b, steps, b->iteration);
+        b->graph_end = parity0;
+        int rc = run_persistent_steps(b, steps, &b->graph_end);
         hipError_t e = hipStreamEndCapture(b->stream, &g);
         if (rc)
             return rc;
@@ -607,20 +692,24 @@ int lbm_batch_run(lbm_batch *b, uint32_t steps, int32_t mode)
         b->graph_parity = parity0;
     }
     BATCH_TRY(hipEventRecord(b->ev0, b->stream));
+    int end = parity0;
     if (mode == LBM_BATCH_GRAPH)
+    {
         BATCH_TRY(hipGraphLaunch(b->graph, b->stream));
+        end = b->graph_end;
+    }
     else if (mode == LBM_BATCH_PERSISTENT)
     {
-        if (int rc = run_persistent_steps(b, steps, b->iteration))
+        if (int rc = run_persistent_steps(b, steps, &end))
             return rc;
     }
     else
     {
-        for (uint32_t i = 0; i < steps; ++i)
+        for (uint32_t i = 0; i < steps; ++i, end ^= 1)
             for (size_t d = 0; d < b->doms.size(); ++d)
                 if (b->tile_count[d])
-                    if (int rc = step_dispatch(b, int((b->iteration + i) & 1u), i + 1 == steps,
-                                               b->d_tiles + b->tile_first[d], b->tile_count[d], b->tile_count[d]))
+                    if (int rc = step_dispatch(b, end, i + 1 == steps, b->d_tiles + b->tile_first[d],
+                                               b->tile_count[d], b->tile_count[d]))
                         return rc;
     }
     BATCH_TRY(hipEventRecord(b->ev1, b->stream));
@@ -628,7 +717,7 @@ int lbm_batch_run(lbm_batch *b, uint32_t steps, int32_t mode)
     float ms = 0.f;
     BATCH_TRY(hipEventElapsedTime(&ms, b->ev0, b->ev1));
     b->last_ms = ms;
-    b->iteration += steps;
+    b->cur = end;
     return LBM_OK;
 }
 
@@ -744,7 +833,7 @@ int lbm_batch_residuals(lbm_batch *b, double *out, uint32_t count)
     }
     double *partials = nullptr;
     BATCH_TRY(hipMalloc(&partials, 2ull * std::max(1u, b->ntiles) * sizeof(double)));
-    const void *src = b->arena[b->iteration & 1u];
+    const void *src = b->arena[b->cur];
     switch (b->storage)
     {
     case LBM_STORE_F64:
@@ -815,7 +904,7 @@ int lbm_batch_residuals_noalloc(lbm_batch *b, double *out, uint32_t count)
     }
     double *partials = b->scratch;
     double *residuals = b->scratch + 2ull * kScratchTiles;
-    const void *src = b->arena[b->iteration & 1u];
+    const void *src = b->arena[b->cur];
     switch (b->storage)
     {
     case LBM_STORE_F64:
@@ -851,7 +940,7 @@ int lbm_batch_reset_domain(lbm_batch *b, uint32_t domain)
     if (!b->initialized)
         return lbm_set_error(LBM_ERR_STATE, "lbm_batch_reset_domain: call lbm_batch_init first");
     const BatchDom &dm = b->doms[domain];
-    void *lat = b->arena[b->iteration & 1u];
+    void *lat = b->arena[b->cur];
     int rc = LBM_OK;
     switch (b->storage)
     {
@@ -886,7 +975,7 @@ int lbm_batch_set_equilibrium(lbm_batch *b, uint32_t domain, const double *rho, 
     for (int k = 0; k < 3 && e == hipSuccess; ++k)
         e = hipMemcpyAsync(tmp + k * count, src[k], count * sizeof(double), hipMemcpyHostToDevice, b->stream);
     const Geom g = batch_geom(dm, b->ones);
-    void *lat = b->arena[b->iteration & 1u];
+    void *lat = b->arena[b->cur];
     if (e == hipSuccess)
     {
         const dim3 grid((g.N + 255u) / 256u), block(256);

@@ -134,30 +134,28 @@ constexpr int march_phases()
     return Lane<S>::N == 4 ? 1 : 3;
 }
 
+template <int L>
+using MarchLds = u32x4[2][L == LBM_LAYOUT_STREAM ? 1 : 320];  // a wave's two row slots (not used in the stream layout)
+
+// One wave: column strip `strip`, rows y0 to y1 - 1 of the lattice that p
+// describes.
 template <int L, int S, int T>
-__global__ __launch_bounds__(MARCH_BLOCK, 2) void k_march(MarchParams a)
+__device__ __forceinline__ void march_wave(const StepParams &p, const uint32_t (&sr)[kFusedMaxSteps], uint32_t strip,
+                                           int y0, int y1, MarchLds<L> &lds)
 {
     using E = typename Storage<S>::T;
     using C = typename Storage<S>::C;
     constexpr int N = Lane<S>::N, CW = Lane<S>::CW;
     constexpr int K = L == LBM_LAYOUT_COLLISION ? 9 : (L == LBM_LAYOUT_BUNDLE ? 3 : 1), NA = 9 / K;
     constexpr int VA = 64 * K / 2;  // 16-byte vectors of a window in one array
-    __shared__ u32x4 lds[MARCH_BLOCK / 64][2][L == LBM_LAYOUT_STREAM ? 1 : 320];
-    // the wave's own slot of row j
-    auto lds_of = [&](int j) { return lds[__builtin_amdgcn_readfirstlane(threadIdx.x / 64)][j & 1]; };
+    auto lds_of = [&](int j) { return lds[j & 1]; };  // the slot of row j
     auto wave_sync = [] { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); };
-    const StepParams &p = a.p;
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * (MARCH_BLOCK / 64) + threadIdx.x / 64);
-    if (wave >= a.strips * a.segs)
-        return;
     const int lane = int(threadIdx.x & 63u);
-    const uint32_t seg = wave / a.strips, strip = wave - seg * a.strips;
     const int Hx = int(p.Hx), Vx = int(p.Vx);
     const int xw = 1 + int(strip) * (MARCH_OWN * N) - MARCH_HALO * N;  // the window's first column
     const int x = xw + lane * N;
     const bool in_range = x <= Hx - 1 && x + N - 1 >= 0;
     const bool owned = lane >= MARCH_HALO && lane < 64 - MARCH_HALO;
-    const int y0 = 1 + int(seg * a.rows), y1 = min(y0 + int(a.rows), Vx - 1);
     const int jb = max(y0 - T, 0), je = y1 - 1 + T;
     const E *src = static_cast<const E *>(p.src);
     E *dst = static_cast<E *>(p.dst);
@@ -413,7 +411,7 @@ __global__ __launch_bounds__(MARCH_BLOCK, 2) void k_march(MarchParams a)
                 else
                     write_moments<C>(p, c, uint32_t(x + i), uint32_t(r), rho, jx, jy, usq);
             }
-            node_bits<S>(f[i], uint32_t(r) * p.P + lp + uint32_t(i), a.sr[k - 1], t[i], 0.f);
+            node_bits<S>(f[i], uint32_t(r) * p.P + lp + uint32_t(i), sr[k - 1], t[i], 0.f);
         }
         u32x2 out[9];
 #pragma unroll
@@ -647,26 +645,43 @@ __global__ __launch_bounds__(MARCH_BLOCK, 2) void k_march(MarchParams a)
 }
 
 template <int L, int S, int T>
+__global__ __launch_bounds__(MARCH_BLOCK, 2) void k_march(MarchParams a)
+{
+    __shared__ MarchLds<L> lds[MARCH_BLOCK / 64];
+    const uint32_t in_block = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    const uint32_t wave = blockIdx.x * (MARCH_BLOCK / 64) + in_block;
+    if (wave >= a.strips * a.segs)
+        return;
+    const uint32_t seg = wave / a.strips, strip = wave - seg * a.strips;
+    const int y0 = 1 + int(seg * a.rows), y1 = min(y0 + int(a.rows), int(a.p.Vx) - 1);
+    march_wave<L, S, T>(a.p, a.sr, strip, y0, y1, lds[in_block]);
+}
+
+// The time of `waves` waves of `rows` rows each, in row visits.  A wave costs
+// rows + T + 1 of them; w waves come to each SIMD, which holds two at a time.
+// One left over runs alone and takes about 1.4 of its share of a pair; an
+// uneven end costs about a third of a wave.  (FP32 stream, 8192 x 2048,
+// T = 4: rows 76 / 50 / 38 / 30 / 25, that is 2 / 3 / 4 / 5 / 6 waves,
+// 106.7 / 117.4 / 102.5 / 112.3 / 103.4 us per step.)
+double march_cost(uint64_t waves, double rows, uint32_t steps, int cus)
+{
+    const uint64_t simds = uint64_t(std::max(cus, 1)) * 4u, each = (waves + simds - 1u) / simds;
+    return (double(each) + (each % 2u ? 0.4 : 0.0)) * (rows + steps + 1.0) + 0.3 * rows;
+}
+
+template <int L, int S, int T>
 static void launch(MarchParams m, int cus, hipStream_t stream)
 {
     constexpr uint32_t own = uint32_t(MARCH_OWN * Lane<S>::N);
     m.strips = (m.p.Hx - 2u + own - 1u) / own;
     const uint32_t inner = m.p.Vx - 2u;
-    // Rows per segment.  A wave costs rows + T + 1 row visits; w of them come
-    // to each SIMD, which holds two at a time.  One left over runs alone and
-    // takes about 1.4 of its share of a pair; an uneven end costs about a
-    // third of a wave.  (FP32 stream, 8192 x 2048, T = 4: rows 76 / 50 / 38 /
-    // 30 / 25, that is 2 / 3 / 4 / 5 / 6 waves, 106.7 / 117.4 / 102.5 / 112.3 /
-    // 103.4 us per step.)
     const uint32_t simds = uint32_t(std::max(cus, 1)) * 4u;
     double best = 0.0;
     for (uint32_t w = 1; w <= 12u; ++w)
     {
         const uint32_t most = std::max(1u, w * simds / m.strips);
         const uint32_t rows = std::max(4u, (inner + most - 1u) / most);
-        const uint32_t waves = m.strips * ((inner + rows - 1u) / rows);
-        const uint32_t each = (waves + simds - 1u) / simds;
-        const double cost = (each + (each % 2u ? 0.4 : 0.0)) * (rows + T + 1u) + 0.3 * rows;
+        const double cost = march_cost(m.strips * ((inner + rows - 1u) / rows), rows, T, cus);
         if (w == 1u || cost < best)
         {
             best = cost;
@@ -676,6 +691,49 @@ static void launch(MarchParams m, int cus, hipStream_t stream)
     m.segs = (inner + m.rows - 1u) / m.rows;
     const uint32_t blocks = (m.strips * m.segs + MARCH_BLOCK / 64 - 1u) / (MARCH_BLOCK / 64);
     hipLaunchKernelGGL((k_march<L, S, T>), dim3(blocks), dim3(MARCH_BLOCK), 0, stream, m);
+}
+
+// The same for the domains of a batch: each wave has its own domain, strip and rows.
+template <int S, int T>
+__global__ __launch_bounds__(MARCH_BLOCK, 2) void k_batch_march(BatchFused a, uint32_t waves)
+{
+    __shared__ MarchLds<LBM_LAYOUT_STREAM> lds[1];
+    const uint32_t wave = blockIdx.x * (MARCH_BLOCK / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    if (wave >= waves)
+        return;
+    const BatchPart part = a.parts[wave];
+    const StepParams p = batch_params<S>(a, part.dom);
+    constexpr uint32_t sr[kFusedMaxSteps] = {};
+    march_wave<LBM_LAYOUT_STREAM, S, T>(p, sr, part.x, int(part.y0), int(part.y1), lds[0]);
+}
+
+uint32_t march_strips(int storage, uint32_t inner_width)
+{
+    const uint32_t own = uint32_t(MARCH_OWN) * (storage == LBM_STORE_F64 ? 1u : (storage == LBM_STORE_F32 ? 2u : 4u));
+    return (inner_width + own - 1u) / own;
+}
+
+template <int S>
+static void batch_steps(uint32_t steps, const BatchFused &a, uint32_t waves, hipStream_t stream)
+{
+    const dim3 grid((waves + MARCH_BLOCK / 64 - 1u) / (MARCH_BLOCK / 64)), block(MARCH_BLOCK);
+    switch (steps)
+    {
+    case 2: hipLaunchKernelGGL((k_batch_march<S, 2>), grid, block, 0, stream, a, waves); break;
+    case 3: hipLaunchKernelGGL((k_batch_march<S, 3>), grid, block, 0, stream, a, waves); break;
+    default: hipLaunchKernelGGL((k_batch_march<S, 4>), grid, block, 0, stream, a, waves); break;
+    }
+}
+
+void batch_march_launch(int storage, uint32_t steps, const BatchFused &a, uint32_t waves, hipStream_t stream)
+{
+    switch (storage)
+    {
+    case LBM_STORE_F64: batch_steps<LBM_STORE_F64>(steps, a, waves, stream); break;
+    case LBM_STORE_F32: batch_steps<LBM_STORE_F32>(steps, a, waves, stream); break;
+    case LBM_STORE_F16_SHIFTED: batch_steps<LBM_STORE_F16_SHIFTED>(steps, a, waves, stream); break;
+    default: batch_steps<LBM_STORE_BF16_SHIFTED>(steps, a, waves, stream); break;
+    }
 }
 
 template <int L, int S>

@@ -74,9 +74,7 @@ struct lbm_ctx
     int cur = 0;          // index of the source lattice
     int uy_cur = 0;       // half of uycol that the next step reads
     int cus = 0;
-    uint32_t fuse_steps = 1;  // steps per launch, at most
-    bool fuse_in_tiles = false;  // by k_tile_steps on regions of fuse_tile, else by k_march
-    TileShape fuse_tile = TileShape::k32x32;
+    FusePlan fuse;        // nptl / lptl: several steps per launch
     int8_t *phase = nullptr;
     uint16_t *code = nullptr;
     double *res = nullptr;    // 4 * D: rho, jx, jy, |j|
@@ -1798,8 +1796,8 @@ struct Impl
         m.p = params(c, macros);
         for (uint32_t k = 0; k < n; ++k)
             m.sr[k] = c->desc.rounding == LBM_ROUND_STOCHASTIC ? (step_seed(c->iteration + k) | 1u) : 0u;
-        if (c->fuse_in_tiles)
-            tile_launch(L, S, n, c->fuse_tile, m, c->stream);
+        if (c->fuse.tiles)
+            tile_launch(L, S, n, c->fuse.shape, m, c->stream);
         else
             march_launch(L, S, n, m, c->cus, c->stream);
         LBM_HIP_TRY(hipGetLastError());
@@ -2103,31 +2101,6 @@ int lbm_device_name(char *buf, size_t len)
     return LBM_OK;
 }
 
-// How nptl and lptl put several steps into one launch.  Small lattices are
-// bound by the launch itself and then by the latency of a step: blocks hold a
-// region of nodes in LDS for several steps (k_tile_steps), the region small
-// enough that every compute unit gets one.  Large lattices are bound by HBM:
-// marching waves read each row once (k_march).  us per step on porous
-// channels (FP64 stream / FP32 stream / FP16 collision), one step per launch,
-// then the shapes around the choice:
-//   256 x 64     3.8 / 3.6 / 4.6     16x16 T 5: 1.25 / 1.23 / 1.45    32x16 T 6: 1.42 / 1.30 / 1.44
-//   512 x 128    4.5 / 3.8 / 5.0     32x32 T 6: 2.12 / 1.75 / 1.73    16x16 T 5: 2.41 / 2.04 / 1.99
-//   1024 x 256   10.2 / 6.1 / 6.3    32x32 T 5: 4.69 / 3.73 / 3.65    32x16 T 4: 4.38 / 3.82 / 3.90
-//   2048 x 512   29.5 / 16.1 / 16.3  32x16 T 4: 12.6 / 10.7 / 11.1    march:     14.6 / 13.0 / 20.3
-//   4096 x 1024  112 / 55.8 / 48.9   32x16 T 4: 59.0 / 42.9 / 38.7    march:     45.4 / 32.7 / 37.5
-static void plan_fusion(lbm_ctx *c)
-{
-    const uint64_t nodes = uint64_t(c->Hx - 2u) * (c->Vx - 2u);
-    if (nodes >= (c->elem == 8 ? 1500000u : (c->elem == 4 ? 2000000u : 3500000u)))
-    {
-        c->fuse_steps = kMarchMaxSteps;
-        return;
-    }
-    c->fuse_in_tiles = true;
-    c->fuse_tile = nodes <= 36000u ? TileShape::k16x16 : (nodes <= 500000u ? TileShape::k32x32 : TileShape::k32x16);
-    c->fuse_steps = nodes <= 36000u ? 5u : (nodes <= 130000u ? 6u : (nodes <= 500000u ? 5u : 4u));
-}
-
 static int validate_desc(const lbm_desc *d)
 {
     if (d->algorithm < LBM_ALG_NPTL || d->algorithm > LBM_ALG_NSOL)
@@ -2325,9 +2298,7 @@ int lbm_create(const lbm_desc *desc, lbm_ctx **out)
     // 1024, 3844 tiles, 154 / 174).
     size_t side_bytes = 0;
     int cus = 0;
-    uint32_t fuse_steps = 1;  // steps per launch, at most
-    bool fuse_in_tiles = false;  // by k_tile_steps on regions of fuse_tile, else by k_march
-    TileShape fuse_tile = TileShape::k32x32;
+    FusePlan fuse;        // nptl / lptl: several steps per launch
     {
         int dev = 0;
         CREATE_TRY(hipGetDevice(&dev));
@@ -2375,7 +2346,7 @@ int lbm_create(const lbm_desc *desc, lbm_ctx **out)
     }
     c->cus = cus;
     if (c->two_lattice)
-        plan_fusion(c);
+        c->fuse = plan_fusion(c->elem, uint64_t(c->Hx - 2u) * (c->Vx - 2u));
     CREATE_TRY(hipMalloc(&c->lat[0], lat_bytes + std::max<size_t>(64, side_bytes)));
     if (c->two_lattice)
         CREATE_TRY(hipMalloc(&c->lat[1], lat_bytes + 64));
@@ -2533,7 +2504,7 @@ int lbm_get_node_codes(lbm_ctx *c, uint16_t *codes, size_t n)
 // rho_ref (that step runs alone).
 static uint32_t fused_steps(const lbm_ctx *c, uint32_t left, uint32_t frame_interval)
 {
-    if (c->fuse_steps < 2u)
+    if (c->fuse.steps < 2u)
         return 1;
     uint32_t n = left;
     if (frame_interval)
@@ -2543,9 +2514,7 @@ static uint32_t fused_steps(const lbm_ctx *c, uint32_t left, uint32_t frame_inte
         const uint32_t at = uint32_t(c->iteration % kRefInterval);
         n = at == 0u && c->iteration ? 1u : std::min(n, kRefInterval - at);
     }
-    // as few launches as there can be, of nearly the same length
-    const uint32_t launches = (n + c->fuse_steps - 1u) / c->fuse_steps;
-    return (n + launches - 1u) / launches;
+    return first_chunk(c->fuse, n);
 }
 
 // The next launch of a run: how many steps, and what its last one writes.

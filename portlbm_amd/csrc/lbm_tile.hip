@@ -21,8 +21,11 @@
 namespace lbm_dev
 {
 
+// One block: stores the nodes from (x0, y0) on that lie at least `halo` nodes
+// inside its region (steps <= halo + 1).
 template <int L, int S, int W, int H>
-__global__ __launch_bounds__(W * H) void k_tile_steps(MarchParams a, uint32_t steps)
+__device__ __forceinline__ void tile_block(const StepParams &p, const uint32_t (&sr)[kFusedMaxSteps], uint32_t steps,
+                                           int halo, int x0, int y0)
 {
     using E = typename Storage<S>::T;
     using C = typename Storage<S>::C;
@@ -30,10 +33,9 @@ __global__ __launch_bounds__(W * H) void k_tile_steps(MarchParams a, uint32_t st
     __shared__ E pop[2][9][NT];
     __shared__ C uy[2][H];
     __shared__ uint16_t codes[NT];
-    const StepParams &p = a.p;
     const E *src = static_cast<const E *>(p.src);
-    const int tid = int(threadIdx.x), tx = tid % W, ty = tid / W, halo = int(steps) - 1;
-    const int x = 1 + int(blockIdx.x) * (W - 2 * halo) - halo + tx, y = 1 + int(blockIdx.y) * (H - 2 * halo) - halo + ty;
+    const int tid = int(threadIdx.x), tx = tid % W, ty = tid / W;
+    const int x = x0 - halo + tx, y = y0 - halo + ty;
     const bool inside = x >= 0 && y >= 0 && x < int(p.Hx) && y < int(p.Vx);
     const bool inner = x >= 1 && y >= 1 && x <= int(p.Hx) - 2 && y <= int(p.Vx) - 2;
     const uint32_t pn = inside ? place(uint32_t(x), uint32_t(y), p.P, p.X0) : 0u;
@@ -55,7 +57,7 @@ __global__ __launch_bounds__(W * H) void k_tile_steps(MarchParams a, uint32_t st
     for (uint32_t k = 1;; ++k)
     {
         const uint32_t b = k & 1u;  // step k leaves its populations in pop[b]
-        if (fluid && depth >= int(k) - 1)
+        if (fluid && depth >= (k < steps ? int(k) - 1 : halo))
         {
             if (k > 1u)
             {
@@ -79,7 +81,7 @@ __global__ __launch_bounds__(W * H) void k_tile_steps(MarchParams a, uint32_t st
             C rho, jx, jy, usq;
             collide_node<C, Storage<S>::kPromote, Storage<S>::kFull>(f, C(p.omega), rho, jx, jy, usq);
             E t[9];
-            node_bits<S>(f, pn, a.sr[k - 1u], t, 0.f);
+            node_bits<S>(f, pn, sr[k - 1u], t, 0.f);
             if (k < steps)
             {
                 if (code & LBM_CODE_UY_SOURCE)
@@ -105,6 +107,24 @@ __global__ __launch_bounds__(W * H) void k_tile_steps(MarchParams a, uint32_t st
             break;
         __syncthreads();
     }
+}
+
+template <int L, int S, int W, int H>
+__global__ __launch_bounds__(W * H) void k_tile_steps(MarchParams a, uint32_t steps)
+{
+    const int halo = int(steps) - 1;
+    tile_block<L, S, W, H>(a.p, a.sr, steps, halo, 1 + int(blockIdx.x) * (W - 2 * halo),
+                           1 + int(blockIdx.y) * (H - 2 * halo));
+}
+
+// The same for the domains of a batch: each block has its own domain and first node.
+template <int S, int W, int H>
+__global__ __launch_bounds__(W * H) void k_batch_tiles(BatchFused a, uint32_t steps, int halo)
+{
+    const BatchPart part = a.parts[blockIdx.x];
+    const StepParams p = batch_params<S>(a, part.dom);
+    constexpr uint32_t sr[kFusedMaxSteps] = {};
+    tile_block<LBM_LAYOUT_STREAM, S, W, H>(p, sr, steps, halo, int(part.x), int(part.y0));
 }
 
 template <int L, int S, int W, int H>
@@ -144,6 +164,36 @@ void tile_launch(int layout, int storage, uint32_t steps, TileShape shape, const
     case LBM_STORE_F32: by_layout(std::integral_constant<int, LBM_STORE_F32>{}); break;
     case LBM_STORE_F16_SHIFTED: by_layout(std::integral_constant<int, LBM_STORE_F16_SHIFTED>{}); break;
     default: by_layout(std::integral_constant<int, LBM_STORE_BF16_SHIFTED>{}); break;
+    }
+}
+
+template <int S>
+static void batch_shape(uint32_t steps, int halo, TileShape shape, const BatchFused &a, uint32_t blocks,
+                        hipStream_t stream)
+{
+    switch (shape)
+    {
+    case TileShape::k16x16:
+        hipLaunchKernelGGL((k_batch_tiles<S, 16, 16>), dim3(blocks), dim3(256), 0, stream, a, steps, halo);
+        break;
+    case TileShape::k32x16:
+        hipLaunchKernelGGL((k_batch_tiles<S, 32, 16>), dim3(blocks), dim3(512), 0, stream, a, steps, halo);
+        break;
+    default:
+        hipLaunchKernelGGL((k_batch_tiles<S, 32, 32>), dim3(blocks), dim3(1024), 0, stream, a, steps, halo);
+        break;
+    }
+}
+
+void batch_tile_launch(int storage, uint32_t steps, uint32_t halo, TileShape shape, const BatchFused &a,
+                       uint32_t blocks, hipStream_t stream)
+{
+    switch (storage)
+    {
+    case LBM_STORE_F64: batch_shape<LBM_STORE_F64>(steps, int(halo), shape, a, blocks, stream); break;
+    case LBM_STORE_F32: batch_shape<LBM_STORE_F32>(steps, int(halo), shape, a, blocks, stream); break;
+    case LBM_STORE_F16_SHIFTED: batch_shape<LBM_STORE_F16_SHIFTED>(steps, int(halo), shape, a, blocks, stream); break;
+    default: batch_shape<LBM_STORE_BF16_SHIFTED>(steps, int(halo), shape, a, blocks, stream); break;
     }
 }
 

@@ -124,3 +124,29 @@ def test_diverging_flow_keeps_its_infinities(storage, size):
         many.run(8)
         assert not np.all(np.isfinite(one.populations()))
         assert same(one.macros(), many.macros())
+
+
+@pytest.mark.parametrize("storage", ["f64", "f32", "f16-shifted", "bf16-shifted"])
+@pytest.mark.parametrize("count", [1, 3, 40, 130])
+def test_batched_domains(count, storage):
+    """Persistent and graph runs, several steps per launch, against one launch
+    per domain and step: few domains (LDS tiles) to many (marching waves)."""
+    rng = np.random.default_rng(count)
+    docs = []
+    for _ in range(count):
+        h, v = (int(rng.integers(a, b)) for a, b in ((4, 700 if count > 3 else 90), (4, 300 if count > 3 else 60)))
+        docs.append(pa.settings("lptl", "stream", inner_h=h, inner_v=v, scenario="porous-circles", time_steps=1,
+                                tau=float(rng.uniform(0.6, 0.9)), rho_in=float(rng.uniform(1.005, 1.03)),
+                                storage=storage, seed=int(rng.integers(1, 1 << 40)), porosity=0.8, radiusMin=2.0,
+                                radiusMax=5.0, obstacleMargin=2))
+    with pa.Batch(docs, storage=storage) as one, pa.Batch(docs, storage=storage) as many:
+        for steps, mode in ((9, "persistent"), (14, "graph"), (14, "graph"), (1, "graph"), (5, "persistent")):
+            one.run(steps, "per-domain")
+            many.run(steps, mode)
+        one.residuals()
+        many.residuals()
+        one.run(7, "per-domain")
+        many.run(7, "graph")
+        assert np.array_equal(one.residuals(), many.residuals(), equal_nan=True)
+        for d in range(count):
+            assert same(one.macros(d), many.macros(d))
