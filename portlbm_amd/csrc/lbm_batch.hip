@@ -17,6 +17,7 @@
 #include "lbm_error.hpp"
 #include "lbm_march.hpp"
 #include "lbm_setup.hpp"
+#include "lbm_transfer.hpp"
 
 using namespace lbm_dev;
 
@@ -522,6 +523,7 @@ void lbm_batch_destroy(lbm_batch *b)
     if (b->stream)
         (void)hipStreamDestroy(b->stream);
     delete b;
+    release_staging();
 }
 
 int lbm_batch_create(const lbm_batch_domain *domains, uint32_t count, int32_t storage, int32_t nan_protection,
@@ -533,6 +535,7 @@ int lbm_batch_create(const lbm_batch_domain *domains, uint32_t count, int32_t st
         return lbm_set_error(LBM_ERR_INVALID_ARGUMENT, "lbm_batch_create: unknown storage type");
     *out = nullptr;
     lbm_batch *b = new lbm_batch();
+    hold_staging();
     b->storage = storage;
     b->nan_protection = nan_protection;
     b->elem = store_bytes(storage);
@@ -547,7 +550,7 @@ int lbm_batch_create(const lbm_batch_domain *domains, uint32_t count, int32_t st
         if (ds.horizontal_nodes < 4 || ds.vertical_nodes < 4 || ds.horizontal_nodes > 65535 ||
             ds.vertical_nodes > 65535 || !(ds.relaxation_time > 0.0))
         {
-            delete b;
+            lbm_batch_destroy(b);
             return lbm_set_error(LBM_ERR_INVALID_ARGUMENT,
                                  "lbm_batch_create: domain " + std::to_string(d) + " has invalid extents or tau");
         }
@@ -571,7 +574,7 @@ int lbm_batch_create(const lbm_batch_domain *domains, uint32_t count, int32_t st
         b->phase_nodes += size_t(dm.H) * dm.V;
         if (b->code_nodes >= (1ull << 32) || b->res_doubles >= (1ull << 32) || 9ull * dm.S >= (1ull << 32))
         {
-            delete b;
+            lbm_batch_destroy(b);
             return lbm_set_error(LBM_ERR_INVALID_ARGUMENT, "lbm_batch_create: batch too large");
         }
     }
@@ -738,11 +741,12 @@ int lbm_batch_get_macros(lbm_batch *b, uint32_t domain, double *rho, double *jx,
     if (count != dm.D)
         return lbm_set_error(LBM_ERR_INVALID_ARGUMENT, "lbm_batch_get_macros: count must be (H-2)*(V-2)");
     double *dst[4] = {rho, jx, jy, jabs};
+    HostPiece pieces[4];
+    size_t n = 0;
     for (int k = 0; k < 4; ++k)
         if (dst[k])
-            BATCH_TRY(hipMemcpyAsync(dst[k], b->res + dm.res + size_t(k) * dm.D, count * sizeof(double),
-                                     hipMemcpyDeviceToHost, b->stream));
-    BATCH_TRY(hipStreamSynchronize(b->stream));
+            pieces[n++] = HostPiece{dst[k], b->res + dm.res + size_t(k) * dm.D, count * sizeof(double)};
+    BATCH_TRY(download(pieces, n, b->stream));
     return LBM_OK;
 }
 

@@ -22,6 +22,7 @@
 #include "lbm_error.hpp"
 #include "lbm_march.hpp"
 #include "lbm_setup.hpp"
+#include "lbm_transfer.hpp"
 
 using namespace lbm_dev;
 
@@ -2189,6 +2190,7 @@ void lbm_destroy(lbm_ctx *c)
     if (c->stream)
         (void)hipStreamDestroy(c->stream);
     delete c;
+    release_staging();
 }
 
 int lbm_create(const lbm_desc *desc, lbm_ctx **out)
@@ -2199,6 +2201,7 @@ int lbm_create(const lbm_desc *desc, lbm_ctx **out)
     if (int rc = validate_desc(desc))
         return rc;
     lbm_ctx *c = new lbm_ctx();
+    hold_staging();
     c->desc = *desc;
     c->H = desc->horizontal_nodes;
     c->V = desc->vertical_nodes;
@@ -2233,7 +2236,7 @@ int lbm_create(const lbm_desc *desc, lbm_ctx **out)
         const uint64_t Sd = (M + align_nodes - 1) / align_nodes * align_nodes + 512u / c->elem;
         if (9ull * Sd >= (1ull << 32))
         {
-            delete c;
+            lbm_destroy(c);
             return fail(LBM_ERR_INVALID_ARGUMENT, "lattice too large for 32-bit population indices");
         }
         c->Sd = uint32_t(Sd);
@@ -2766,11 +2769,12 @@ int lbm_get_macros(lbm_ctx *c, double *rho, double *jx, double *jy, double *jabs
     if (count != c->D)
         return fail(LBM_ERR_INVALID_ARGUMENT, "lbm_get_macros: count must equal (H-2)*(V-2)");
     double *dst[4] = {rho, jx, jy, jabs};
+    HostPiece pieces[4];
+    size_t n = 0;
     for (int k = 0; k < 4; ++k)
-        if (dst[k] && count)
-            LBM_HIP_TRY(hipMemcpyAsync(dst[k], c->res + size_t(k) * c->D, count * sizeof(double),
-                                       hipMemcpyDeviceToHost, c->stream));
-    LBM_HIP_TRY(hipStreamSynchronize(c->stream));
+        if (dst[k])
+            pieces[n++] = HostPiece{dst[k], c->res + size_t(k) * c->D, count * sizeof(double)};
+    LBM_HIP_TRY(download(pieces, n, c->stream));
     return LBM_OK;
 }
 
@@ -2964,8 +2968,8 @@ int lbm_get_populations(lbm_ctx *c, double *values, size_t count)
         const uint32_t n = uint32_t(std::min<size_t>(kStageDoubles, count - i0));
         if (int rc = vt.decode(c, c->stage, i0, n))
             return rc;
-        LBM_HIP_TRY(hipMemcpyAsync(values + i0, c->stage, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-        LBM_HIP_TRY(hipStreamSynchronize(c->stream));  // the next chunk reuses the staging buffer
+        const HostPiece piece{values + i0, c->stage, n * sizeof(double)};
+        LBM_HIP_TRY(download(&piece, 1, c->stream));  // the next chunk reuses the staging buffer
     }
     return LBM_OK;
 }

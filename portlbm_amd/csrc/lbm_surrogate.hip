@@ -27,6 +27,7 @@
 #include "lbm_error.hpp"
 #include "lbm_hip.h"
 #include "lbm_surrogate.h"
+#include "lbm_transfer.hpp"
 
 namespace
 {
@@ -848,6 +849,7 @@ void lbm_surrogate_destroy(lbm_surrogate *s)
     if (s->stream)
         (void)hipStreamDestroy(s->stream);
     delete s;
+    lbm_dev::release_staging();
 }
 
 int lbm_surrogate_create(uint32_t height, uint32_t width, uint32_t max_batch, lbm_surrogate **out)
@@ -861,6 +863,7 @@ int lbm_surrogate_create(uint32_t height, uint32_t width, uint32_t max_batch, lb
                              "lbm_surrogate_create: height and width must be positive multiples of 16 (<= 8192), "
                              "max_batch in 1..4096");
     auto *s = new lbm_surrogate;
+    lbm_dev::hold_staging();
     s->H = int(height);
     s->W = int(width);
     s->Bmax = int(max_batch);
@@ -1022,9 +1025,9 @@ static int predict(lbm_surrogate *s, const float *inputs, uint32_t batch, float 
                              size_t(B) * LBM_SURROGATE_INPUTS * hw * sizeof(float), hipMemcpyHostToDevice, s->stream));
         forward(s, B, bf16);
         S_TRY(hipGetLastError());
-        S_TRY(hipMemcpyAsync(outputs + size_t(b0) * LBM_SURROGATE_OUTPUTS * hw, s->out,
-                             size_t(B) * LBM_SURROGATE_OUTPUTS * hw * sizeof(float), hipMemcpyDeviceToHost,
-                             s->stream));
+        const lbm_dev::HostPiece piece{outputs + size_t(b0) * LBM_SURROGATE_OUTPUTS * hw, s->out,
+                                       size_t(B) * LBM_SURROGATE_OUTPUTS * hw * sizeof(float)};
+        S_TRY(lbm_dev::download(&piece, 1, s->stream));
     }
     S_TRY(hipEventRecord(s->ev1, s->stream));
     S_TRY(hipStreamSynchronize(s->stream));
@@ -1074,9 +1077,8 @@ int lbm_surrogate_loss_grad(lbm_surrogate *s, const float *inputs, const float *
     forward(s, int(batch));
     loss_backward(s, int(batch), norm, nullptr, 0);
     S_TRY(hipGetLastError());
-    S_TRY(hipMemcpyAsync(loss, s->loss_dev, sizeof(double), hipMemcpyDeviceToHost, s->stream));
-    S_TRY(hipMemcpyAsync(grad, s->grad, count * sizeof(float), hipMemcpyDeviceToHost, s->stream));
-    S_TRY(hipStreamSynchronize(s->stream));
+    const lbm_dev::HostPiece pieces[2] = {{loss, s->loss_dev, sizeof(double)}, {grad, s->grad, count * sizeof(float)}};
+    S_TRY(lbm_dev::download(pieces, 2, s->stream));
     return LBM_OK;
 }
 
