@@ -5,17 +5,17 @@
 //
 // Kernels (NCHW float32, 256-thread blocks):
 //   k_conv3x3_f32  implicit GEMM on the matrix cores in FP32
-//                  (v_mfma_f32_16x16x4f32): 4 output rows x 16 pixels per
-//                  block (one row per wave) for all output channels; the input
-//                  tile with its 1-node halo staged in LDS; weights packed
-//                  [Cout16][K16], K = 9 Cin in the weights' own (c, tap) order.
-//                  The data gradient is the same kernel on flipped, transposed
-//                  weights.
-//   k_conv_wgrad   16 x 16 (out, in) channel pairs per block, each thread one
-//                  pair's 9 taps + bias over a sliding 3x3 register window;
-//                  per-slice partials summed in two fixed-order stages
-//                  (32 slice groups in parallel, then the groups).
-//   pooling, upsampling, ReLU mask, loss and Adam: one thread per element.
+//                  (v_mfma_f32_16x16x4f32); the input tile with its 1-node
+//                  halo staged in LDS with the channels of a pixel together;
+//                  weights packed [Cout16][tap][Cin16].  The data gradient is
+//                  the same kernel on flipped, transposed weights.
+//   k_conv_wgrad   the weight gradient on the same instruction, pixels as the
+//                  inner dimension: a block has a 16 x 16 (out, in) channel
+//                  pair and a slice of the pixel tiles; the slices' partial
+//                  sums are added in a fixed order by k_wgrad_reduce, all
+//                  convolutions in one launch.
+//   pooling, upsampling, loss and Adam: one thread per element; the gradient
+//   kernels that finish a layer's gradient apply its ReLU mask as they store.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -36,11 +36,8 @@ constexpr int kConvs = LBM_SURROGATE_CONVS;
 constexpr int kCin[kConvs] = {4, 16, 16, 32, 32, 48, 48, 64, 64, 64, 48, 32, 16, 16};
 constexpr int kCout[kConvs] = {16, 16, 32, 32, 48, 48, 64, 64, 64, 48, 32, 16, 16, 3};
 
-constexpr int kTile = 16;                    // output tile edge (pixels)
-constexpr int kHalo = kTile + 2;             // input tile edge with halo
-constexpr int kHaloStride = kHalo * kHalo + 1;  // LDS floats per channel (odd: spreads banks)
-constexpr int kWgT = 16;                     // channel tile of the weight gradient
-constexpr int kGStride = kTile * kTile + 1;  // LDS floats per gradient channel
+constexpr int kTile = 16;  // pixel tile edge of the weight gradient
+constexpr int kWgT = 16;   // its channel tile
 
 constexpr double kPi = 3.14159265358979323846;
 
@@ -50,94 +47,127 @@ inline int round16(int c) { return (c + 15) / 16 * 16; }
 inline int conv_level(int k) { return k < 8 ? k / 2 : k == 8 ? 4 : k == 13 ? 0 : 12 - k; }
 
 // ---- FP32 convolution on the matrix cores ---------------------------------
-// y[b][o][p] = act(bias[o] + sum_k Wm[o][k] X[k][p]), k = c*9 + tap, with
-// v_mfma_f32_16x16x4f32 (A 16x4, B 4x16, FP32 products and accumulation).
+// y[b][o][p] = act(bias[o] + sum over tap, c of Wm[o][tap][c] X[c][p + tap]),
+// with v_mfma_f32_16x16x4f32 (A 16x4, B 4x16, FP32 products and accumulation).
 // Lane layout (the same as the BF16 instruction's, one element per lane):
 // A[i][kk] in lane i + 16 kk, B[kk][j] in lane j + 16 kk, D[i][j] in lane
 // j + 16 (i/4), element i%4.  Which k an operand slot kk carries is free as
-// long as A and B agree: in a 16-wide chunk at kc, MFMA s of the chunk gives
-// slot kk the k = kc + 4 kk + s, so that each lane reads its four A values
-// as one 16-byte load.  A 256-thread block computes 16 pixels of 4 rows (one
-// row per wave) for all output channels (at most 64: four 16-row tiles).
+// long as A and B agree: within a tap's 16 channels from c0 on, MFMA s gives
+// slot kk the channel c0 + 4 kk + s, so that a lane reads its four values of
+// either operand as one 16-byte load (LDS holds a pixel's channels together,
+// 4 floats of padding per pixel keep the 16 pixels of a read on different
+// banks).  A wave computes R rows of 16 pixels for CT tiles of 16 output
+// channels: R rows share each weight load, CT tiles each pixel load.
+//
+// A channel-major weight order and a channel plane per LDS row would need a
+// division per operand value and single-float LDS reads, and one row per wave
+// a weight load per pixel row: the 27 launches of a training batch of 16
+// samples of 256 x 256 took 2.34 ms that way and take 1.3 ms this way.  16 ->
+// 16 channels at 256 x 256, 16 samples: 136 -> 79 us, 61 TFLOP/s of 152
+// reachable, bound by the staging of the tile (134 MB moved would take 27 us).
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int kMfmaRows = 4;  // output rows per block (one per wave)
 constexpr int kMfmaCols = 16;
-constexpr int kMaxCoTiles = 4;  // Cout <= 64
 
-__global__ __launch_bounds__(256) void k_conv3x3_f32(const float *__restrict__ x, const float *__restrict__ wm,
-                                                     const float *__restrict__ bias, float *__restrict__ y, int Cin,
-                                                     int Cout, int Kp, int H, int W, int tiles_x, int relu)
+// A block's place (tile, sample) in a grid of (tiles, samples): the blocks that
+// one XCD gets (every eighth in launch order) are neighbours, so that the
+// halos and the lines that two tiles share are read into one L2.
+__device__ __forceinline__ void xcd_place(unsigned &tile, unsigned &sample)
 {
-    constexpr int TR = kMfmaRows + 2, TC = kMfmaCols + 2;
-    extern __shared__ float tile_f[];  // Cin x TR x TC
-    const int b = blockIdx.y;
-    const int x0 = int(blockIdx.x % unsigned(tiles_x)) * kMfmaCols;
-    const int y0 = int(blockIdx.x / unsigned(tiles_x)) * kMfmaRows;
-    const float *xb = x + size_t(b) * Cin * H * W;
-    for (int i = threadIdx.x; i < Cin * TR * TC; i += 256)
+    const unsigned total = gridDim.x * gridDim.y, at = blockIdx.y * gridDim.x + blockIdx.x;
+    const unsigned place = total % 8 == 0 ? (at % 8) * (total / 8) + at / 8 : at;
+    tile = place % gridDim.x;
+    sample = place / gridDim.x;
+}
+
+// relu: outputs below 0 become 0; mask (or null): outputs become 0 where it is
+// not above 0 (the ReLU derivative of the layer below, for a data gradient).
+template <int CT, int R>
+__global__ __launch_bounds__(256) void k_conv3x3_f32(const float *__restrict__ x, const float *__restrict__ wm,
+                                                     const float *__restrict__ bias, const float *__restrict__ mask,
+                                                     float *__restrict__ y, int Cin, int Cout, int H, int W,
+                                                     int tiles_x, int relu)
+{
+    constexpr int TR = 4 * R + 2, TC = kMfmaCols + 2;
+    extern __shared__ __align__(16) float tile_f[];  // TR x TC pixels x (Cin16 + 4)
+    const int CinP = (Cin + 15) / 16 * 16, stride = CinP + 4, Kp = 9 * CinP;
+    unsigned at, b;
+    xcd_place(at, b);
+    const int x0 = int(at % unsigned(tiles_x)) * kMfmaCols, y0 = int(at / unsigned(tiles_x)) * (4 * R);
+    const size_t plane = size_t(H) * W;
+    const float *xb = x + size_t(b) * Cin * plane;
+    for (int i = threadIdx.x; i < TR * TC * (CinP / 4); i += 256)
     {
-        const int c = i / (TR * TC), r = (i / TC) % TR, col = i % TC;
-        const int yy = y0 - 1 + r, xx = x0 - 1 + col;
-        float v = 0.f;
+        const int c = i / (TR * TC) * 4, px = i % (TR * TC);
+        const int yy = y0 - 1 + px / TC, xx = x0 - 1 + px % TC;
+        f32x4 v{0.f, 0.f, 0.f, 0.f};
         if (yy >= 0 && yy < H && xx >= 0 && xx < W)
-            v = xb[(size_t(c) * H + yy) * W + xx];
-        tile_f[i] = v;
+        {
+            const float *from = xb + size_t(c) * plane + size_t(yy) * W + xx;
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                if (c + q < Cin)
+                    v[q] = from[q * plane];
+        }
+        *reinterpret_cast<f32x4 *>(tile_f + px * stride + c) = v;
     }
     __syncthreads();
     const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
     const int j = lane % 16, kq = 4 * (lane / 16);
-    const int co_tiles = (Cout + 15) / 16;
-    const int K = 9 * Cin;
-    f32x4 acc[kMaxCoTiles];
+    const int t0 = int(blockIdx.z) * CT;  // first tile of output channels
+    f32x4 acc[CT][R];
 #pragma unroll
-    for (int t = 0; t < kMaxCoTiles; ++t)
-        acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int kc = 0; kc < Kp; kc += 16)
+    for (int t = 0; t < CT; ++t)
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+            acc[t][r] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const float *wl = wm + size_t(t0 * 16 + j) * Kp + kq;
+    const float *xl = tile_f + (wave * R * TC + j) * stride + kq;
+#pragma unroll
+    for (int tap = 0; tap < 9; ++tap)
     {
-        float bv[4];
-#pragma unroll
-        for (int s = 0; s < 4; ++s)
+        for (int c = 0; c < CinP; c += 16)
         {
-            const int k = kc + kq + s;
-            float v = 0.f;
-            if (k < K)
-            {
-                const int c = k / 9, tap = k - 9 * c;
-                v = tile_f[(c * TR + wave + tap / 3) * TC + j + tap % 3];
-            }
-            bv[s] = v;
-        }
+            f32x4 av[CT], bv[R];
 #pragma unroll
-        for (int t = 0; t < kMaxCoTiles; ++t)
-        {
-            if (t < co_tiles)
-            {
-                const f32x4 av = *reinterpret_cast<const f32x4 *>(wm + size_t(t * 16 + j) * Kp + kc + kq);
+            for (int t = 0; t < CT; ++t)
+                av[t] = *reinterpret_cast<const f32x4 *>(wl + size_t(t) * 16 * Kp + tap * CinP + c);
 #pragma unroll
-                for (int s = 0; s < 4; ++s)
-                    acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[s], bv[s], acc[t], 0, 0, 0);
-            }
+            for (int r = 0; r < R; ++r)
+                bv[r] = *reinterpret_cast<const f32x4 *>(xl + ((r + tap / 3) * TC + tap % 3) * stride + c);
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+#pragma unroll
+                for (int t = 0; t < CT; ++t)
+#pragma unroll
+                    for (int r = 0; r < R; ++r)
+                        acc[t][r] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[t][s], bv[r][s], acc[t][r], 0, 0, 0);
         }
     }
-    const int oy = y0 + wave, ox = x0 + j;
-    if (oy >= H || ox >= W)
-        return;
+    const int ox = x0 + j;
 #pragma unroll
-    for (int t = 0; t < kMaxCoTiles; ++t)
+    for (int r = 0; r < R; ++r)
     {
-        if (t >= co_tiles)
-            break;
+        const int oy = y0 + wave * R + r;
+        if (oy >= H || ox >= W)
+            continue;
 #pragma unroll
-        for (int v = 0; v < 4; ++v)
+        for (int t = 0; t < CT; ++t)
         {
-            const int co = t * 16 + kq + v;
-            if (co < Cout)
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
             {
-                float r = acc[t][v] + (bias ? bias[co] : 0.f);
-                if (relu)
-                    r = r > 0.f ? r : 0.f;
-                y[((size_t(b) * Cout + co) * H + oy) * W + ox] = r;
+                const int co = (t0 + t) * 16 + kq + v;
+                if (co < Cout)
+                {
+                    const size_t to = (size_t(b) * Cout + co) * plane + size_t(oy) * W + ox;
+                    float o = acc[t][r][v] + (bias ? bias[co] : 0.f);
+                    if (relu)
+                        o = o > 0.f ? o : 0.f;
+                    if (mask && !(mask[to] > 0.f))
+                        o = 0.f;
+                    y[to] = o;
+                }
             }
         }
     }
@@ -145,145 +175,189 @@ __global__ __launch_bounds__(256) void k_conv3x3_f32(const float *__restrict__ x
 
 // Partial weight/bias gradient of one slice of (sample, tile) pairs:
 // partial[((slice*CoutP + o)*CinP + c)*10 + k] = sum g[b,o,i,j] x[b,c,i+ky-1,j+kx-1] (k < 9),
-// slot 9 = sum g[b,o,i,j].
+// slot 9 = sum g[b,o,i,j].  Per 16-pixel row of a tile and tap, four
+// v_mfma_f32_16x16x4f32 with A = g (16 output channels x 4 pixels) and B = x
+// (4 pixels x 16 input channels); slot kk of MFMA s is pixel 4 kk + s.  A
+// lane's six pixels of an input row serve the three taps of that row.  A wave
+// takes four rows of the tile; the four waves' sums are added in wave order.
+// The strides put the 16 channels of a read on different banks.
+//
+// Bound by the staging: the loads of a tile are all issued before the barrier
+// that ends the tile before it.  16 x 16 channels, 16 samples of 256 x 256: 70
+// us; 96 us with a loop of guarded loads.  All convolutions of that batch with
+// their reductions: 1.38 ms with one thread per channel pair (no matrix unit,
+// four times the slices, two reduction launches each), 0.65 ms this way.
+constexpr int kGStride = kTile * kTile + 4;
+constexpr int kXRow = kTile + 4, kXStride = (kTile + 2) * kXRow + 4;
+
 __global__ __launch_bounds__(256) void k_conv_wgrad(const float *__restrict__ x, const float *__restrict__ g,
                                                     float *__restrict__ partial, int B, int Cin, int Cout, int CinP,
                                                     int CoutP, int H, int W, int tiles_x, int tiles_per_image,
                                                     int slices)
 {
-    __shared__ float gs[kWgT * kGStride];
-    __shared__ float xs[kWgT * kHaloStride];
+    __shared__ __align__(16) float lds[kWgT * (kGStride + kXStride)];
+    float *gs = lds, *xs = lds + kWgT * kGStride;
+    static_assert(3 * 9 * 256 + 3 * 64 <= kWgT * (kGStride + kXStride), "the waves' sums fit");
     const int ci_tiles = CinP / kWgT;
     const int co0 = int(blockIdx.x / unsigned(ci_tiles)) * kWgT, ci0 = int(blockIdx.x % unsigned(ci_tiles)) * kWgT;
-    const int ol = threadIdx.x / kWgT, cl = threadIdx.x % kWgT;
-    float acc[10];
+    const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, ch = lane % 16, kk = 4 * (lane / 16);
+    f32x4 acc[9];
 #pragma unroll
-    for (int k = 0; k < 10; ++k)
-        acc[k] = 0.f;
+    for (int k = 0; k < 9; ++k)
+        acc[k] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float bsum = 0.f;
     const int total = B * tiles_per_image;
     for (int t = blockIdx.y; t < total; t += slices)
     {
         const int b = t / tiles_per_image, tt = t % tiles_per_image;
         const int tx0 = (tt % tiles_x) * kTile, ty0 = (tt / tiles_x) * kTile;
-        __syncthreads();
-        for (int i = threadIdx.x; i < kWgT * kTile * kTile; i += 256)
-        {
-            const int c = i / (kTile * kTile), p = i % (kTile * kTile);
-            const int yy = ty0 + p / kTile, xx = tx0 + p % kTile;
-            float v = 0.f;
-            if (co0 + c < Cout && yy < H && xx < W)
-                v = g[((size_t(b) * Cout + co0 + c) * H + yy) * W + xx];
-            gs[c * kGStride + p] = v;
-        }
-        for (int i = threadIdx.x; i < kWgT * kHalo * kHalo; i += 256)
-        {
-            const int c = i / (kHalo * kHalo), r = i % (kHalo * kHalo);
-            const int yy = ty0 + r / kHalo - 1, xx = tx0 + r % kHalo - 1;
-            float v = 0.f;
-            if (ci0 + c < Cin && yy >= 0 && yy < H && xx >= 0 && xx < W)
-                v = x[((size_t(b) * Cin + ci0 + c) * H + yy) * W + xx];
-            xs[c * kHaloStride + r] = v;
-        }
-        __syncthreads();
-        const float *xr = xs + cl * kHaloStride;
-        const float *gr = gs + ol * kGStride;
+        // Sixteen threads per channel, one per column: every load of a thread
+        // is a fixed number of rows from its first, and none waits for
+        // another; the columns left and right of the tile come last.
+        const int c = threadIdx.x / kTile, col = threadIdx.x % kTile;
+        const float *gc = g + (size_t(b) * Cout + min(co0 + c, Cout - 1)) * H * W;
+        const float *xc = x + (size_t(b) * Cin + min(ci0 + c, Cin - 1)) * H * W;
+        const bool gin = co0 + c < Cout && tx0 + col < W, xin = ci0 + c < Cin;
+        float gv[kTile], xv[kTile + 2], ev[3];
+#pragma unroll
         for (int r = 0; r < kTile; ++r)
         {
-            float w0[3], w1[3], w2[3];
-            w0[0] = xr[r * kHalo];
-            w0[1] = xr[r * kHalo + 1];
-            w1[0] = xr[(r + 1) * kHalo];
-            w1[1] = xr[(r + 1) * kHalo + 1];
-            w2[0] = xr[(r + 2) * kHalo];
-            w2[1] = xr[(r + 2) * kHalo + 1];
-#pragma unroll 4
-            for (int c = 0; c < kTile; ++c)
+            const bool in = gin && ty0 + r < H;
+            gv[r] = gc[in ? (ty0 + r) * W + tx0 + col : 0];
+            gv[r] = in ? gv[r] : 0.f;
+        }
+#pragma unroll
+        for (int r = 0; r < kTile + 2; ++r)
+        {
+            const int yy = ty0 + r - 1;
+            const bool in = xin && tx0 + col < W && yy >= 0 && yy < H;
+            xv[r] = xc[in ? yy * W + tx0 + col : 0];
+            xv[r] = in ? xv[r] : 0.f;
+        }
+#pragma unroll
+        for (int e = 0; e < 3; ++e)
+        {
+            const int i = col + e * kTile, yy = ty0 + i / 2 - 1, xx = tx0 + (i % 2 ? kTile : -1);
+            const bool in = xin && i < 2 * (kTile + 2) && xx >= 0 && xx < W && yy >= 0 && yy < H;
+            ev[e] = xc[in ? yy * W + xx : 0];
+            ev[e] = in ? ev[e] : 0.f;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < kTile; ++r)
+            gs[c * kGStride + r * kTile + col] = gv[r];
+#pragma unroll
+        for (int r = 0; r < kTile + 2; ++r)
+            xs[c * kXStride + r * kXRow + 1 + col] = xv[r];
+#pragma unroll
+        for (int e = 0; e < 3; ++e)
+        {
+            const int i = col + e * kTile;
+            if (i < 2 * (kTile + 2))
+                xs[c * kXStride + i / 2 * kXRow + (i % 2 ? kTile + 1 : 0)] = ev[e];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+        {
+            const int r = 4 * wave + q;
+            const f32x4 a = *reinterpret_cast<const f32x4 *>(gs + ch * kGStride + r * kTile + kk);
+            bsum += ((a[0] + a[1]) + a[2]) + a[3];
+#pragma unroll
+            for (int ky = 0; ky < 3; ++ky)
             {
-                w0[2] = xr[r * kHalo + c + 2];
-                w1[2] = xr[(r + 1) * kHalo + c + 2];
-                w2[2] = xr[(r + 2) * kHalo + c + 2];
-                const float gv = gr[r * kTile + c];
-                acc[0] = fmaf(gv, w0[0], acc[0]);
-                acc[1] = fmaf(gv, w0[1], acc[1]);
-                acc[2] = fmaf(gv, w0[2], acc[2]);
-                acc[3] = fmaf(gv, w1[0], acc[3]);
-                acc[4] = fmaf(gv, w1[1], acc[4]);
-                acc[5] = fmaf(gv, w1[2], acc[5]);
-                acc[6] = fmaf(gv, w2[0], acc[6]);
-                acc[7] = fmaf(gv, w2[1], acc[7]);
-                acc[8] = fmaf(gv, w2[2], acc[8]);
-                acc[9] += gv;
-                w0[0] = w0[1];
-                w0[1] = w0[2];
-                w1[0] = w1[1];
-                w1[1] = w1[2];
-                w2[0] = w2[1];
-                w2[1] = w2[2];
+                const float *xr = xs + ch * kXStride + (r + ky) * kXRow + kk;
+                const f32x4 lo = *reinterpret_cast<const f32x4 *>(xr);
+                const float v[6] = {lo[0], lo[1], lo[2], lo[3], xr[4], xr[5]};
+#pragma unroll
+                for (int kx = 0; kx < 3; ++kx)
+#pragma unroll
+                    for (int s = 0; s < 4; ++s)
+                        acc[3 * ky + kx] =
+                            __builtin_amdgcn_mfma_f32_16x16x4f32(a[s], v[s + kx], acc[3 * ky + kx], 0, 0, 0);
             }
         }
     }
-    float *out = partial + ((size_t(blockIdx.y) * CoutP + co0 + ol) * CinP + ci0 + cl) * 10;
+    // D[i][j]: output channel 4 (lane / 16) + v, input channel lane % 16
+    __syncthreads();
+    bsum += __shfl_xor(bsum, 16, 64);
+    bsum += __shfl_xor(bsum, 32, 64);  // every lane: its channel's (lane % 16) sum
+    if (wave > 0)
+    {
 #pragma unroll
-    for (int k = 0; k < 10; ++k)
-        out[k] = acc[k];
-}
-
-// Weight-gradient sums over the slices in two stages, each in a fixed order
-// (bitwise reproducible): stage 1 sums group g's slices [g*per, (g+1)*per)
-// of one weight per thread into part2[g][weight] (FP64); stage 2 adds the
-// groups.  Weight index w < Cout*Cin*9 is (o, c, k), then Cout biases (slot 9
-// of channel 0).
-constexpr int kReduceGroups = 32;
-
-__device__ __forceinline__ size_t wgrad_slot(int w, int Cin, int Cout, int CinP)
-{
-    const int nw = Cout * Cin * 9;
-    int o, c, k;
-    if (w < nw)
-    {
-        o = w / (Cin * 9);
-        c = (w / 9) % Cin;
-        k = w % 9;
+        for (int k = 0; k < 9; ++k)
+            *reinterpret_cast<f32x4 *>(lds + (((wave - 1) * 9 + k) * 64 + lane) * 4) = acc[k];
+        lds[3 * 9 * 256 + (wave - 1) * 64 + lane] = bsum;
     }
-    else
+    __syncthreads();
+    if (wave > 0)
+        return;
+    for (int w = 0; w < 3; ++w)
     {
-        o = w - nw;
-        c = 0;
-        k = 9;
+#pragma unroll
+        for (int k = 0; k < 9; ++k)
+            acc[k] += *reinterpret_cast<const f32x4 *>(lds + ((w * 9 + k) * 64 + lane) * 4);
+        bsum += lds[3 * 9 * 256 + w * 64 + lane];
     }
-    return (size_t(o) * CinP + c) * 10 + k;
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+    {
+        float *out = partial + ((size_t(blockIdx.y) * CoutP + co0 + kk + v) * CinP + ci0 + ch) * 10;
+#pragma unroll
+        for (int k = 0; k < 9; ++k)
+            out[k] = acc[k][v];
+    }
+    if (lane < 16)
+        partial[((size_t(blockIdx.y) * CoutP + co0 + ch) * CinP + ci0) * 10 + 9] = bsum;
 }
 
-__global__ void k_wgrad_reduce(const float *__restrict__ partial, double *__restrict__ part2, int Cin, int Cout,
-                               int CinP, int CoutP, int slices, int per)
-{
-    const int w = blockIdx.x * blockDim.x + threadIdx.x;
-    const int nall = Cout * Cin * 9 + Cout;
-    if (w >= nall)
-        return;
-    const size_t slot = wgrad_slot(w, Cin, Cout, CinP);
-    const size_t stride = size_t(CoutP) * CinP * 10;
-    const int s0 = blockIdx.y * per, s1 = min(slices, s0 + per);
-    double s = 0.0;
-    for (int sl = s0; sl < s1; ++sl)
-        s += double(partial[size_t(sl) * stride + slot]);
-    part2[size_t(blockIdx.y) * nall + w] = s;
-}
+// The gradients of every convolution from the slices' partial sums, in one
+// launch and a fixed order (bitwise reproducible, FP64): a block has 32
+// weights of one convolution, eight threads each take every eighth slice, and
+// their sums are added in order.  Weight index w < Cout*Cin*9 is (o, c, k),
+// then Cout biases (slot 9 of channel 0).
+constexpr int kReduceWeights = 32, kReduceGroups = 8;
 
-__global__ void k_wgrad_final(const double *__restrict__ part2, float *__restrict__ gw, float *__restrict__ gb,
-                              int Cin, int Cout, int groups)
+struct ReduceConv
 {
-    const int w = blockIdx.x * blockDim.x + threadIdx.x;
-    const int nw = Cout * Cin * 9, nall = nw + Cout;
-    if (w >= nall)
-        return;
-    double s = 0.0;
-    for (int g = 0; g < groups; ++g)
-        s += part2[size_t(g) * nall + w];
-    if (w < nw)
-        gw[w] = float(s);
-    else
-        gb[w - nw] = float(s);
+    const float *partial;
+    float *grad;  // weights, then biases
+    int Cin, Cout, CinP, CoutP, slices;
+    int first_block;
+};
+struct ReduceAll
+{
+    ReduceConv conv[kConvs];
+};
+
+__global__ __launch_bounds__(kReduceWeights *kReduceGroups) void k_wgrad_reduce(ReduceAll a)
+{
+    int k = 0;
+    while (k + 1 < kConvs && int(blockIdx.x) >= a.conv[k + 1].first_block)
+        ++k;
+    const ReduceConv cv = a.conv[k];
+    const int wl = threadIdx.x % kReduceWeights, group = threadIdx.x / kReduceWeights;
+    const int w = (int(blockIdx.x) - cv.first_block) * kReduceWeights + wl;
+    const int nw = cv.Cout * cv.Cin * 9, nall = nw + cv.Cout;
+    double sum = 0.0;
+    if (w < nall)
+    {
+        const int o = w < nw ? w / (cv.Cin * 9) : w - nw, c = w < nw ? (w / 9) % cv.Cin : 0;
+        const size_t slot = (size_t(o) * cv.CinP + c) * 10 + (w < nw ? w % 9 : 9);
+        const size_t stride = size_t(cv.CoutP) * cv.CinP * 10;
+#pragma unroll 8
+        for (int s = group; s < cv.slices; s += kReduceGroups)
+            sum += double(cv.partial[size_t(s) * stride + slot]);
+    }
+    __shared__ double part[kReduceGroups][kReduceWeights];
+    part[group][wl] = sum;
+    __syncthreads();
+    if (group == 0 && w < nall)
+    {
+        for (int g = 1; g < kReduceGroups; ++g)
+            sum += part[g][wl];
+        cv.grad[w] = float(sum);
+    }
 }
 
 // ---- BF16 inference: implicit-GEMM convolution on the matrix cores --------
@@ -307,77 +381,96 @@ __device__ __forceinline__ short f32_to_bf16_rne(float f)
     return short(u >> 16);
 }
 
+// The k order is kept (a change of summation order moves activations across
+// BF16 rounding bounds, which the layers above amplify), so a lane's four
+// values of a chunk come from four places of the tile: their offsets are
+// looked up in a table in LDS, once per chunk for the R rows of a wave.
+// Dividing per value, with one row per wave, took 242 us for 16
+// -> 16 channels at 256 x 256, 32 samples; this takes 95 us, bound by the
+// 2-byte LDS reads (four per lane and chunk).  A prediction of 64 samples:
+// 3.5 -> 1.65 ms in these kernels.
+template <int CT, int R>
 __global__ __launch_bounds__(256) void k_conv3x3_bf16(const float *__restrict__ x, const short *__restrict__ wb,
                                                       const float *__restrict__ bias, float *__restrict__ y, int Cin,
                                                       int Cout, int Kp, int H, int W, int tiles_x, int relu)
 {
-    constexpr int TR = kMfmaRows + 2, TC = kMfmaCols + 2;
-    extern __shared__ short tile_bf[];  // Cin x TR x TC
-    const int b = blockIdx.y;
-    const int x0 = int(blockIdx.x % unsigned(tiles_x)) * kMfmaCols;
-    const int y0 = int(blockIdx.x / unsigned(tiles_x)) * kMfmaRows;
+    constexpr int TR = 4 * R + 2, TC = kMfmaCols + 2;
+    extern __shared__ __align__(16) short tile_bf[];  // Kp offsets (a zero's for the padding), then the tile, a zero
+    short *offset = tile_bf, *tile = tile_bf + Kp;
+    const int n = Cin * TR * TC;
+    unsigned at, b;
+    xcd_place(at, b);
+    const int x0 = int(at % unsigned(tiles_x)) * kMfmaCols, y0 = int(at / unsigned(tiles_x)) * (4 * R);
     const float *xb = x + size_t(b) * Cin * H * W;
-    for (int i = threadIdx.x; i < Cin * TR * TC; i += 256)
+    for (int k = threadIdx.x; k < Kp; k += 256)
     {
-        const int c = i / (TR * TC), r = (i / TC) % TR, col = i % TC;
-        const int yy = y0 - 1 + r, xx = x0 - 1 + col;
-        float v = 0.f;
-        if (yy >= 0 && yy < H && xx >= 0 && xx < W)
-            v = xb[(size_t(c) * H + yy) * W + xx];
-        tile_bf[i] = f32_to_bf16_rne(v);
+        const int c = k / 9, tap = k - 9 * c;
+        offset[k] = short((c * TR + tap / 3) * TC + tap % 3);  // below 64 * 18 * 18; c < Cin + 2
     }
+    // loads without branches, so that several are in flight
+#pragma unroll 4
+    for (int i = threadIdx.x; i < n; i += 256)
+    {
+        const int c = i / (TR * TC), px = i % (TR * TC);
+        const int yy = y0 - 1 + px / TC, xx = x0 - 1 + px % TC;
+        const bool in = yy >= 0 && yy < H && xx >= 0 && xx < W;
+        const float v = xb[in ? (size_t(c) * H + yy) * W + xx : 0];
+        tile[i] = f32_to_bf16_rne(in ? v : 0.f);
+    }
+    for (int i = n + threadIdx.x; i < n + 2 * TR * TC; i += 256)
+        tile[i] = 0;  // the padding's k reach two channels past the last
     __syncthreads();
     const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
     const int j = lane % 16, kq = 4 * (lane / 16);
-    const int co_tiles = (Cout + 15) / 16;
-    const int K = 9 * Cin;
-    f32x4 acc[kMaxCoTiles];
+    const int t0 = int(blockIdx.z) * CT;
+    f32x4 acc[CT][R];
 #pragma unroll
-    for (int t = 0; t < kMaxCoTiles; ++t)
-        acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int t = 0; t < CT; ++t)
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+            acc[t][r] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const short *xl = tile + wave * R * TC + j;
+    const short *wl = wb + size_t(t0 * 16 + j) * Kp + kq;
     for (int kc = 0; kc < Kp; kc += 16)
     {
-        bf16x4 bv;
+        const bf16x4 from = *reinterpret_cast<const bf16x4 *>(offset + kc + kq);
+        bf16x4 av[CT];
 #pragma unroll
-        for (int it = 0; it < 4; ++it)
-        {
-            const int k = kc + kq + it;
-            short v = 0;
-            if (k < K)
-            {
-                const int c = k / 9, tap = k - 9 * (k / 9);
-                v = tile_bf[(c * TR + wave + tap / 3) * TC + j + tap % 3];
-            }
-            bv[it] = v;
-        }
+        for (int t = 0; t < CT; ++t)
+            av[t] = *reinterpret_cast<const bf16x4 *>(wl + size_t(t) * 16 * Kp + kc);
 #pragma unroll
-        for (int t = 0; t < kMaxCoTiles; ++t)
+        for (int r = 0; r < R; ++r)
         {
-            if (t < co_tiles)
-            {
-                const bf16x4 av = *reinterpret_cast<const bf16x4 *>(wb + size_t(t * 16 + j) * Kp + kc + kq);
-                acc[t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, bv, acc[t], 0, 0, 0);
-            }
+            bf16x4 bv;
+#pragma unroll
+            for (int it = 0; it < 4; ++it)
+                bv[it] = xl[int(from[it]) + r * TC];
+#pragma unroll
+            for (int t = 0; t < CT; ++t)
+                acc[t][r] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av[t], bv, acc[t][r], 0, 0, 0);
         }
     }
-    const int oy = y0 + wave, ox = x0 + j;
-    if (oy >= H || ox >= W)
-        return;
+    const int ox = x0 + j;
 #pragma unroll
-    for (int t = 0; t < kMaxCoTiles; ++t)
+    for (int r = 0; r < R; ++r)
     {
-        if (t >= co_tiles)
-            break;
+        const int oy = y0 + wave * R + r;
+        if (oy >= H || ox >= W)
+            continue;
 #pragma unroll
-        for (int v = 0; v < 4; ++v)
+        for (int t = 0; t < CT; ++t)
         {
-            const int co = t * 16 + kq + v;
-            if (co < Cout)
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
             {
-                float r = acc[t][v] + bias[co];
-                if (relu)
-                    r = r > 0.f ? r : 0.f;
-                y[((size_t(b) * Cout + co) * H + oy) * W + ox] = r;
+                const int co = (t0 + t) * 16 + kq + v;
+                if (co < Cout)
+                {
+                    float o = acc[t][r][v] + bias[co];
+                    if (relu)
+                        o = o > 0.f ? o : 0.f;
+                    y[((size_t(b) * Cout + co) * H + oy) * W + ox] = o;
+                }
             }
         }
     }
@@ -394,19 +487,19 @@ __global__ void k_pack_bf16(const float *__restrict__ w, short *__restrict__ wb,
     wb[size_t(o) * Kp + k] = f32_to_bf16_rne(w[idx]);
 }
 
-// wm[o*Kp + c*9 + k] = w[o][c][k] (Kp = round16(9 Cin));
-// wt[c*KpT + o*9 + 8-k] = w[o][c][k] (KpT = round16(9 Cout)): the data
+// wm[o*Kp + k*CinP + c] = w[o][c][k] (Kp = 9 CinP);
+// wt[c*KpT + (8-k)*CoutP + o] = w[o][c][k] (KpT = 9 CoutP): the data
 // gradient's weights, input and output channels swapped, taps flipped.
 // Padding rows and columns stay zero.
 __global__ void k_pack(const float *__restrict__ w, float *__restrict__ wm, float *__restrict__ wt, int Cin, int Cout,
-                       int Kp, int KpT)
+                       int CinP, int CoutP)
 {
     const int idx = blockIdx.x * blockDim.x + threadIdx.x;
     if (idx >= Cout * Cin * 9)
         return;
     const int o = idx / (Cin * 9), c = (idx / 9) % Cin, k = idx % 9;
-    wm[size_t(o) * Kp + c * 9 + k] = w[idx];
-    wt[size_t(c) * KpT + o * 9 + (8 - k)] = w[idx];
+    wm[(size_t(o) * 9 + k) * CinP + c] = w[idx];
+    wt[(size_t(c) * 9 + 8 - k) * CoutP + o] = w[idx];
 }
 
 __global__ void k_pool2(const float *__restrict__ x, float *__restrict__ y, int BC, int H, int W)
@@ -422,15 +515,18 @@ __global__ void k_pool2(const float *__restrict__ x, float *__restrict__ y, int 
     }
 }
 
-// dx[b,c,y,x] += 0.25 dy[b,c,y/2,x/2]
-__global__ void k_pool2_backward_add(const float *__restrict__ dy, float *__restrict__ dx, int BC, int H, int W)
+// dx[b,c,y,x] = [a > 0] (dx + 0.25 dy[b,c,y/2,x/2]): the last share of the
+// gradient of a, with its ReLU mask
+__global__ void k_pool2_backward_add(const float *__restrict__ dy, const float *__restrict__ a,
+                                     float *__restrict__ dx, int BC, int H, int W)
 {
     const size_t n = size_t(BC) * H * W;
     for (size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += size_t(gridDim.x) * blockDim.x)
     {
         const size_t bc = i / (size_t(H) * W);
         const int r = int(i % (size_t(H) * W)), yi = r / W, xi = r % W;
-        dx[i] += 0.25f * dy[(bc * (H / 2) + yi / 2) * (W / 2) + xi / 2];
+        const float v = dx[i] + 0.25f * dy[(bc * (H / 2) + yi / 2) * (W / 2) + xi / 2];
+        dx[i] = a[i] > 0.f ? v : 0.f;
     }
 }
 
@@ -447,8 +543,9 @@ __global__ void k_upadd(const float *__restrict__ lo, const float *__restrict__ 
     }
 }
 
-// dlo[b,c,i,j] = sum of dz over the 2x2 block (dlo: H/2 x W/2)
-__global__ void k_upsample_backward(const float *__restrict__ dz, float *__restrict__ dlo, int BC, int H, int W)
+// dlo[b,c,i,j] = [a > 0] (sum of dz over the 2x2 block) (dlo, a: H/2 x W/2)
+__global__ void k_upsample_backward(const float *__restrict__ dz, const float *__restrict__ a,
+                                    float *__restrict__ dlo, int BC, int H, int W)
 {
     const int h = H / 2, w = W / 2;
     const size_t n = size_t(BC) * h * w;
@@ -457,19 +554,11 @@ __global__ void k_upsample_backward(const float *__restrict__ dz, float *__restr
         const size_t bc = i / (size_t(h) * w);
         const int r = int(i % (size_t(h) * w)), yi = r / w, xi = r % w;
         const float *p = dz + (bc * H + 2 * yi) * W + 2 * xi;
-        dlo[i] = ((p[0] + p[1]) + p[W]) + p[W + 1];
+        dlo[i] = a[i] > 0.f ? ((p[0] + p[1]) + p[W]) + p[W + 1] : 0.f;
     }
 }
 
-// g *= [a > 0]
-__global__ void k_relu_mask(float *__restrict__ g, const float *__restrict__ a, size_t n)
-{
-    for (size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += size_t(gridDim.x) * blockDim.x)
-        if (!(a[i] > 0.f))
-            g[i] = 0.f;
-}
-
-constexpr int kLossBlocks = 256;
+constexpr int kLossBlocks = 2048;  // at most
 
 // dout = 2 m (out - t) norm; partial[block] = sum m (out - t)^2 (FP64)
 __global__ __launch_bounds__(256) void k_loss(const float *__restrict__ out, const float *__restrict__ tgt,
@@ -498,15 +587,23 @@ __global__ __launch_bounds__(256) void k_loss(const float *__restrict__ out, con
         partial[blockIdx.x] = ((part[0] + part[1]) + part[2]) + part[3];
 }
 
-__global__ void k_loss_final(const double *__restrict__ partial, int blocks, double norm, double *__restrict__ loss,
-                             float *__restrict__ history, int slot)
+// the blocks' sums in a fixed order: a thread's every 256th, then the threads'
+__global__ __launch_bounds__(256) void k_loss_final(const double *__restrict__ partial, int blocks, double norm,
+                                                    double *__restrict__ loss, float *__restrict__ history, int slot)
 {
-    if (threadIdx.x != 0 || blockIdx.x != 0)
-        return;
     double s = 0.0;
-    for (int i = 0; i < blocks; ++i)
+    for (int i = threadIdx.x; i < blocks; i += 256)
         s += partial[i];
-    s *= norm;
+    __shared__ double part[4];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1)
+        s += __shfl_xor(s, off, 64);
+    if ((threadIdx.x & 63) == 0)
+        part[threadIdx.x >> 6] = s;
+    __syncthreads();
+    if (threadIdx.x != 0)
+        return;
+    s = (((part[0] + part[1]) + part[2]) + part[3]) * norm;
     *loss = s;
     if (history)
         history[slot] = float(s);
@@ -564,9 +661,7 @@ struct lbm_surrogate
     uint32_t adam_t = 0;
     float *in = nullptr, *tgt = nullptr, *out = nullptr, *dout = nullptr, *dtmp = nullptr;
     float *a[14] = {}, *p[5] = {}, *z[4] = {}, *da[14] = {};
-    float *partial = nullptr;
-    size_t partial_floats = 0;
-    double *part2 = nullptr;  // kReduceGroups x (weights + biases) of the largest conv
+    float *partial[kConvs] = {};  // the weight gradients' slices
     double *loss_part = nullptr, *loss_dev = nullptr;
     float *history = nullptr;
     size_t history_cap = 0;
@@ -613,12 +708,13 @@ size_t act_floats(const lbm_surrogate *s, int C, int level)
 int tiles_x(const lbm_surrogate *s, int l) { return (s->LW[l] + kTile - 1) / kTile; }
 int tiles(const lbm_surrogate *s, int l) { return tiles_x(s, l) * ((s->LH[l] + kTile - 1) / kTile); }
 
-// Weight-gradient slices: enough blocks to fill the GPU, at most one tile each.
+// Weight-gradient slices: the blocks that fit the GPU at once (four per compute
+// unit by their LDS), at most one tile each.  Half as many took 140 instead of
+// 96 us for 16 x 16 channels at 256 x 256, 16 samples.
 int wgrad_slices(const lbm_surrogate *s, int k, int l, int B)
 {
     const int blocks = (round16(kCout[k]) / kWgT) * (round16(kCin[k]) / kWgT);
-    const int want = std::max(1, 2048 / blocks);
-    return std::min(want, B * tiles(s, l));
+    return std::min(std::max(1, 1024 / blocks), B * tiles(s, l));
 }
 
 int pack_all(lbm_surrogate *s)
@@ -627,7 +723,7 @@ int pack_all(lbm_surrogate *s)
     {
         const int n = kCout[k] * kCin[k] * 9;
         hipLaunchKernelGGL(k_pack, dim3((n + 255) / 256), dim3(256), 0, s->stream, s->params + s->w_off[k], s->wp[k],
-                           s->wt[k], kCin[k], kCout[k], round16(9 * kCin[k]), round16(9 * kCout[k]));
+                           s->wt[k], kCin[k], kCout[k], round16(kCin[k]), round16(kCout[k]));
         hipLaunchKernelGGL(k_pack_bf16, dim3((n + 255) / 256), dim3(256), 0, s->stream, s->params + s->w_off[k],
                            s->wb[k], kCin[k], kCout[k], round16(9 * kCin[k]));
     }
@@ -636,23 +732,66 @@ int pack_all(lbm_surrogate *s)
     return LBM_OK;
 }
 
-// FP32 convolution of x (Cin channels) with packed weights wm ([Cout16][round16(9 Cin)]) into y.
-void conv_f32(lbm_surrogate *s, const float *x, const float *wm, const float *bias, float *y, int Cin, int Cout, int l,
-              int B, bool relu)
+// Calls f(CT, R) with the output-channel tiles per block and the rows per wave
+// of a convolution.  Rows of a wave share the weights and most of the halo,
+// channel tiles share the staged input: four rows and all channel tiles where
+// that leaves two blocks per compute unit (512), two rows, then one row below
+// that (two at most for more than 32 input channels, whose tile would leave one
+// block per compute unit in LDS); the channel tiles of a layer too small for
+// 512 blocks of one row get blocks of their own.  16 -> 16 channels at 256 x
+// 256, 16 samples in FP32: 136 us with one row, 79 us with four.
+template <class F>
+void conv_shape(int Cin, int Cout, int H, int W, int B, F f)
 {
-    const int tx = (s->LW[l] + kMfmaCols - 1) / kMfmaCols, ty = (s->LH[l] + kMfmaRows - 1) / kMfmaRows;
-    const size_t lds = size_t(Cin) * (kMfmaRows + 2) * (kMfmaCols + 2) * sizeof(float);
-    hipLaunchKernelGGL(k_conv3x3_f32, dim3(unsigned(tx * ty), unsigned(B)), dim3(256), lds, s->stream, x, wm, bias, y,
-                       Cin, Cout, round16(9 * Cin), s->LH[l], s->LW[l], tx, relu ? 1 : 0);
+    using std::integral_constant;
+    const int co_tiles = (Cout + 15) / 16, cols = (W + kMfmaCols - 1) / kMfmaCols;
+    auto blocks = [&](int rows) { return size_t(cols) * ((H + 4 * rows - 1) / (4 * rows)) * B; };
+    auto by_rows = [&](auto ct) {
+        if (Cin <= 32 && blocks(4) * (co_tiles / ct.value) >= 512)
+            f(ct, integral_constant<int, 4>{});
+        else if (blocks(2) * (co_tiles / ct.value) >= 512)
+            f(ct, integral_constant<int, 2>{});
+        else
+            f(ct, integral_constant<int, 1>{});
+    };
+    if (co_tiles > 1 && blocks(1) < 512)
+        by_rows(integral_constant<int, 1>{});
+    else if (co_tiles == 1)
+        by_rows(integral_constant<int, 1>{});
+    else if (co_tiles == 2)
+        by_rows(integral_constant<int, 2>{});
+    else if (co_tiles == 3)
+        by_rows(integral_constant<int, 3>{});
+    else
+        by_rows(integral_constant<int, 4>{});
+}
+
+// FP32 convolution of x (Cin channels) with packed weights wm ([Cout16][9][Cin16]) into y.
+void conv_f32(lbm_surrogate *s, const float *x, const float *wm, const float *bias, const float *mask, float *y, int Cin,
+              int Cout, int l, int B, bool relu)
+{
+    const int H = s->LH[l], W = s->LW[l], tx = (W + kMfmaCols - 1) / kMfmaCols;
+    conv_shape(Cin, Cout, H, W, B, [&](auto ct, auto rows) {
+        constexpr int CT = decltype(ct)::value, R = decltype(rows)::value;
+        const int ty = (H + 4 * R - 1) / (4 * R);
+        const size_t lds = size_t(4 * R + 2) * (kMfmaCols + 2) * (round16(Cin) + 4) * sizeof(float);
+        hipLaunchKernelGGL((k_conv3x3_f32<CT, R>), dim3(unsigned(tx * ty), unsigned(B), unsigned((Cout + 15) / 16 / CT)),
+                           dim3(256), lds, s->stream, x, wm, bias, mask, y, Cin, Cout, H, W, tx, relu ? 1 : 0);
+    });
 }
 
 void conv_forward_bf16(lbm_surrogate *s, const float *x, int k, float *y, int l, int B, bool relu)
 {
-    const int tx = (s->LW[l] + kMfmaCols - 1) / kMfmaCols, ty = (s->LH[l] + kMfmaRows - 1) / kMfmaRows;
-    const size_t lds = size_t(kCin[k]) * (kMfmaRows + 2) * (kMfmaCols + 2) * sizeof(short);
-    hipLaunchKernelGGL(k_conv3x3_bf16, dim3(unsigned(tx * ty), unsigned(B)), dim3(256), lds, s->stream, x, s->wb[k],
-                       s->params + s->b_off[k], y, kCin[k], kCout[k], round16(9 * kCin[k]), s->LH[l], s->LW[l], tx,
-                       relu ? 1 : 0);
+    const int H = s->LH[l], W = s->LW[l], tx = (W + kMfmaCols - 1) / kMfmaCols, Kp = round16(9 * kCin[k]);
+    conv_shape(kCin[k], kCout[k], H, W, B, [&](auto ct, auto rows) {
+        constexpr int CT = decltype(ct)::value, R = decltype(rows)::value;
+        const int ty = (H + 4 * R - 1) / (4 * R);
+        const size_t lds = (size_t(kCin[k] + 2) * (4 * R + 2) * (kMfmaCols + 2) + Kp) * sizeof(short);
+        hipLaunchKernelGGL((k_conv3x3_bf16<CT, R>),
+                           dim3(unsigned(tx * ty), unsigned(B), unsigned((kCout[k] + 15) / 16 / CT)), dim3(256), lds,
+                           s->stream, x, s->wb[k], s->params + s->b_off[k], y, kCin[k], kCout[k], Kp, H, W, tx,
+                           relu ? 1 : 0);
+    });
 }
 
 void conv_forward(lbm_surrogate *s, const float *x, int k, float *y, int l, int B, bool relu, bool bf16 = false)
@@ -662,13 +801,14 @@ void conv_forward(lbm_surrogate *s, const float *x, int k, float *y, int l, int 
         conv_forward_bf16(s, x, k, y, l, B, relu);
         return;
     }
-    conv_f32(s, x, s->wp[k], s->params + s->b_off[k], y, kCin[k], kCout[k], l, B, relu);
+    conv_f32(s, x, s->wp[k], s->params + s->b_off[k], nullptr, y, kCin[k], kCout[k], l, B, relu);
 }
 
-// dx = data gradient of conv k for output gradient g (dx written, not accumulated)
-void conv_dgrad(lbm_surrogate *s, const float *g, int k, float *dx, int l, int B)
+// dx = data gradient of conv k for output gradient g (dx written, not
+// accumulated), with the ReLU mask of activation a (null: none)
+void conv_dgrad(lbm_surrogate *s, const float *g, int k, const float *a, float *dx, int l, int B)
 {
-    conv_f32(s, g, s->wt[k], nullptr, dx, kCout[k], kCin[k], l, B, false);
+    conv_f32(s, g, s->wt[k], nullptr, a, dx, kCout[k], kCin[k], l, B, false);
 }
 
 void conv_wgrad(lbm_surrogate *s, const float *x, const float *g, int k, int l, int B)
@@ -676,14 +816,24 @@ void conv_wgrad(lbm_surrogate *s, const float *x, const float *g, int k, int l, 
     const int CinP = round16(kCin[k]), CoutP = round16(kCout[k]);
     const int slices = wgrad_slices(s, k, l, B);
     const dim3 grid(unsigned((CoutP / kWgT) * (CinP / kWgT)), unsigned(slices));
-    hipLaunchKernelGGL(k_conv_wgrad, grid, dim3(256), 0, s->stream, x, g, s->partial, B, kCin[k], kCout[k], CinP,
+    hipLaunchKernelGGL(k_conv_wgrad, grid, dim3(256), 0, s->stream, x, g, s->partial[k], B, kCin[k], kCout[k], CinP,
                        CoutP, s->LH[l], s->LW[l], tiles_x(s, l), tiles(s, l), slices);
-    const int n = kCout[k] * kCin[k] * 9 + kCout[k];
-    const int groups = std::min(kReduceGroups, slices), per = (slices + groups - 1) / groups;
-    hipLaunchKernelGGL(k_wgrad_reduce, dim3((n + 255) / 256, groups), dim3(256), 0, s->stream, s->partial,
-                       s->part2, kCin[k], kCout[k], CinP, CoutP, slices, per);
-    hipLaunchKernelGGL(k_wgrad_final, dim3((n + 255) / 256), dim3(256), 0, s->stream, s->part2,
-                       s->grad + s->w_off[k], s->grad + s->b_off[k], kCin[k], kCout[k], groups);
+}
+
+// every convolution's gradient from its slices
+void wgrad_reduce(lbm_surrogate *s, int B)
+{
+    ReduceAll a{};
+    int blocks = 0;
+    for (int k = 0; k < kConvs; ++k)
+    {
+        a.conv[k] = ReduceConv{s->partial[k],        s->grad + s->w_off[k],
+                               kCin[k],              kCout[k],
+                               round16(kCin[k]),     round16(kCout[k]),
+                               wgrad_slices(s, k, conv_level(k), B), blocks};
+        blocks += (kCout[k] * kCin[k] * 9 + kCout[k] + kReduceWeights - 1) / kReduceWeights;
+    }
+    hipLaunchKernelGGL(k_wgrad_reduce, dim3(unsigned(blocks)), dim3(kReduceWeights * kReduceGroups), 0, s->stream, a);
 }
 
 void pool(lbm_surrogate *s, const float *x, float *y, int C, int l_in, int B)
@@ -692,10 +842,10 @@ void pool(lbm_surrogate *s, const float *x, float *y, int C, int l_in, int B)
     hipLaunchKernelGGL(k_pool2, dim3(elem_grid(n)), dim3(256), 0, s->stream, x, y, B * C, s->LH[l_in], s->LW[l_in]);
 }
 
-void pool_backward_add(lbm_surrogate *s, const float *dy, float *dx, int C, int l_in, int B)
+void pool_backward_add(lbm_surrogate *s, const float *dy, const float *a, float *dx, int C, int l_in, int B)
 {
     const size_t n = size_t(B) * C * s->LH[l_in] * s->LW[l_in];
-    hipLaunchKernelGGL(k_pool2_backward_add, dim3(elem_grid(n)), dim3(256), 0, s->stream, dy, dx, B * C,
+    hipLaunchKernelGGL(k_pool2_backward_add, dim3(elem_grid(n)), dim3(256), 0, s->stream, dy, a, dx, B * C,
                        s->LH[l_in], s->LW[l_in]);
 }
 
@@ -705,17 +855,11 @@ void upadd(lbm_surrogate *s, const float *lo, const float *skip, float *z, int C
     hipLaunchKernelGGL(k_upadd, dim3(elem_grid(n)), dim3(256), 0, s->stream, lo, skip, z, B * C, s->LH[l], s->LW[l]);
 }
 
-void upsample_backward(lbm_surrogate *s, const float *dz, float *dlo, int C, int l, int B)
+void upsample_backward(lbm_surrogate *s, const float *dz, const float *a, float *dlo, int C, int l, int B)
 {
     const size_t n = size_t(B) * C * s->LH[l + 1] * s->LW[l + 1];
-    hipLaunchKernelGGL(k_upsample_backward, dim3(elem_grid(n)), dim3(256), 0, s->stream, dz, dlo, B * C, s->LH[l],
+    hipLaunchKernelGGL(k_upsample_backward, dim3(elem_grid(n)), dim3(256), 0, s->stream, dz, a, dlo, B * C, s->LH[l],
                        s->LW[l]);
-}
-
-void relu_mask(lbm_surrogate *s, float *g, const float *a, int C, int l, int B)
-{
-    const size_t n = size_t(B) * C * s->LH[l] * s->LW[l];
-    hipLaunchKernelGGL(k_relu_mask, dim3(elem_grid(n)), dim3(256), 0, s->stream, g, a, n);
 }
 
 // Forward over s->in (B samples) into s->a, s->p, s->z, s->out; bf16: the
@@ -745,40 +889,41 @@ void forward(lbm_surrogate *s, int B, bool bf16 = false)
 void loss_backward(lbm_surrogate *s, int B, double norm, float *history, int slot)
 {
     const int HW = s->H * s->W;
-    hipLaunchKernelGGL(k_loss, dim3(kLossBlocks), dim3(256), 0, s->stream, s->out, s->tgt, s->in, s->dout,
-                       s->loss_part, B, HW, float(norm));
-    hipLaunchKernelGGL(k_loss_final, dim3(1), dim3(64), 0, s->stream, s->loss_part, kLossBlocks, norm, s->loss_dev,
+    const unsigned blocks =
+        std::min<unsigned>(kLossBlocks, elem_grid(size_t(B) * LBM_SURROGATE_OUTPUTS * size_t(HW)));
+    hipLaunchKernelGGL(k_loss, dim3(blocks), dim3(256), 0, s->stream, s->out, s->tgt, s->in, s->dout, s->loss_part, B,
+                       HW, float(norm));
+    hipLaunchKernelGGL(k_loss_final, dim3(1), dim3(256), 0, s->stream, s->loss_part, int(blocks), norm, s->loss_dev,
                        history, slot);
+    // Every da[] is complete, ReLU mask included, once its last share is in.
     // conv13 (no ReLU)
     conv_wgrad(s, s->a[13], s->dout, 13, 0, B);
-    conv_dgrad(s, s->dout, 13, s->da[13], 0, B);
+    conv_dgrad(s, s->dout, 13, s->a[13], s->da[13], 0, B);
     for (int m = 3; m >= 0; --m)
     {
         const int l = 3 - m, kk = 9 + m;
-        relu_mask(s, s->da[10 + m], s->a[10 + m], kCout[kk], l, B);
         conv_wgrad(s, s->z[l], s->da[10 + m], kk, l, B);
-        // dz is the skip's gradient: written straight into da[8-2m]
-        conv_dgrad(s, s->da[10 + m], kk, s->da[8 - 2 * m], l, B);
-        upsample_backward(s, s->da[8 - 2 * m], s->da[9 + m], kCin[kk], l, B);
+        // dz is the skip's gradient: written straight into da[8-2m], which
+        // the pool's share completes
+        conv_dgrad(s, s->da[10 + m], kk, nullptr, s->da[8 - 2 * m], l, B);
+        upsample_backward(s, s->da[8 - 2 * m], s->a[9 + m], s->da[9 + m], kCin[kk], l, B);
     }
-    relu_mask(s, s->da[9], s->a[9], kCout[8], 4, B);
     conv_wgrad(s, s->p[4], s->da[9], 8, 4, B);
-    conv_dgrad(s, s->da[9], 8, s->dtmp, 4, B);
-    pool_backward_add(s, s->dtmp, s->da[8], kCin[8], 3, B);
+    conv_dgrad(s, s->da[9], 8, nullptr, s->dtmp, 4, B);
+    pool_backward_add(s, s->dtmp, s->a[8], s->da[8], kCin[8], 3, B);
     for (int l = 3; l >= 0; --l)
     {
         const int k1 = 2 * l + 1, k0 = 2 * l;
-        relu_mask(s, s->da[k1 + 1], s->a[k1 + 1], kCout[k1], l, B);
         conv_wgrad(s, s->a[k1], s->da[k1 + 1], k1, l, B);
-        conv_dgrad(s, s->da[k1 + 1], k1, s->da[k1], l, B);
-        relu_mask(s, s->da[k1], s->a[k1], kCout[k0], l, B);
+        conv_dgrad(s, s->da[k1 + 1], k1, s->a[k1], s->da[k1], l, B);
         conv_wgrad(s, l == 0 ? s->in : s->p[l], s->da[k1], k0, l, B);
         if (l > 0)
         {
-            conv_dgrad(s, s->da[k1], k0, s->dtmp, l, B);
-            pool_backward_add(s, s->dtmp, s->da[k0], kCin[k0], l - 1, B);
+            conv_dgrad(s, s->da[k1], k0, nullptr, s->dtmp, l, B);
+            pool_backward_add(s, s->dtmp, s->a[k0], s->da[k0], kCin[k0], l - 1, B);
         }
     }
+    wgrad_reduce(s, B);
 }
 
 int adam_step(lbm_surrogate *s, float lr)
@@ -903,7 +1048,6 @@ int lbm_surrogate_create(uint32_t height, uint32_t width, uint32_t max_batch, lb
     C_TRY(alloc(s, &s->grad, s->nparams));
     C_TRY(alloc(s, &s->adam_m, s->nparams));
     C_TRY(alloc(s, &s->adam_v, s->nparams));
-    size_t partial = 0;
     for (int k = 0; k < kConvs; ++k)
     {
         const size_t cin_p = size_t(round16(kCin[k])), cout_p = size_t(round16(kCout[k]));
@@ -919,17 +1063,7 @@ int lbm_surrogate_create(uint32_t height, uint32_t width, uint32_t max_batch, lb
             S_TRY(hipMemsetAsync(s->wb[k], 0, cout_p * kp * sizeof(short), s->stream));
             return LBM_OK;
         }());
-        partial = std::max(partial, size_t(wgrad_slices(s, k, conv_level(k), s->Bmax)) * cout_p * cin_p * 10);
-    }
-    s->partial_floats = partial;
-    C_TRY(alloc(s, &s->partial, partial));
-    {
-        size_t most = 0;
-        for (int k = 0; k < kConvs; ++k)
-            most = std::max(most, size_t(kCout[k]) * kCin[k] * 9 + kCout[k]);
-        float *p2 = nullptr;
-        C_TRY(alloc(s, &p2, 2 * kReduceGroups * most));  // doubles
-        s->part2 = reinterpret_cast<double *>(p2);
+        C_TRY(alloc(s, &s->partial[k], size_t(wgrad_slices(s, k, conv_level(k), s->Bmax)) * cout_p * cin_p * 10));
     }
     C_TRY(alloc(s, &s->in, act_floats(s, LBM_SURROGATE_INPUTS, 0)));
     C_TRY(alloc(s, &s->tgt, act_floats(s, LBM_SURROGATE_OUTPUTS, 0)));
