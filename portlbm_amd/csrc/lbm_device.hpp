@@ -129,13 +129,14 @@ __device__ __forceinline__ uint32_t mix32(uint32_t x)
 // the 13 random bits r (< 2^13) and cut, so |v| rounds up with probability
 // equal to the dropped fraction.  Exact for the binary16 normal range; below
 // it the conversion's own rounding applies to the remainder.  Inf/NaN pass
-// through.
+// through: the 13 bits are zero in an infinity, in the NaN that arithmetic
+// makes, and in one that came from a binary16, so that r cannot carry out of
+// them.  (A test of the exponent per value, instead, made 2000 steps of an
+// 8192 x 2048 cylinder channel 270 ms against 245; the random numbers from
+// 16-bit halves, by v_dot2 or v_mad_u16 for v_mul_lo_u32, 280 and 297.)
 __device__ __forceinline__ _Float16 f32_to_f16_sr(float v, uint32_t r)
 {
-    uint32_t u = __float_as_uint(v);
-    if ((u & 0x7f800000u) != 0x7f800000u)
-        u = (u + r) & ~0x1fffu;
-    return _Float16(__uint_as_float(u));
+    return _Float16(__uint_as_float((__float_as_uint(v) + r) & ~0x1fffu));
 }
 
 // The shift of direction d at a node whose rho_ref is rt (float).
@@ -192,13 +193,10 @@ __device__ __forceinline__ uint16_t f32_to_bf16(float f)
 __device__ __forceinline__ float bf16_to_f32(uint16_t h) { return __uint_as_float(uint32_t(h) << 16); }
 
 // binary32 -> bfloat16, stochastic (16 dropped bits against the 16 random
-// bits r < 2^16).
+// bits r < 2^16; Inf/NaN pass through as above).
 __device__ __forceinline__ uint16_t f32_to_bf16_sr(float f, uint32_t r)
 {
-    const uint32_t u = __float_as_uint(f);
-    if ((u & 0x7f800000u) == 0x7f800000u)
-        return f32_to_bf16(f);
-    return uint16_t((u + r) >> 16);
+    return uint16_t((__float_as_uint(f) + r) >> 16);
 }
 
 // BF16 deviation storage: HBM holds f_d - w_d rho_ref(x) as bfloat16 (RNE,

@@ -25,6 +25,7 @@
 //   FP64     383 -> 139      362 -> 157      366 -> 151
 //   FP32     204 -> 104      235 -> 115      242 -> 116
 //   FP16     128 -> 106      177 -> 113      184 -> 113
+// (FP16 with stochastic rounding, cylinder channel: 160 -> 122.)
 // What bounds it at T = 4: vector instructions, 62 % of the cycles in FP64
 // (rocprofv3: 2.06e8 per launch of 557 us) with two waves per SIMD, next to
 // 2.55 GB moved per launch (4.6 TB/s).
@@ -401,7 +402,7 @@ __device__ __forceinline__ void march_wave(const StepParams &p, const uint32_t (
             C rho, jx, jy, usq;
             collide_node<C, Storage<S>::kPromote, Storage<S>::kFull>(f[i], C(p.omega), rho, jx, jy, usq);
             if constexpr (k < T)
-                uy[k][i] = clamp_output(jy, p.nan_protection);
+                uy[k][i] = N == 4 ? clamp_output(jy, p.nan_protection) : jy;
             else if ((p.write_macros || bit(i, LBM_CODE_UY_SOURCE)) && owned && bit(i, LBM_CODE_FLUID))
             {
                 const uint32_t c = (cd[i / 2] >> (16 * (i & 1))) & 0xffffu;
@@ -413,6 +414,14 @@ __device__ __forceinline__ void march_wave(const StepParams &p, const uint32_t (
             }
             node_bits<S>(f[i], uint32_t(r) * p.P + lp + uint32_t(i), sr[k - 1], t[i], 0.f);
         }
+        // The next stage reads them only beside an outlet.  (With four nodes a
+        // lane the clamp of all four at once costs registers: 252 against 245
+        // ms over 2000 steps; with fewer it saves 1 %.)
+        if constexpr (k < T && N < 4)
+            if (rf & ROW_OUTLET)
+#pragma unroll
+                for (int i = 0; i < N; ++i)
+                    uy[k][i] = clamp_output(uy[k][i], p.nan_protection);
         u32x2 out[9];
 #pragma unroll
         for (int d = 0; d < 9; ++d)

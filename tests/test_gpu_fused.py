@@ -126,6 +126,25 @@ def test_diverging_flow_keeps_its_infinities(storage, size):
         assert same(one.macros(), many.macros())
 
 
+@pytest.mark.parametrize("size", [(3001, 1171), (300, 100)])
+@pytest.mark.parametrize("storage", ["f16-shifted", "bf16-shifted"])
+def test_stochastic_rounding_keeps_infinities(storage, size):
+    """The random bits carry into neither an infinity nor a NaN: they stand
+    where rounding to nearest leaves them."""
+    fields = []
+    for rounding in ("nearest", "stochastic"):
+        doc = document("nptl", "stream", storage, rounding, *size, "walls")
+        with pa.Lattice(pa.desc_from_settings(doc), pa.build_phase(doc)) as lattice:
+            f = lattice.populations()
+            f[::7919], f[1::15838], f[2::31676] = np.inf, -np.inf, np.nan
+            lattice.set_populations(f)
+            lattice.run(3)
+            fields.append(lattice.populations())
+    assert not np.all(np.isfinite(fields[0]))
+    for kind in (np.isnan, np.isposinf, np.isneginf):
+        np.testing.assert_array_equal(kind(fields[0]), kind(fields[1]))
+
+
 @pytest.mark.parametrize("storage", ["f64", "f32", "f16-shifted", "bf16-shifted"])
 @pytest.mark.parametrize("count", [1, 3, 40, 130])
 def test_batched_domains(count, storage):
