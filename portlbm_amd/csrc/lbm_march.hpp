@@ -43,15 +43,25 @@ struct FusePlan
 //   1024 x 256   10.2 / 6.1 / 6.3    32x32 T 5: 4.69 / 3.73 / 3.65    32x16 T 4: 4.38 / 3.82 / 3.90
 //   2048 x 512   29.5 / 16.1 / 16.3  32x16 T 4: 12.6 / 10.7 / 11.1    march:     14.6 / 13.0 / 20.3
 //   4096 x 1024  112 / 55.8 / 48.9   32x16 T 4: 59.0 / 42.9 / 38.7    march:     45.4 / 32.7 / 37.5
+// and at the lines between the shapes (bundle layout, FP64 / FP32 / BF16;
+// "1.8e5": inner nodes):
+//   1.8e5  32x32 T 6: 3.77 / 3.18 / 3.27   T 5: 4.06 / 3.38 / 3.42
+//   2.6e5  32x32 T 6: 5.06 / 4.20 / 4.16   T 5: 4.52 / 3.59 / 3.74
+//   3.9e5  32x32 T 5: 6.39 / 4.96 / 5.00   32x16 T 4: 5.81 / 4.98 / 5.12 (FP64 collision 7.12, 6.90)
+//   1.0e6  32x16 T 3: 11.7 / 10.1 / 10.4   32x16 T 4: 12.2 / 10.7 / 11.1   march: 14.8 / 13.9 / 18.0
+//   2.0e6  32x16 T 3: 23.2 / 18.5 / 19.1   32x16 T 4: 22.9 / 19.8 / 20.5   march: 24.8 / 19.8 / 24.1
+//   3.0e6  32x16 T 3: 39.0 / 27.2 / 28.0   march: 35.1 / 27.2 / 27.5
+// FP64 marches from 1.5e6: at 2.0e6 the collision layout takes 24.7 marched
+// and 27.3 in tiles.
 inline FusePlan plan_fusion(size_t elem, uint64_t nodes)
 {
-    if (nodes >= (elem == 8 ? 1500000u : (elem == 4 ? 2000000u : 3500000u)))
+    if (nodes >= (elem == 8 ? 1500000u : (elem == 4 ? 3000000u : 3500000u)))
         return FusePlan{kMarchMaxSteps, false, TileShape::k32x32};
     if (nodes <= 36000u)
         return FusePlan{5u, true, TileShape::k16x16};
-    if (nodes <= 500000u)
-        return FusePlan{nodes <= 130000u ? 6u : 5u, true, TileShape::k32x32};
-    return FusePlan{4u, true, TileShape::k32x16};
+    if (nodes <= (elem == 8 ? 300000u : 500000u))
+        return FusePlan{nodes <= 200000u ? 6u : 5u, true, TileShape::k32x32};
+    return FusePlan{elem == 8 ? 4u : 3u, true, TileShape::k32x16};
 }
 
 // The first launch of n steps: as few launches as there can be, of nearly the same length.

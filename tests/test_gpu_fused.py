@@ -42,10 +42,10 @@ def check(doc, steps, frame_interval=0):
 
 # Inner extents.  Marching waves own strips of 56, 112 or 224 columns (FP64,
 # FP32, 16-bit): whole strips, ragged ones, one strip and a half.
-MARCHED = {"f64": [(2240, 700), (3001, 503), (85, 17700)], "f32": [(2240, 901), (1999, 1013)],
+MARCHED = {"f64": [(2240, 700), (3001, 503), (85, 17700)], "f32": [(2240, 901), (1999, 1013), (2241, 1360)],
            "f16-shifted": [(3001, 1171)], "bf16-shifted": [(2688, 1310)]}
 # Small lattices: less than a region, each shape's whole and ragged numbers of them.
-TILED = [(4, 9), (30, 12), (61, 37), (256, 64), (257, 131), (500, 250), (1031, 301), (1030, 800)]
+TILED = [(4, 9), (30, 12), (61, 37), (256, 64), (257, 131), (500, 250), (1031, 301), (1030, 800), (700, 260)]
 
 
 @pytest.mark.parametrize("storage,rounding", STORAGES)
