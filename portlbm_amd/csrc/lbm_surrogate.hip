@@ -4,11 +4,11 @@
 // loss sums.  The network has no counterpart in the reference.
 //
 // Kernels (NCHW float32, 256-thread blocks):
-//   k_conv3x3_f32  implicit GEMM on the matrix cores in FP32
-//                  (v_mfma_f32_16x16x4f32); the input tile with its 1-node
-//                  halo staged in LDS with the channels of a pixel together;
-//                  weights packed [Cout16][tap][Cin16].  The data gradient is
-//                  the same kernel on flipped, transposed weights.
+//   k_conv3x3      implicit GEMM on the matrix cores, in FP32 or, for BF16
+//                  inference, with BF16 operands; the input tile with its
+//                  1-node halo staged in LDS; weights packed [Cout16][K16],
+//                  K = 9 Cin in the weights' own (c, tap) order.  The data
+//                  gradient is the same kernel on flipped, transposed weights.
 //   k_conv_wgrad   the weight gradient on the same instruction, pixels as the
 //                  inner dimension: a block has a 16 x 16 (out, in) channel
 //                  pair and a slice of the pixel tiles; the slices' partial
@@ -46,28 +46,45 @@ inline int round16(int c) { return (c + 15) / 16 * 16; }
 // Resolution level (0 = full, 4 = 1/16) at which conv k runs.
 inline int conv_level(int k) { return k < 8 ? k / 2 : k == 8 ? 4 : k == 13 ? 0 : 12 - k; }
 
-// ---- FP32 convolution on the matrix cores ---------------------------------
-// y[b][o][p] = act(bias[o] + sum over tap, c of Wm[o][tap][c] X[c][p + tap]),
-// with v_mfma_f32_16x16x4f32 (A 16x4, B 4x16, FP32 products and accumulation).
-// Lane layout (the same as the BF16 instruction's, one element per lane):
-// A[i][kk] in lane i + 16 kk, B[kk][j] in lane j + 16 kk, D[i][j] in lane
-// j + 16 (i/4), element i%4.  Which k an operand slot kk carries is free as
-// long as A and B agree: within a tap's 16 channels from c0 on, MFMA s gives
-// slot kk the channel c0 + 4 kk + s, so that a lane reads its four values of
-// either operand as one 16-byte load (LDS holds a pixel's channels together,
-// 4 floats of padding per pixel keep the 16 pixels of a read on different
-// banks).  A wave computes R rows of 16 pixels for CT tiles of 16 output
-// channels: R rows share each weight load, CT tiles each pixel load.
+// ---- convolution on the matrix cores --------------------------------------
+// y[b][o][p] = act(bias[o] + sum_k Wm[o][k] X[k][p]), k = c*9 + tap (the
+// weights' own order), as an implicit GEMM in chunks of 16 k: in FP32 (E =
+// float) four v_mfma_f32_16x16x4f32 per chunk, for BF16 inference (E = short)
+// one v_mfma_f32_16x16x16bf16_1k, both with FP32 accumulation.
+// Lane layouts, checked on the device.  BF16: A[i][k] in lane i + 16 (k/4),
+// element k%4; B[k][j] in lane j + 16 (k/4), element k%4; D[i][j] in lane
+// j + 16 (i/4), element i%4.  FP32: A[i][kk] in lane i + 16 kk, B[kk][j] in
+// lane j + 16 kk, D as above; MFMA s of a chunk at kc gives slot kk the
+// k = kc + 4 kk + s.  Either way a lane holds k = kc + 4 (lane/16) + 0..3 of
+// both operands: its four weights are one load.
+// A wave computes R rows of 16 pixels for CT tiles of 16 output channels: the
+// rows share the weights, the tiles the pixels; four waves have 4 R rows, whose
+// input with its 1-node halo is staged in LDS.
 //
-// A channel-major weight order and a channel plane per LDS row would need a
-// division per operand value and single-float LDS reads, and one row per wave
-// a weight load per pixel row: the 27 launches of a training batch of 16
-// samples of 256 x 256 took 2.34 ms that way and take 1.3 ms this way.  16 ->
-// 16 channels at 256 x 256, 16 samples: 136 -> 79 us, 61 TFLOP/s of 152
-// reachable, bound by the staging of the tile (134 MB moved would take 27 us).
+// The order of the sums is that of k.  Another order moves activations across
+// BF16 rounding bounds and across the zero of a ReLU, where the gradient jumps
+// (taps before channels, with 16-byte LDS reads: no faster in FP32, and a
+// gradient up to six times as far from FP64).  A lane's four pixels of a chunk
+// so come from four places of the tile: their offsets are looked up in a table
+// in LDS, once per chunk for the R rows.  Dividing per value instead, with one
+// row per wave: 16 -> 16 channels at 256 x 256, BF16, 32 samples 242 us, here
+// 97 us, bound by the 2-byte LDS reads; FP32, 16 samples 136 us, here 74 us (65
+// TFLOP/s of 152 reachable; the 134 MB moved would take 27 us).  All
+// convolutions of a BF16 prediction of 64 samples: 3.5 -> 1.7 ms, the 27 of a
+// training batch of 16: 2.34 -> 1.4 ms.
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef short s16x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kMfmaCols = 16;
+
+__device__ __forceinline__ short f32_to_bf16_rne(float f)
+{
+    uint32_t u = __float_as_uint(f);
+    if ((u & 0x7fffffffu) > 0x7f800000u)
+        return short((u >> 16) | 0x40u);
+    u += 0x7fffu + ((u >> 16) & 1u);
+    return short(u >> 16);
+}
 
 // A block's place (tile, sample) in a grid of (tiles, samples): the blocks that
 // one XCD gets (every eighth in launch order) are neighbours, so that the
@@ -82,35 +99,49 @@ __device__ __forceinline__ void xcd_place(unsigned &tile, unsigned &sample)
 
 // relu: outputs below 0 become 0; mask (or null): outputs become 0 where it is
 // not above 0 (the ReLU derivative of the layer below, for a data gradient).
-template <int CT, int R>
-__global__ __launch_bounds__(256) void k_conv3x3_f32(const float *__restrict__ x, const float *__restrict__ wm,
-                                                     const float *__restrict__ bias, const float *__restrict__ mask,
-                                                     float *__restrict__ y, int Cin, int Cout, int H, int W,
-                                                     int tiles_x, int relu)
+// lo (or null): the input is x + up2(lo), lo of half the extents; a sum in
+// memory of its own would be written and read once more (35 us for 16 channels
+// at 256 x 256, 32 samples).
+template <class E, int CT, int R>
+__global__ __launch_bounds__(256) void k_conv3x3(const float *__restrict__ x, const float *__restrict__ lo,
+                                                 const E *__restrict__ wm, const float *__restrict__ bias,
+                                                 const float *__restrict__ mask, float *__restrict__ y, int Cin,
+                                                 int Cout, int Kp, int H, int W, int tiles_x, int relu)
 {
+    typedef E E4 __attribute__((ext_vector_type(4)));
+    constexpr bool kBf16 = sizeof(E) == 2;
     constexpr int TR = 4 * R + 2, TC = kMfmaCols + 2;
-    extern __shared__ __align__(16) float tile_f[];  // TR x TC pixels x (Cin16 + 4)
-    const int CinP = (Cin + 15) / 16 * 16, stride = CinP + 4, Kp = 9 * CinP;
+    extern __shared__ __align__(16) short conv_lds[];  // Kp offsets, then the tile and two channels of zeros
+    short *offset = conv_lds;
+    E *tile = reinterpret_cast<E *>(conv_lds + Kp);
+    const int n = Cin * TR * TC;
     unsigned at, b;
     xcd_place(at, b);
     const int x0 = int(at % unsigned(tiles_x)) * kMfmaCols, y0 = int(at / unsigned(tiles_x)) * (4 * R);
-    const size_t plane = size_t(H) * W;
-    const float *xb = x + size_t(b) * Cin * plane;
-    for (int i = threadIdx.x; i < TR * TC * (CinP / 4); i += 256)
+    const float *xb = x + size_t(b) * Cin * H * W;
+    for (int k = threadIdx.x; k < Kp; k += 256)
     {
-        const int c = i / (TR * TC) * 4, px = i % (TR * TC);
-        const int yy = y0 - 1 + px / TC, xx = x0 - 1 + px % TC;
-        f32x4 v{0.f, 0.f, 0.f, 0.f};
-        if (yy >= 0 && yy < H && xx >= 0 && xx < W)
-        {
-            const float *from = xb + size_t(c) * plane + size_t(yy) * W + xx;
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-                if (c + q < Cin)
-                    v[q] = from[q * plane];
-        }
-        *reinterpret_cast<f32x4 *>(tile_f + px * stride + c) = v;
+        const int c = k / 9, tap = k - 9 * c;
+        offset[k] = short((c * TR + tap / 3) * TC + tap % 3);  // below 66 * 18 * 18
     }
+    // loads without branches, so that several are in flight
+#pragma unroll 4
+    for (int i = threadIdx.x; i < n; i += 256)
+    {
+        const int c = i / (TR * TC), px = i % (TR * TC);
+        const int yy = y0 - 1 + px / TC, xx = x0 - 1 + px % TC;
+        const bool in = yy >= 0 && yy < H && xx >= 0 && xx < W;
+        float v = xb[in ? (size_t(c) * H + yy) * W + xx : 0];
+        if (lo)
+            v = lo[in ? ((size_t(b) * Cin + c) * (H / 2) + yy / 2) * (W / 2) + xx / 2 : 0] + v;
+        v = in ? v : 0.f;
+        if constexpr (kBf16)
+            tile[i] = f32_to_bf16_rne(v);
+        else
+            tile[i] = v;
+    }
+    for (int i = n + threadIdx.x; i < n + 2 * TR * TC; i += 256)
+        tile[i] = 0;  // the padding's k reach two channels past the last
     __syncthreads();
     const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
     const int j = lane % 16, kq = 4 * (lane / 16);
@@ -121,27 +152,32 @@ __global__ __launch_bounds__(256) void k_conv3x3_f32(const float *__restrict__ x
 #pragma unroll
         for (int r = 0; r < R; ++r)
             acc[t][r] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const float *wl = wm + size_t(t0 * 16 + j) * Kp + kq;
-    const float *xl = tile_f + (wave * R * TC + j) * stride + kq;
-#pragma unroll
-    for (int tap = 0; tap < 9; ++tap)
+    const E *xl = tile + wave * R * TC + j;
+    const E *wl = wm + size_t(t0 * 16 + j) * Kp + kq;
+    for (int kc = 0; kc < Kp; kc += 16)
     {
-        for (int c = 0; c < CinP; c += 16)
+        const s16x4 from = *reinterpret_cast<const s16x4 *>(offset + kc + kq);
+        E4 av[CT];
+#pragma unroll
+        for (int t = 0; t < CT; ++t)
+            av[t] = *reinterpret_cast<const E4 *>(wl + size_t(t) * 16 * Kp + kc);
+#pragma unroll
+        for (int r = 0; r < R; ++r)
         {
-            f32x4 av[CT], bv[R];
+            E4 bv;
+#pragma unroll
+            for (int it = 0; it < 4; ++it)
+                bv[it] = xl[int(from[it]) + r * TC];
 #pragma unroll
             for (int t = 0; t < CT; ++t)
-                av[t] = *reinterpret_cast<const f32x4 *>(wl + size_t(t) * 16 * Kp + tap * CinP + c);
+            {
+                if constexpr (kBf16)
+                    acc[t][r] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av[t], bv, acc[t][r], 0, 0, 0);
+                else
 #pragma unroll
-            for (int r = 0; r < R; ++r)
-                bv[r] = *reinterpret_cast<const f32x4 *>(xl + ((r + tap / 3) * TC + tap % 3) * stride + c);
-#pragma unroll
-            for (int s = 0; s < 4; ++s)
-#pragma unroll
-                for (int t = 0; t < CT; ++t)
-#pragma unroll
-                    for (int r = 0; r < R; ++r)
-                        acc[t][r] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[t][s], bv[r][s], acc[t][r], 0, 0, 0);
+                    for (int s = 0; s < 4; ++s)
+                        acc[t][r] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[t][s], bv[s], acc[t][r], 0, 0, 0);
+            }
         }
     }
     const int ox = x0 + j;
@@ -160,7 +196,7 @@ __global__ __launch_bounds__(256) void k_conv3x3_f32(const float *__restrict__ x
                 const int co = (t0 + t) * 16 + kq + v;
                 if (co < Cout)
                 {
-                    const size_t to = (size_t(b) * Cout + co) * plane + size_t(oy) * W + ox;
+                    const size_t to = ((size_t(b) * Cout + co) * H + oy) * W + ox;
                     float o = acc[t][r][v] + (bias ? bias[co] : 0.f);
                     if (relu)
                         o = o > 0.f ? o : 0.f;
@@ -190,10 +226,10 @@ __global__ __launch_bounds__(256) void k_conv3x3_f32(const float *__restrict__ x
 constexpr int kGStride = kTile * kTile + 4;
 constexpr int kXRow = kTile + 4, kXStride = (kTile + 2) * kXRow + 4;
 
-__global__ __launch_bounds__(256) void k_conv_wgrad(const float *__restrict__ x, const float *__restrict__ g,
-                                                    float *__restrict__ partial, int B, int Cin, int Cout, int CinP,
-                                                    int CoutP, int H, int W, int tiles_x, int tiles_per_image,
-                                                    int slices)
+__global__ __launch_bounds__(256) void k_conv_wgrad(const float *__restrict__ x, const float *__restrict__ lo,
+                                                    const float *__restrict__ g, float *__restrict__ partial, int B,
+                                                    int Cin, int Cout, int CinP, int CoutP, int H, int W, int tiles_x,
+                                                    int tiles_per_image, int slices)
 {
     __shared__ __align__(16) float lds[kWgT * (kGStride + kXStride)];
     float *gs = lds, *xs = lds + kWgT * kGStride;
@@ -241,6 +277,30 @@ __global__ __launch_bounds__(256) void k_conv_wgrad(const float *__restrict__ x,
             const bool in = xin && i < 2 * (kTile + 2) && xx >= 0 && xx < W && yy >= 0 && yy < H;
             ev[e] = xc[in ? yy * W + xx : 0];
             ev[e] = in ? ev[e] : 0.f;
+        }
+        if (lo)  // the input is x + up2(lo)
+        {
+            const float *lc = lo + (size_t(b) * Cin + min(ci0 + c, Cin - 1)) * (H / 2) * (W / 2);
+            float lv[kTile / 2 + 2], le[3];
+#pragma unroll
+            for (int r = 0; r < kTile / 2 + 2; ++r)  // rows 2 r - 1 and 2 r of the tile with its halo
+            {
+                const int yy = ty0 / 2 + r - 1;
+                const bool in = xin && tx0 + col < W && yy >= 0 && yy < H / 2;
+                lv[r] = lc[in ? yy * (W / 2) + (tx0 + col) / 2 : 0];
+                lv[r] = in ? lv[r] : 0.f;
+            }
+#pragma unroll
+            for (int e = 0; e < 3; ++e)
+            {
+                const int i = col + e * kTile, yy = ty0 + i / 2 - 1, xx = tx0 + (i % 2 ? kTile : -1);
+                const bool in = xin && i < 2 * (kTile + 2) && xx >= 0 && xx < W && yy >= 0 && yy < H;
+                le[e] = lc[in ? yy / 2 * (W / 2) + xx / 2 : 0];
+                ev[e] += in ? le[e] : 0.f;
+            }
+#pragma unroll
+            for (int r = 0; r < kTile + 2; ++r)
+                xv[r] += lv[(r + 1) / 2];
         }
         __syncthreads();
 #pragma unroll
@@ -360,122 +420,6 @@ __global__ __launch_bounds__(kReduceWeights *kReduceGroups) void k_wgrad_reduce(
     }
 }
 
-// ---- BF16 inference: implicit-GEMM convolution on the matrix cores --------
-// out[o][p] = sum_k Wb[o][k] X[k][p], k = c*9 + tap (the FP32 weight order),
-// with v_mfma_f32_16x16x16bf16_1k (FP32 accumulation).  Lane layout of that
-// instruction, checked on the device: A[i][k] in lane i + 16 (k/4), element
-// k%4; B[k][j] in lane j + 16 (k/4), element k%4; D[i][j] in lane
-// j + 16 (i/4), element i%4.  A 256-thread block computes 16 pixels of 4 rows
-// (one row per wave) for all output channels: the input tile with its halo
-// is staged in LDS as BF16 (round to nearest even), each wave builds the
-// im2col fragment of a 16-wide K chunk once and reuses it for every 16-channel
-// output tile; weights come packed as BF16 [Cout16][K16] (zero padded).
-typedef short bf16x4 __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ short f32_to_bf16_rne(float f)
-{
-    uint32_t u = __float_as_uint(f);
-    if ((u & 0x7fffffffu) > 0x7f800000u)
-        return short((u >> 16) | 0x40u);
-    u += 0x7fffu + ((u >> 16) & 1u);
-    return short(u >> 16);
-}
-
-// The k order is kept (a change of summation order moves activations across
-// BF16 rounding bounds, which the layers above amplify), so a lane's four
-// values of a chunk come from four places of the tile: their offsets are
-// looked up in a table in LDS, once per chunk for the R rows of a wave.
-// Dividing per value, with one row per wave, took 242 us for 16
-// -> 16 channels at 256 x 256, 32 samples; this takes 95 us, bound by the
-// 2-byte LDS reads (four per lane and chunk).  A prediction of 64 samples:
-// 3.5 -> 1.65 ms in these kernels.
-template <int CT, int R>
-__global__ __launch_bounds__(256) void k_conv3x3_bf16(const float *__restrict__ x, const short *__restrict__ wb,
-                                                      const float *__restrict__ bias, float *__restrict__ y, int Cin,
-                                                      int Cout, int Kp, int H, int W, int tiles_x, int relu)
-{
-    constexpr int TR = 4 * R + 2, TC = kMfmaCols + 2;
-    extern __shared__ __align__(16) short tile_bf[];  // Kp offsets (a zero's for the padding), then the tile, a zero
-    short *offset = tile_bf, *tile = tile_bf + Kp;
-    const int n = Cin * TR * TC;
-    unsigned at, b;
-    xcd_place(at, b);
-    const int x0 = int(at % unsigned(tiles_x)) * kMfmaCols, y0 = int(at / unsigned(tiles_x)) * (4 * R);
-    const float *xb = x + size_t(b) * Cin * H * W;
-    for (int k = threadIdx.x; k < Kp; k += 256)
-    {
-        const int c = k / 9, tap = k - 9 * c;
-        offset[k] = short((c * TR + tap / 3) * TC + tap % 3);  // below 64 * 18 * 18; c < Cin + 2
-    }
-    // loads without branches, so that several are in flight
-#pragma unroll 4
-    for (int i = threadIdx.x; i < n; i += 256)
-    {
-        const int c = i / (TR * TC), px = i % (TR * TC);
-        const int yy = y0 - 1 + px / TC, xx = x0 - 1 + px % TC;
-        const bool in = yy >= 0 && yy < H && xx >= 0 && xx < W;
-        const float v = xb[in ? (size_t(c) * H + yy) * W + xx : 0];
-        tile[i] = f32_to_bf16_rne(in ? v : 0.f);
-    }
-    for (int i = n + threadIdx.x; i < n + 2 * TR * TC; i += 256)
-        tile[i] = 0;  // the padding's k reach two channels past the last
-    __syncthreads();
-    const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
-    const int j = lane % 16, kq = 4 * (lane / 16);
-    const int t0 = int(blockIdx.z) * CT;
-    f32x4 acc[CT][R];
-#pragma unroll
-    for (int t = 0; t < CT; ++t)
-#pragma unroll
-        for (int r = 0; r < R; ++r)
-            acc[t][r] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const short *xl = tile + wave * R * TC + j;
-    const short *wl = wb + size_t(t0 * 16 + j) * Kp + kq;
-    for (int kc = 0; kc < Kp; kc += 16)
-    {
-        const bf16x4 from = *reinterpret_cast<const bf16x4 *>(offset + kc + kq);
-        bf16x4 av[CT];
-#pragma unroll
-        for (int t = 0; t < CT; ++t)
-            av[t] = *reinterpret_cast<const bf16x4 *>(wl + size_t(t) * 16 * Kp + kc);
-#pragma unroll
-        for (int r = 0; r < R; ++r)
-        {
-            bf16x4 bv;
-#pragma unroll
-            for (int it = 0; it < 4; ++it)
-                bv[it] = xl[int(from[it]) + r * TC];
-#pragma unroll
-            for (int t = 0; t < CT; ++t)
-                acc[t][r] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av[t], bv, acc[t][r], 0, 0, 0);
-        }
-    }
-    const int ox = x0 + j;
-#pragma unroll
-    for (int r = 0; r < R; ++r)
-    {
-        const int oy = y0 + wave * R + r;
-        if (oy >= H || ox >= W)
-            continue;
-#pragma unroll
-        for (int t = 0; t < CT; ++t)
-        {
-#pragma unroll
-            for (int v = 0; v < 4; ++v)
-            {
-                const int co = (t0 + t) * 16 + kq + v;
-                if (co < Cout)
-                {
-                    float o = acc[t][r][v] + bias[co];
-                    if (relu)
-                        o = o > 0.f ? o : 0.f;
-                    y[((size_t(b) * Cout + co) * H + oy) * W + ox] = o;
-                }
-            }
-        }
-    }
-}
-
 // wb[o*Kp + k] = bf16(w[o*9Cin + k]) for k < 9 Cin (padding stays zero)
 __global__ void k_pack_bf16(const float *__restrict__ w, short *__restrict__ wb, int Cin, int Cout, int Kp)
 {
@@ -487,19 +431,19 @@ __global__ void k_pack_bf16(const float *__restrict__ w, short *__restrict__ wb,
     wb[size_t(o) * Kp + k] = f32_to_bf16_rne(w[idx]);
 }
 
-// wm[o*Kp + k*CinP + c] = w[o][c][k] (Kp = 9 CinP);
-// wt[c*KpT + (8-k)*CoutP + o] = w[o][c][k] (KpT = 9 CoutP): the data
+// wm[o*Kp + c*9 + k] = w[o][c][k] (Kp = round16(9 Cin));
+// wt[c*KpT + o*9 + 8-k] = w[o][c][k] (KpT = round16(9 Cout)): the data
 // gradient's weights, input and output channels swapped, taps flipped.
 // Padding rows and columns stay zero.
 __global__ void k_pack(const float *__restrict__ w, float *__restrict__ wm, float *__restrict__ wt, int Cin, int Cout,
-                       int CinP, int CoutP)
+                       int Kp, int KpT)
 {
     const int idx = blockIdx.x * blockDim.x + threadIdx.x;
     if (idx >= Cout * Cin * 9)
         return;
     const int o = idx / (Cin * 9), c = (idx / 9) % Cin, k = idx % 9;
-    wm[(size_t(o) * 9 + k) * CinP + c] = w[idx];
-    wt[(size_t(c) * 9 + 8 - k) * CoutP + o] = w[idx];
+    wm[size_t(o) * Kp + c * 9 + k] = w[idx];
+    wt[size_t(c) * KpT + o * 9 + (8 - k)] = w[idx];
 }
 
 __global__ void k_pool2(const float *__restrict__ x, float *__restrict__ y, int BC, int H, int W)
@@ -527,19 +471,6 @@ __global__ void k_pool2_backward_add(const float *__restrict__ dy, const float *
         const int r = int(i % (size_t(H) * W)), yi = r / W, xi = r % W;
         const float v = dx[i] + 0.25f * dy[(bc * (H / 2) + yi / 2) * (W / 2) + xi / 2];
         dx[i] = a[i] > 0.f ? v : 0.f;
-    }
-}
-
-// z = up2(lo) + skip
-__global__ void k_upadd(const float *__restrict__ lo, const float *__restrict__ skip, float *__restrict__ z, int BC,
-                        int H, int W)
-{
-    const size_t n = size_t(BC) * H * W;
-    for (size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += size_t(gridDim.x) * blockDim.x)
-    {
-        const size_t bc = i / (size_t(H) * W);
-        const int r = int(i % (size_t(H) * W)), yi = r / W, xi = r % W;
-        z[i] = lo[(bc * (H / 2) + yi / 2) * (W / 2) + xi / 2] + skip[i];
     }
 }
 
@@ -660,7 +591,7 @@ struct lbm_surrogate
     bool packed = false;
     uint32_t adam_t = 0;
     float *in = nullptr, *tgt = nullptr, *out = nullptr, *dout = nullptr, *dtmp = nullptr;
-    float *a[14] = {}, *p[5] = {}, *z[4] = {}, *da[14] = {};
+    float *a[14] = {}, *p[5] = {}, *da[14] = {};
     float *partial[kConvs] = {};  // the weight gradients' slices
     double *loss_part = nullptr, *loss_dev = nullptr;
     float *history = nullptr;
@@ -723,7 +654,7 @@ int pack_all(lbm_surrogate *s)
     {
         const int n = kCout[k] * kCin[k] * 9;
         hipLaunchKernelGGL(k_pack, dim3((n + 255) / 256), dim3(256), 0, s->stream, s->params + s->w_off[k], s->wp[k],
-                           s->wt[k], kCin[k], kCout[k], round16(kCin[k]), round16(kCout[k]));
+                           s->wt[k], kCin[k], kCout[k], round16(9 * kCin[k]), round16(9 * kCout[k]));
         hipLaunchKernelGGL(k_pack_bf16, dim3((n + 255) / 256), dim3(256), 0, s->stream, s->params + s->w_off[k],
                            s->wb[k], kCin[k], kCout[k], round16(9 * kCin[k]));
     }
@@ -739,7 +670,7 @@ int pack_all(lbm_surrogate *s)
 // that (two at most for more than 32 input channels, whose tile would leave one
 // block per compute unit in LDS); the channel tiles of a layer too small for
 // 512 blocks of one row get blocks of their own.  16 -> 16 channels at 256 x
-// 256, 16 samples in FP32: 136 us with one row, 79 us with four.
+// 256, 16 samples in FP32: 136 us with one row, 74 us with four.
 template <class F>
 void conv_shape(int Cin, int Cout, int H, int W, int B, F f)
 {
@@ -766,58 +697,46 @@ void conv_shape(int Cin, int Cout, int H, int W, int B, F f)
         by_rows(integral_constant<int, 4>{});
 }
 
-// FP32 convolution of x (Cin channels) with packed weights wm ([Cout16][9][Cin16]) into y.
-void conv_f32(lbm_surrogate *s, const float *x, const float *wm, const float *bias, const float *mask, float *y, int Cin,
-              int Cout, int l, int B, bool relu)
+// Convolution of x, or of x + up2(lo), with packed weights wm ([Cout16][round16(9 Cin)]) into y.
+template <class E>
+void conv(lbm_surrogate *s, const float *x, const float *lo, const E *wm, const float *bias, const float *mask,
+          float *y, int Cin, int Cout, int l, int B, bool relu)
 {
-    const int H = s->LH[l], W = s->LW[l], tx = (W + kMfmaCols - 1) / kMfmaCols;
+    const int H = s->LH[l], W = s->LW[l], tx = (W + kMfmaCols - 1) / kMfmaCols, Kp = round16(9 * Cin);
     conv_shape(Cin, Cout, H, W, B, [&](auto ct, auto rows) {
         constexpr int CT = decltype(ct)::value, R = decltype(rows)::value;
         const int ty = (H + 4 * R - 1) / (4 * R);
-        const size_t lds = size_t(4 * R + 2) * (kMfmaCols + 2) * (round16(Cin) + 4) * sizeof(float);
-        hipLaunchKernelGGL((k_conv3x3_f32<CT, R>), dim3(unsigned(tx * ty), unsigned(B), unsigned((Cout + 15) / 16 / CT)),
-                           dim3(256), lds, s->stream, x, wm, bias, mask, y, Cin, Cout, H, W, tx, relu ? 1 : 0);
+        const size_t lds = size_t(Cin + 2) * (4 * R + 2) * (kMfmaCols + 2) * sizeof(E) + size_t(Kp) * sizeof(short);
+        const dim3 grid(unsigned(tx * ty), unsigned(B), unsigned((Cout + 15) / 16 / CT));
+        hipLaunchKernelGGL((k_conv3x3<E, CT, R>), grid, dim3(256), lds, s->stream, x, lo, wm, bias, mask, y, Cin, Cout,
+                           Kp, H, W, tx, relu ? 1 : 0);
     });
 }
 
-void conv_forward_bf16(lbm_surrogate *s, const float *x, int k, float *y, int l, int B, bool relu)
+void conv_forward(lbm_surrogate *s, const float *x, const float *lo, int k, float *y, int l, int B, bool relu,
+                  bool bf16)
 {
-    const int H = s->LH[l], W = s->LW[l], tx = (W + kMfmaCols - 1) / kMfmaCols, Kp = round16(9 * kCin[k]);
-    conv_shape(kCin[k], kCout[k], H, W, B, [&](auto ct, auto rows) {
-        constexpr int CT = decltype(ct)::value, R = decltype(rows)::value;
-        const int ty = (H + 4 * R - 1) / (4 * R);
-        const size_t lds = (size_t(kCin[k] + 2) * (4 * R + 2) * (kMfmaCols + 2) + Kp) * sizeof(short);
-        hipLaunchKernelGGL((k_conv3x3_bf16<CT, R>),
-                           dim3(unsigned(tx * ty), unsigned(B), unsigned((kCout[k] + 15) / 16 / CT)), dim3(256), lds,
-                           s->stream, x, s->wb[k], s->params + s->b_off[k], y, kCin[k], kCout[k], Kp, H, W, tx,
-                           relu ? 1 : 0);
-    });
-}
-
-void conv_forward(lbm_surrogate *s, const float *x, int k, float *y, int l, int B, bool relu, bool bf16 = false)
-{
+    const float *bias = s->params + s->b_off[k];
     if (bf16)
-    {
-        conv_forward_bf16(s, x, k, y, l, B, relu);
-        return;
-    }
-    conv_f32(s, x, s->wp[k], s->params + s->b_off[k], nullptr, y, kCin[k], kCout[k], l, B, relu);
+        conv<short>(s, x, lo, s->wb[k], bias, nullptr, y, kCin[k], kCout[k], l, B, relu);
+    else
+        conv<float>(s, x, lo, s->wp[k], bias, nullptr, y, kCin[k], kCout[k], l, B, relu);
 }
 
 // dx = data gradient of conv k for output gradient g (dx written, not
 // accumulated), with the ReLU mask of activation a (null: none)
 void conv_dgrad(lbm_surrogate *s, const float *g, int k, const float *a, float *dx, int l, int B)
 {
-    conv_f32(s, g, s->wt[k], nullptr, a, dx, kCout[k], kCin[k], l, B, false);
+    conv<float>(s, g, nullptr, s->wt[k], nullptr, a, dx, kCout[k], kCin[k], l, B, false);
 }
 
-void conv_wgrad(lbm_surrogate *s, const float *x, const float *g, int k, int l, int B)
+void conv_wgrad(lbm_surrogate *s, const float *x, const float *lo, const float *g, int k, int l, int B)
 {
     const int CinP = round16(kCin[k]), CoutP = round16(kCout[k]);
     const int slices = wgrad_slices(s, k, l, B);
     const dim3 grid(unsigned((CoutP / kWgT) * (CinP / kWgT)), unsigned(slices));
-    hipLaunchKernelGGL(k_conv_wgrad, grid, dim3(256), 0, s->stream, x, g, s->partial[k], B, kCin[k], kCout[k], CinP,
-                       CoutP, s->LH[l], s->LW[l], tiles_x(s, l), tiles(s, l), slices);
+    hipLaunchKernelGGL(k_conv_wgrad, grid, dim3(256), 0, s->stream, x, lo, g, s->partial[k], B, kCin[k], kCout[k],
+                       CinP, CoutP, s->LH[l], s->LW[l], tiles_x(s, l), tiles(s, l), slices);
 }
 
 // every convolution's gradient from its slices
@@ -849,12 +768,6 @@ void pool_backward_add(lbm_surrogate *s, const float *dy, const float *a, float 
                        s->LH[l_in], s->LW[l_in]);
 }
 
-void upadd(lbm_surrogate *s, const float *lo, const float *skip, float *z, int C, int l, int B)
-{
-    const size_t n = size_t(B) * C * s->LH[l] * s->LW[l];
-    hipLaunchKernelGGL(k_upadd, dim3(elem_grid(n)), dim3(256), 0, s->stream, lo, skip, z, B * C, s->LH[l], s->LW[l]);
-}
-
 void upsample_backward(lbm_surrogate *s, const float *dz, const float *a, float *dlo, int C, int l, int B)
 {
     const size_t n = size_t(B) * C * s->LH[l + 1] * s->LW[l + 1];
@@ -862,27 +775,26 @@ void upsample_backward(lbm_surrogate *s, const float *dz, const float *a, float 
                        s->LW[l]);
 }
 
-// Forward over s->in (B samples) into s->a, s->p, s->z, s->out; bf16: the
+// Forward over s->in (B samples) into s->a, s->p, s->out; bf16: the
 // convolutions on the matrix cores (inference).
 void forward(lbm_surrogate *s, int B, bool bf16 = false)
 {
-    conv_forward(s, s->in, 0, s->a[1], 0, B, true, bf16);
-    conv_forward(s, s->a[1], 1, s->a[2], 0, B, true, bf16);
+    conv_forward(s, s->in, nullptr, 0, s->a[1], 0, B, true, bf16);
+    conv_forward(s, s->a[1], nullptr, 1, s->a[2], 0, B, true, bf16);
     for (int l = 1; l <= 3; ++l)
     {
         pool(s, s->a[2 * l], s->p[l], kCout[2 * l - 1], l - 1, B);
-        conv_forward(s, s->p[l], 2 * l, s->a[2 * l + 1], l, B, true, bf16);
-        conv_forward(s, s->a[2 * l + 1], 2 * l + 1, s->a[2 * l + 2], l, B, true, bf16);
+        conv_forward(s, s->p[l], nullptr, 2 * l, s->a[2 * l + 1], l, B, true, bf16);
+        conv_forward(s, s->a[2 * l + 1], nullptr, 2 * l + 1, s->a[2 * l + 2], l, B, true, bf16);
     }
     pool(s, s->a[8], s->p[4], kCout[7], 3, B);
-    conv_forward(s, s->p[4], 8, s->a[9], 4, B, true, bf16);
+    conv_forward(s, s->p[4], nullptr, 8, s->a[9], 4, B, true, bf16);
     for (int m = 0; m < 4; ++m)
     {
         const int l = 3 - m, kk = 9 + m;
-        upadd(s, s->a[9 + m], s->a[8 - 2 * m], s->z[l], kCin[kk], l, B);
-        conv_forward(s, s->z[l], kk, s->a[10 + m], l, B, true, bf16);
+        conv_forward(s, s->a[8 - 2 * m], s->a[9 + m], kk, s->a[10 + m], l, B, true, bf16);
     }
-    conv_forward(s, s->a[13], 13, s->out, 0, B, false, bf16);
+    conv_forward(s, s->a[13], nullptr, 13, s->out, 0, B, false, bf16);
 }
 
 // Loss of s->out against s->tgt and the full parameter gradient into s->grad.
@@ -897,26 +809,26 @@ void loss_backward(lbm_surrogate *s, int B, double norm, float *history, int slo
                        history, slot);
     // Every da[] is complete, ReLU mask included, once its last share is in.
     // conv13 (no ReLU)
-    conv_wgrad(s, s->a[13], s->dout, 13, 0, B);
+    conv_wgrad(s, s->a[13], nullptr, s->dout, 13, 0, B);
     conv_dgrad(s, s->dout, 13, s->a[13], s->da[13], 0, B);
     for (int m = 3; m >= 0; --m)
     {
         const int l = 3 - m, kk = 9 + m;
-        conv_wgrad(s, s->z[l], s->da[10 + m], kk, l, B);
-        // dz is the skip's gradient: written straight into da[8-2m], which
+        conv_wgrad(s, s->a[8 - 2 * m], s->a[9 + m], s->da[10 + m], kk, l, B);
+        // the gradient of the sum is the skip's: written straight into da[8-2m], which
         // the pool's share completes
         conv_dgrad(s, s->da[10 + m], kk, nullptr, s->da[8 - 2 * m], l, B);
         upsample_backward(s, s->da[8 - 2 * m], s->a[9 + m], s->da[9 + m], kCin[kk], l, B);
     }
-    conv_wgrad(s, s->p[4], s->da[9], 8, 4, B);
+    conv_wgrad(s, s->p[4], nullptr, s->da[9], 8, 4, B);
     conv_dgrad(s, s->da[9], 8, nullptr, s->dtmp, 4, B);
     pool_backward_add(s, s->dtmp, s->a[8], s->da[8], kCin[8], 3, B);
     for (int l = 3; l >= 0; --l)
     {
         const int k1 = 2 * l + 1, k0 = 2 * l;
-        conv_wgrad(s, s->a[k1], s->da[k1 + 1], k1, l, B);
+        conv_wgrad(s, s->a[k1], nullptr, s->da[k1 + 1], k1, l, B);
         conv_dgrad(s, s->da[k1 + 1], k1, s->a[k1], s->da[k1], l, B);
-        conv_wgrad(s, l == 0 ? s->in : s->p[l], s->da[k1], k0, l, B);
+        conv_wgrad(s, l == 0 ? s->in : s->p[l], nullptr, s->da[k1], k0, l, B);
         if (l > 0)
         {
             conv_dgrad(s, s->da[k1], k0, nullptr, s->dtmp, l, B);
@@ -1080,7 +992,6 @@ int lbm_surrogate_create(uint32_t height, uint32_t width, uint32_t max_batch, lb
     {
         C_TRY(alloc(s, &s->a[10 + m], act_floats(s, kCout[9 + m], 3 - m)));
         C_TRY(alloc(s, &s->da[10 + m], act_floats(s, kCout[9 + m], 3 - m)));
-        C_TRY(alloc(s, &s->z[3 - m], act_floats(s, kCin[9 + m], 3 - m)));
     }
     for (int l = 1; l <= 4; ++l)
         C_TRY(alloc(s, &s->p[l], act_floats(s, kCout[2 * l - 1], l)));
