@@ -50,12 +50,12 @@ struct FusePlan
 //   3.9e5  32x32 T 5: 6.39 / 4.96 / 5.00   32x16 T 4: 5.81 / 4.98 / 5.12 (FP64 collision 7.12, 6.90)
 //   1.0e6  32x16 T 3: 11.7 / 10.1 / 10.4   32x16 T 4: 12.2 / 10.7 / 11.1   march: 14.8 / 13.9 / 18.0
 //   2.0e6  32x16 T 3: 23.2 / 18.5 / 19.1   32x16 T 4: 22.9 / 19.8 / 20.5   march: 24.8 / 19.8 / 24.1
-//   3.0e6  32x16 T 3: 39.0 / 27.2 / 28.0   march: 35.1 / 27.2 / 27.5
+//   3.0e6  32x16 T 3: 39.0 / 27.2 / 28.0   march: 35.1 / 27.2 / 27.5 (3001 x 997 for nsol, FP32: 31.0, 28.4)
 // FP64 marches from 1.5e6: at 2.0e6 the collision layout takes 24.7 marched
 // and 27.3 in tiles.
 inline FusePlan plan_fusion(size_t elem, uint64_t nodes)
 {
-    if (nodes >= (elem == 8 ? 1500000u : (elem == 4 ? 3000000u : 3500000u)))
+    if (nodes >= (elem == 8 ? 1500000u : (elem == 4 ? 2500000u : 3500000u)))
         return FusePlan{kMarchMaxSteps, false, TileShape::k32x32};
     if (nodes <= 36000u)
         return FusePlan{5u, true, TileShape::k16x16};
