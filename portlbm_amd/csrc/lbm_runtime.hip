@@ -1,19 +1,24 @@
 // MI355X (gfx950) implementation of the C ABI declared in include/lbm_hip.h.
 //
-// One launch per time step fuses what the reference runs as three to seven
-// blocking launches (include/lbm/gpu/nptl/nptl.hpp:116-141,
-// npol/npol.hpp:180-201, nsol/nsol.hpp:184-205): bounce-back is folded into
-// the pull through the per-node code table, the Zou-He outlet is computed by
-// the outlet nodes themselves, and macroscopic outputs are written only on
-// the steps whose values the host can observe.  The one-lattice schemes keep
-// the reference's buffered geometry and need one halo refresh before each
-// step (two small launches).
+// One launch fuses what the reference runs as three to seven blocking launches
+// per step (include/lbm/gpu/nptl/nptl.hpp:116-141, npol/npol.hpp:180-201,
+// nsol/nsol.hpp:184-205): bounce-back is folded into the pull through the
+// per-node code table, the Zou-He outlet is computed by the outlet nodes
+// themselves, and macroscopic outputs are written only on the steps whose
+// values the host can observe.  Where several steps are asked for, one launch
+// does several of them (lbm_march.hpp); the one-step kernels of this file do
+// single steps, the steps at which the 16-bit forms change their reference,
+// and the one-lattice schemes in place.  Those keep the reference's buffered
+// geometry, with the edge copies in side arrays or one halo refresh before
+// each step (two small launches), unless a second, unexpanded lattice is cheap
+// (plan_compact): then they run the two-lattice launches on it.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <new>
 #include <string>
 #include <utility>
 #include <vector>
@@ -38,6 +43,20 @@ int lbm_set_error(int code, const std::string &msg)
 }
 
 static int fail(int code, const std::string &msg) { return lbm_set_error(code, msg); }
+
+// f(), whose host buffers may be larger than memory: no exception leaves a C entry.
+template <class F>
+static int with_host_memory(const char *what, F f)
+{
+    try
+    {
+        return f();
+    }
+    catch (const std::bad_alloc &)
+    {
+        return fail(LBM_ERR_OUT_OF_MEMORY, std::string(what) + ": no host memory to convert the lattice in");
+    }
+}
 
 #define LBM_HIP_TRY(expr)                                                                          \
     do                                                                                             \
@@ -2256,11 +2275,18 @@ int lbm_create(const lbm_desc *desc, lbm_ctx **out)
         if (lbm_create(&d, &c->inner) == LBM_OK)
         {
             c->inner->outlet_active = c->outlet_active;
-            if (c->inner->ref_len)
-                c->ref_len = std::max(c->Hx, c->H) + 64u;
-            c->outer_phase.assign(c->N, int8_t(-1));
-            *out = c;
-            return LBM_OK;
+            try
+            {
+                c->outer_phase.assign(c->N, int8_t(-1));
+                if (c->inner->ref_len)
+                    c->ref_len = std::max(c->Hx, c->H) + 64u;
+                *out = c;
+                return LBM_OK;
+            }
+            catch (const std::bad_alloc &)
+            {
+                lbm_destroy(c->inner);
+            }
         }
         (void)hipGetLastError();
         c->inner = nullptr;  // no memory for two lattices: in place
@@ -2301,7 +2327,6 @@ int lbm_create(const lbm_desc *desc, lbm_ctx **out)
     // 1024, 3844 tiles, 154 / 174).
     size_t side_bytes = 0;
     int cus = 0;
-    FusePlan fuse;        // nptl / lptl: several steps per launch
     {
         int dev = 0;
         CREATE_TRY(hipGetDevice(&dev));
@@ -2393,12 +2418,14 @@ int lbm_set_phase(lbm_ctx *c, const int8_t *phase, size_t n)
         return fail(LBM_ERR_INVALID_ARGUMENT, "lbm_set_phase: node_count must equal the expanded node count");
     if (c->inner)
     {
-        std::vector<int8_t> own(size_t(c->H) * c->V);
-        for_runs(c, [&](size_t u, size_t e, size_t k) { std::copy_n(phase + e, k, own.begin() + u); });
-        if (int rc = lbm_set_phase(c->inner, own.data(), own.size()))
-            return rc;
-        std::copy_n(phase, n, c->outer_phase.begin());
-        return LBM_OK;
+        return with_host_memory("lbm_set_phase", [&]() -> int {
+            std::vector<int8_t> own(size_t(c->H) * c->V);
+            for_runs(c, [&](size_t u, size_t e, size_t k) { std::copy_n(phase + e, k, own.begin() + u); });
+            if (int rc = lbm_set_phase(c->inner, own.data(), own.size()))
+                return rc;
+            std::copy_n(phase, n, c->outer_phase.begin());
+            return LBM_OK;
+        });
     }
     LBM_HIP_TRY(hipMemcpyAsync(c->phase, phase, n, hipMemcpyHostToDevice, c->stream));
     LBM_HIP_TRY(hipStreamSynchronize(c->stream));
@@ -2474,14 +2501,17 @@ int lbm_get_node_codes(lbm_ctx *c, uint16_t *codes, size_t n)
         return fail(LBM_ERR_INVALID_ARGUMENT, "lbm_get_node_codes: null argument");
     if (c->inner)
     {
-        if (n != c->N)
-            return fail(LBM_ERR_INVALID_ARGUMENT, "lbm_get_node_codes: node_count must equal the expanded node count");
-        std::vector<uint16_t> own(size_t(c->H) * c->V);
-        if (int rc = lbm_get_node_codes(c->inner, own.data(), own.size()))
-            return rc;
-        std::fill_n(codes, n, uint16_t(0));
-        for_runs(c, [&](size_t u, size_t e, size_t k) { std::copy_n(own.begin() + u, k, codes + e); });
-        return LBM_OK;
+        return with_host_memory("lbm_get_node_codes", [&]() -> int {
+            if (n != c->N)
+                return fail(LBM_ERR_INVALID_ARGUMENT,
+                            "lbm_get_node_codes: node_count must equal the expanded node count");
+            std::vector<uint16_t> own(size_t(c->H) * c->V);
+            if (int rc = lbm_get_node_codes(c->inner, own.data(), own.size()))
+                return rc;
+            std::fill_n(codes, n, uint16_t(0));
+            for_runs(c, [&](size_t u, size_t e, size_t k) { std::copy_n(own.begin() + u, k, codes + e); });
+            return LBM_OK;
+        });
     }
     if (!c->initialized)
         return fail(LBM_ERR_STATE, "lbm_get_node_codes: call lbm_init_populations first");
@@ -2696,19 +2726,23 @@ int lbm_get_pass_populations(lbm_ctx *c, double *values, size_t count)
         return fail(LBM_ERR_INVALID_ARGUMENT, "lbm_get_pass_populations: null argument");
     if (c->inner)
     {
-        if (!c->inner->pass)
-            return fail(LBM_ERR_STATE, "lbm_get_pass_populations: no split step has run");
-        if (count != 9ull * c->N)
-            return fail(LBM_ERR_INVALID_ARGUMENT,
-                        "lbm_get_pass_populations: count must be 9 * expanded node count");
-        const size_t M = size_t(c->H) * c->V;
-        std::vector<double> own(9 * M);
-        if (int rc = lbm_get_pass_populations(c->inner, own.data(), own.size()))
-            return rc;
-        std::fill_n(values, count, 0.0);
-        for (uint32_t d = 0; d < 9; ++d)
-            for_runs(c, [&](size_t u, size_t e, size_t k) { std::copy_n(&own[d * M + u], k, values + size_t(d) * c->N + e); });
-        return LBM_OK;
+        return with_host_memory("lbm_get_pass_populations", [&]() -> int {
+            if (!c->inner->pass)
+                return fail(LBM_ERR_STATE, "lbm_get_pass_populations: no split step has run");
+            if (count != 9ull * c->N)
+                return fail(LBM_ERR_INVALID_ARGUMENT,
+                            "lbm_get_pass_populations: count must be 9 * expanded node count");
+            const size_t M = size_t(c->H) * c->V;
+            std::vector<double> own(9 * M);
+            if (int rc = lbm_get_pass_populations(c->inner, own.data(), own.size()))
+                return rc;
+            std::fill_n(values, count, 0.0);
+            for (uint32_t d = 0; d < 9; ++d)
+                for_runs(c, [&](size_t u, size_t e, size_t k) {
+                    std::copy_n(&own[d * M + u], k, values + size_t(d) * c->N + e);
+                });
+            return LBM_OK;
+        });
     }
     if (!c->pass)
         return fail(LBM_ERR_STATE, "lbm_get_pass_populations: no split step has run");
@@ -2879,7 +2913,7 @@ int lbm_get_state(lbm_ctx *c, void *buf, size_t bytes)
         return fail(LBM_ERR_INVALID_ARGUMENT, "lbm_get_state: size must be lbm_state_size()");
     char *out = static_cast<char *>(buf);
     if (c->inner)
-        return get_inner_state(c, out);
+        return with_host_memory("lbm_get_state", [&] { return get_inner_state(c, out); });
     const uint32_t lattices = c->two_lattice ? 2u : 1u;
     const uint32_t cur = uint32_t(c->cur);
     std::memcpy(out, &c->iteration, 8);
@@ -2912,7 +2946,7 @@ int lbm_set_state(lbm_ctx *c, const void *buf, size_t bytes)
     if (lattices != (c->two_lattice ? 2u : 1u) || cur >= lattices)
         return fail(LBM_ERR_INVALID_ARGUMENT, "lbm_set_state: state of another algorithm");
     if (c->inner)
-        return set_inner_state(c, in, iteration);
+        return with_host_memory("lbm_set_state", [&] { return set_inner_state(c, in, iteration); });
     size_t off = 16;
     const size_t lat_bytes = c->lattice_elems * c->elem;
     // pageable source: blocking copies once the context's stream is idle,
@@ -2943,22 +2977,25 @@ int lbm_get_populations(lbm_ctx *c, double *values, size_t count)
         return fail(LBM_ERR_INVALID_ARGUMENT, "lbm_get_populations: count must be 9 * expanded node count");
     if (c->inner)
     {
-        const size_t M = size_t(c->H) * c->V;
-        std::vector<double> own(9 * M);
-        if (int rc = lbm_get_populations(c->inner, own.data(), own.size()))
-            return rc;
-        // buffer nodes are not kept: the rest state, as after lbm_init_populations
-        static const double w[9] = {1.0 / 36, 1.0 / 9, 1.0 / 36, 1.0 / 9, 4.0 / 9, 1.0 / 9, 1.0 / 36, 1.0 / 9, 1.0 / 36};
-        const int layout = c->desc.layout;
-        for (uint32_t d = 0; d < 9; ++d)
-            for (size_t e = 0; e < c->N; ++e)
-                values[flat_index(layout, e, d, c->N)] = w[d];
-        for (uint32_t d = 0; d < 9; ++d)
-            for_runs(c, [&](size_t u, size_t e, size_t k) {
-                for (size_t i = 0; i < k; ++i)
-                    values[flat_index(layout, e + i, d, c->N)] = own[flat_index(layout, u + i, d, M)];
-            });
-        return LBM_OK;
+        return with_host_memory("lbm_get_populations", [&]() -> int {
+            const size_t M = size_t(c->H) * c->V;
+            std::vector<double> own(9 * M);
+            if (int rc = lbm_get_populations(c->inner, own.data(), own.size()))
+                return rc;
+            // buffer nodes are not kept: the rest state, as after lbm_init_populations
+            static const double w[9] = {1.0 / 36, 1.0 / 9, 1.0 / 36, 1.0 / 9, 4.0 / 9,
+                                        1.0 / 9,  1.0 / 36, 1.0 / 9, 1.0 / 36};
+            const int layout = c->desc.layout;
+            for (uint32_t d = 0; d < 9; ++d)
+                for (size_t e = 0; e < c->N; ++e)
+                    values[flat_index(layout, e, d, c->N)] = w[d];
+            for (uint32_t d = 0; d < 9; ++d)
+                for_runs(c, [&](size_t u, size_t e, size_t k) {
+                    for (size_t i = 0; i < k; ++i)
+                        values[flat_index(layout, e + i, d, c->N)] = own[flat_index(layout, u + i, d, M)];
+                });
+            return LBM_OK;
+        });
     }
     if (int rc = ensure_stage(c))
         return rc;
@@ -2980,19 +3017,21 @@ int lbm_set_populations(lbm_ctx *c, const double *values, size_t count)
         return fail(LBM_ERR_INVALID_ARGUMENT, "lbm_set_populations: null argument");
     if (c->inner)
     {
-        if (!c->inner->initialized)
-            return fail(LBM_ERR_STATE, "lbm_set_populations: call lbm_init_populations first");
-        if (count != 9ull * c->N)
-            return fail(LBM_ERR_INVALID_ARGUMENT, "lbm_set_populations: count must be 9 * expanded node count");
-        const size_t M = size_t(c->H) * c->V;
-        const int layout = c->desc.layout;
-        std::vector<double> own(9 * M);
-        for (uint32_t d = 0; d < 9; ++d)
-            for_runs(c, [&](size_t u, size_t e, size_t k) {
-                for (size_t i = 0; i < k; ++i)
-                    own[flat_index(layout, u + i, d, M)] = values[flat_index(layout, e + i, d, c->N)];
-            });
-        return lbm_set_populations(c->inner, own.data(), own.size());
+        return with_host_memory("lbm_set_populations", [&]() -> int {
+            if (!c->inner->initialized)
+                return fail(LBM_ERR_STATE, "lbm_set_populations: call lbm_init_populations first");
+            if (count != 9ull * c->N)
+                return fail(LBM_ERR_INVALID_ARGUMENT, "lbm_set_populations: count must be 9 * expanded node count");
+            const size_t M = size_t(c->H) * c->V;
+            const int layout = c->desc.layout;
+            std::vector<double> own(9 * M);
+            for (uint32_t d = 0; d < 9; ++d)
+                for_runs(c, [&](size_t u, size_t e, size_t k) {
+                    for (size_t i = 0; i < k; ++i)
+                        own[flat_index(layout, u + i, d, M)] = values[flat_index(layout, e + i, d, c->N)];
+                });
+            return lbm_set_populations(c->inner, own.data(), own.size());
+        });
     }
     if (!c->initialized)
         return fail(LBM_ERR_STATE, "lbm_set_populations: call lbm_init_populations first");

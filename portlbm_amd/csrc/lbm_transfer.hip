@@ -9,7 +9,9 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
+#include <memory>
 #include <mutex>
+#include <new>
 #include <thread>
 #include <vector>
 
@@ -136,6 +138,17 @@ hipError_t download(const HostPiece *pieces, size_t count, hipStream_t stream)
     // chunks of at most a slot, over pieces that adjoin on the device
     std::vector<Chunk> chunks;
     size_t total = 0;
+    try
+    {
+        size_t bytes = 0;
+        for (size_t p = 0; p < count; ++p)
+            bytes += pieces[p].bytes;
+        chunks.reserve(bytes / kSlotBytes + count + 1);
+    }
+    catch (const std::bad_alloc &)
+    {
+        return through_runtime(pieces, count, stream);
+    }
     for (size_t p = 0; p < count; ++p)
     {
         const char *src = static_cast<const char *>(pieces[p].src);
@@ -152,9 +165,11 @@ hipError_t download(const HostPiece *pieces, size_t count, hipStream_t stream)
     const size_t nc = chunks.size();
     std::atomic<size_t> issued{0}, next{0};
     std::atomic<int> error{hipSuccess};
-    std::vector<std::atomic<bool>> emptied(nc);
-    for (auto &e : emptied)
-        e.store(false, std::memory_order_relaxed);
+    const std::unique_ptr<std::atomic<bool>[]> emptied(new (std::nothrow) std::atomic<bool>[nc]);
+    if (!emptied)
+        return through_runtime(pieces, count, stream);
+    for (size_t i = 0; i < nc; ++i)
+        emptied[i].store(false, std::memory_order_relaxed);
     // takes the next chunk below `limit`, if there is one: waits for it to
     // arrive, copies it, frees its slot
     auto drain_one = [&](size_t limit) -> bool {
