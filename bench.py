@@ -6,13 +6,15 @@
 
 Workload: the 8192 x 2048 porous channel (seeded non-overlapping discs,
 radii U[4, 16), porosity 0.7), tau 0.6, inlet density 1.05, outlet 1.0.
-The default line is nptl in FP64 in its fastest layout on this workload,
-the collision layout (the sweep times every algorithm x layout x storage).
-A step is one fused time step of the whole lattice with the inputs resident
-in HBM.  The unit of work is a fluid-node update; the line reports MFLUPS
-(10^6 fluid-node updates per second), the kernel's achieved HBM bandwidth
+The default line is nptl in FP64 in the collision layout (the sweep times
+every algorithm x layout x storage).
+A step is one time step of the whole lattice with the inputs resident in
+HBM; one launch advances up to four steps and reads and writes the lattice
+once.  The unit of work is a fluid-node update; the line reports MFLUPS
+(10^6 fluid-node updates per second), the launches' achieved HBM bandwidth
 against the MI355X peak (algorithmic bytes: 2 x 9 x sizeof(storage) per
-fluid node), and the CPU oracle timed on the host cores as a baseline.
+fluid node and launch), and the CPU oracle timed on the host cores as a
+baseline.
 
 Prints one JSON line.  Optional studies, each written to its own JSON file
 before the line is printed:
@@ -23,8 +25,8 @@ before the line is printed:
                          number of steps (--study-scenario, --study-taus,
                          --study-steps, --study-average)
   --steady-study OUT     the same at the steady state of a 1024x256 channel
-  --batched OUT          512 uneven channels: per-domain launches, one
-                         persistent launch per step, autotuned graph replay
+  --batched OUT          512 uneven channels: per-domain launches, persistent
+                         launches for all domains, autotuned graph replay
 """
 from __future__ import annotations
 
@@ -122,24 +124,15 @@ def measured_traffic(algorithm: str, layout: str, storage: str, scenario: str = 
     return None if rec is None else float(rec["bytes_per_launch"])
 
 
-def kernel_of(algorithm: str, layout: str, storage: str) -> str:
-    """The step kernel the library launches for a cell of the default
-    workload (work-group 1024 for npol / nsol: 32 x 32 and 30 x 31 tiles,
-    the staged block kernel in their FP64/FP32 collision layout, the tile
-    sweep elsewhere; 256 for lptl's 1-D kernel).
-    lptl runs nptl's kernels where those are faster: the staged kernel in the
-    collision layout and the FP64/FP32 bundle layout, the row kernel in
-    16-bit storage; its own 1-D kernel only in the FP64/FP32 stream layout."""
-    sixteen = storage in ("f16-shifted", "bf16-shifted")
-    if algorithm in ("nptl", "lptl"):
-        if layout == "collision" or (layout == "bundle" and not sixteen):
-            return "k_step_nptl_staged"
-        if algorithm == "lptl" and not sixteen:
-            return "k_step_lptl"
-        return "k_step_nptl"
-    if layout == "collision" and not sixteen:
-        return "k_step_tile_staged"
-    return "k_step_tile_sweep"
+# Steps per launch and the kernel of every cell of the default workload: the
+# lattice is large enough for the marching kernel in every storage, and npol
+# and nsol run it on their unexpanded lattice.
+STEPS_PER_LAUNCH = 4
+STEP_KERNEL = "k_march"
+
+
+def launches_of(steps: int) -> int:
+    return -(-steps // STEPS_PER_LAUNCH)
 
 
 def sweep(out_path: str, steps: int, warmup: int, cpu_budget_s: float = 0.0) -> None:
@@ -159,9 +152,9 @@ def sweep(out_path: str, steps: int, warmup: int, cpu_budget_s: float = 0.0) -> 
             for layout in ("collision", "stream", "bundle"):
                 r = time_gpu(workload(algorithm, layout, storage, steps), steps, warmup)
                 mflups = r["fluid"] * steps / (r["dev_ms"] * 1e-3) / 1e6
-                gbps = mflups * 1e6 * 2 * 9 * storage_bytes(storage) / 1e9
+                gbps = r["fluid"] * 2 * 9 * storage_bytes(storage) * launches_of(steps) / (r["dev_ms"] * 1e-3) / 1e9
                 row = {"algorithm": algorithm, "layout": layout, "storage": storage,
-                       "kernel": kernel_of(algorithm, layout, storage), "mflups": round(mflups, 1),
+                       "kernel": STEP_KERNEL, "mflups": round(mflups, 1),
                        "mlups_all": round(INNER_H * INNER_V * steps / (r["dev_ms"] * 1e-3) / 1e6, 1),
                        "gbps": round(gbps, 1), "hbm_frac": round(gbps / HBM_PEAK_GBPS, 4),
                        "ms_per_step": round(r["dev_ms"] / steps, 4)}
@@ -315,7 +308,7 @@ def steady_precision_study(out_path: str, inner_h: int = 1024, inner_v: int = 25
 def batched(out_path: str, steps: int, count: int = 512,
             modes=("per-domain", "persistent", "graph")) -> dict:
     """512 uneven porous channels in FP32 (portlbm_amd.workloads.batch_channels):
-    per-domain launches vs one persistent launch per step vs the whole run in
+    per-domain launches vs launches for all domains at once vs the whole run in
     one hipGraph with autotuned tiles (`modes` picks which are timed)."""
     docs = workloads.batch_channels(count, steps=steps)
     rows = {}
@@ -399,7 +392,7 @@ def main() -> int:
     secs = r["dev_ms"] * 1e-3
     mflups = r["fluid"] * args.steps / secs / 1e6
     bytes_per_node = 2 * 9 * storage_bytes(args.storage)
-    launch_ms = r["dev_ms"] / args.steps  # one kernel launch per step for nptl/lptl
+    launch_ms = r["dev_ms"] / launches_of(args.steps)
     achieved = r["fluid"] * bytes_per_node / (launch_ms * 1e-3) / 1e9
     line = {
         "metric": "MLUPS & % HBM roofline at 8192x2048; steps-to-steady warm-start vs plain",
@@ -426,6 +419,7 @@ def main() -> int:
                      "frac": round(achieved / HBM_PEAK_GBPS, 4),
                      "traffic": measured_traffic(args.algorithm, args.layout, args.storage, args.scenario)},
         "kernel_ms": round(launch_ms, 5),
+        "steps_per_launch": STEPS_PER_LAUNCH,
         "bytes_per_fluid_node": bytes_per_node,
         "mass": r["mass"],
     }

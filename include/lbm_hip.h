@@ -316,7 +316,7 @@ typedef struct lbm_batch_domain {
 
 enum lbm_batch_mode {
     LBM_BATCH_PER_DOMAIN = 0, /* one launch per domain and step */
-    LBM_BATCH_PERSISTENT = 1, /* one launch per step: a fixed grid strides over the tiles of all domains */
+    LBM_BATCH_PERSISTENT = 1, /* launches for all domains at once, of up to six steps */
     LBM_BATCH_GRAPH = 2       /* the persistent launches of the whole run captured in one hipGraph */
 };
 

@@ -1,9 +1,10 @@
-// Batched domains: many independent channels of uneven size advanced by one
-// persistent kernel per step (a fixed grid striding over the tiles of all
-// domains), optionally with the whole run captured in one hipGraph.  Each
-// domain is an unexpanded two-lattice pull in the stream layout, updated by
-// the same device functions as the single-lattice kernels (pull with
-// bounce-back bits, Zou-He outlet, BGK, full-segment stores).
+// Batched domains: many independent channels of uneven size advanced by
+// launches for all of them: several steps at a time by marching waves or LDS
+// tiles (lbm_march.hpp), a single step by one persistent kernel (a fixed grid
+// striding over the tiles of all domains); optionally the whole run captured in
+// one hipGraph.  Each domain is an unexpanded two-lattice pull in the stream
+// layout, updated by the same device functions as the single-lattice kernels
+// (pull with bounce-back bits, Zou-He outlet, BGK, full-segment stores).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

@@ -22,13 +22,13 @@
 // us per step, 8192 x 2048 porous channel, one step per launch -> T = 4
 // (T = 2, 3 in between: FP64 stream 239, 168):
 //            stream          collision       bundle
-//   FP64     383 -> 139      362 -> 157      366 -> 151
+//   FP64     383 -> 139      362 -> 151      366 -> 151
 //   FP32     204 -> 104      235 -> 115      242 -> 116
 //   FP16     128 -> 106      177 -> 113      184 -> 113
 // (FP16 with stochastic rounding, cylinder channel: 160 -> 122.)
 // What bounds it at T = 4: vector instructions, 62 % of the cycles in FP64
 // (rocprofv3: 2.06e8 per launch of 557 us) with two waves per SIMD, next to
-// 2.55 GB moved per launch (4.6 TB/s).
+// 2.65 GB moved per launch (4.8 TB/s).
 
 #include "lbm_march.hpp"
 
