@@ -463,9 +463,13 @@ __device__ __forceinline__ void collide(C f[9], C omega, C &rho, C &jx, C &jy, C
         f[d] = -omega * (f[d] - feq[d]) + f[d];
 }
 
-// collide<C, kPromote, kFull> where every population is finite: the terms that
-// kFull keeps (x + 0 f) change nothing then.  A population that is not makes
-// the density infinite or NaN, and the wave takes the full sums.
+// collide<C, kPromote, kFull> where the populations and their moments are
+// finite: the terms that kFull keeps (x + 0 f, 0 jx + jy) change nothing then.
+// A population that is not finite makes the density infinite or NaN; the
+// momentum can overflow beside a finite density (f5 and -f3 near the largest
+// number).  All of that ends in rho - 1.5 |j|^2, the rest population's
+// equilibrium but for its weight: where it is not finite the wave takes the
+// full sums.
 template <class C, bool kPromote, bool kFull>
 __device__ __forceinline__ void collide_node(C f[9], C omega, C &rho, C &jx, C &jy, C &usq)
 {
@@ -474,18 +478,18 @@ __device__ __forceinline__ void collide_node(C f[9], C omega, C &rho, C &jx, C &
 #pragma unroll
     for (int d = 1; d < 9; ++d)
         rho += f[d];
+    jx = ((((-f[0] + f[2]) - f[3]) + f[5]) - f[6]) + f[8];
+    jy = ((((-f[0] - f[1]) - f[2]) + f[6]) + f[7]) + f[8];
+    usq = jx * jx + jy * jy;
+    const A s = A(1.5) * A(usq), rest = A(rho) - s;
     if constexpr (kFull)
     {
-        if (__builtin_expect(__any(!__builtin_isfinite(rho)), 0))
+        if (__builtin_expect(__any(!__builtin_isfinite(rest)), 0))
         {
             collide<C, kPromote, true>(f, omega, rho, jx, jy, usq);
             return;
         }
     }
-    jx = ((((-f[0] + f[2]) - f[3]) + f[5]) - f[6]) + f[8];
-    jy = ((((-f[0] - f[1]) - f[2]) + f[6]) + f[7]) + f[8];
-    usq = jx * jx + jy * jy;
-    const A s = A(1.5) * A(usq);
     C feq[9];
 #pragma unroll
     for (int d = 0; d < 4; ++d)
@@ -496,7 +500,7 @@ __device__ __forceinline__ void collide_node(C f[9], C omega, C &rho, C &jx, C &
         feq[d] = C(A(weight<C>(d)) * (A(rho + t) + q - s));
         feq[8 - d] = C(A(weight<C>(8 - d)) * (A(rho - t) + q - s));
     }
-    feq[4] = C(A(weight<C>(4)) * (A(rho) - s));
+    feq[4] = C(A(weight<C>(4)) * rest);
 #pragma unroll
     for (int d = 0; d < 9; ++d)
         f[d] = -omega * (f[d] - feq[d]) + f[d];
