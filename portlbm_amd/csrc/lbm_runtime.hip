@@ -2595,6 +2595,23 @@ int lbm_run(lbm_ctx *c, uint32_t steps, uint32_t frame_interval)
     return LBM_OK;
 }
 
+// What the frame copies need and does not exist yet: a call that ran out of
+// memory half-way leaves the rest to the next.
+static hipError_t ensure_frames(lbm_ctx *c)
+{
+    if (!c->copy_stream)
+        if (hipError_t e = hipStreamCreateWithFlags(&c->copy_stream, hipStreamNonBlocking))
+            return e;
+    for (hipEvent_t *event : {&c->ev_frame, &c->ev_copied[0], &c->ev_copied[1]})
+        if (!*event)
+            if (hipError_t e = hipEventCreateWithFlags(event, hipEventDisableTiming))
+                return e;
+    if (!c->frame_host)
+        return hipHostMalloc(reinterpret_cast<void **>(&c->frame_host), 4ull * std::max(1u, c->D) * sizeof(double),
+                             hipHostMallocDefault);
+    return hipSuccess;
+}
+
 int lbm_run_frames(lbm_ctx *c, uint32_t steps, uint32_t frame_interval)
 {
     if (!c)
@@ -2603,19 +2620,16 @@ int lbm_run_frames(lbm_ctx *c, uint32_t steps, uint32_t frame_interval)
         return lbm_run_frames(c->inner, steps, frame_interval);
     if (!c->initialized)
         return fail(LBM_ERR_STATE, "lbm_run_frames: call lbm_init_populations first");
-    if (!c->copy_stream)
+    if (hipError_t e = ensure_frames(c))
     {
-        LBM_HIP_TRY(hipStreamCreateWithFlags(&c->copy_stream, hipStreamNonBlocking));
-        LBM_HIP_TRY(hipEventCreateWithFlags(&c->ev_frame, hipEventDisableTiming));
-        for (hipEvent_t &e : c->ev_copied)
-            LBM_HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-        if (hipMalloc(&c->res_other, 4ull * std::max(1u, c->D) * sizeof(double)) != hipSuccess)
-        {
-            (void)hipGetLastError();
-            c->res_other = nullptr;  // frames then wait for each other's copies
-        }
-        LBM_HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&c->frame_host),
-                                  4ull * std::max(1u, c->D) * sizeof(double), hipHostMallocDefault));
+        (void)hipGetLastError();
+        return fail(e == hipErrorOutOfMemory ? LBM_ERR_OUT_OF_MEMORY : LBM_ERR_DEVICE,
+                    std::string("lbm_run_frames: the frame copies: ") + hipGetErrorString(e));
+    }
+    if (!c->res_other && hipMalloc(&c->res_other, 4ull * std::max(1u, c->D) * sizeof(double)) != hipSuccess)
+    {
+        (void)hipGetLastError();
+        c->res_other = nullptr;  // frames then wait for each other's copies
     }
     const VTable vt = vtable(c);
     uint64_t last_frame = ~0ull;
