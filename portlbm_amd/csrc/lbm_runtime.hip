@@ -112,7 +112,7 @@ struct lbm_ctx
     double *frame_host = nullptr;  // pinned, 4 * D
     // Frames write two result arrays in turn, so that the steps to the next
     // frame need not wait for the copy of the last one; c->res is the latest.
-    double *res_other = nullptr;   // allocated by the first lbm_run_frames; none if memory ran out
+    double *res_other = nullptr;   // allocated by the first run of two frames; none if memory ran out
     bool res_other_valid = false;  // its nodes that are not fluid hold what c->res holds
     int res_half = 0;              // which of the two c->res is
     bool copy_pending[2] = {false, false};  // a copy may still be reading it
@@ -2626,7 +2626,10 @@ int lbm_run_frames(lbm_ctx *c, uint32_t steps, uint32_t frame_interval)
         return fail(e == hipErrorOutOfMemory ? LBM_ERR_OUT_OF_MEMORY : LBM_ERR_DEVICE,
                     std::string("lbm_run_frames: the frame copies: ") + hipGetErrorString(e));
     }
-    if (!c->res_other && hipMalloc(&c->res_other, 4ull * std::max(1u, c->D) * sizeof(double)) != hipSuccess)
+    // Alone in a run, a frame has no steps after it to hold up.
+    const uint64_t frames =
+        frame_interval ? (c->iteration + steps) / frame_interval - c->iteration / frame_interval : 0u;
+    if (frames > 1u && !c->res_other && hipMalloc(&c->res_other, 4ull * std::max(1u, c->D) * sizeof(double)) != hipSuccess)
     {
         (void)hipGetLastError();
         c->res_other = nullptr;  // frames then wait for each other's copies

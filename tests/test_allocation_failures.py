@@ -32,3 +32,28 @@ for nth in range(1, {count} + 1):
     lat.close()
     assert live()[:2] == [0, 0] and live()[2] == 0, live()
 """)
+
+
+def test_a_second_result_array_only_for_several_frames(runtime):
+    """Two result arrays alternate so that steps need not wait for a copy: a
+    run without a frame, or with one, takes no second one."""
+    stand_in.run(runtime, """
+doc = pa.settings("lptl", "stream", inner_h=64, inner_v=32, time_steps=1)
+with pa.Lattice.from_settings(doc) as lat:
+    before = live()[0]
+    lat.run_frames(10, 0)
+    lat.run_frames(9, 100)
+    lat.run_frames(2, 10)
+    assert live()[0] == before
+    lat.run_frames(20, 10)
+    assert live()[0] == before + 4 * 64 * 32 * 8
+    assert lat.frame()[0] == 39
+assert live() == [0, 0, 0], live()
+# where it cannot be had, frames share one array
+with pa.Lattice.from_settings(doc) as lat:
+    before = live()[0]
+    log()
+    fail("hipMalloc", 1)
+    lat.run_frames(20, 5)
+    assert live()[0] == before and len([k for k in log() if "k_copy_frame" in k]) == 4
+""")
