@@ -333,11 +333,15 @@ int lbm_batch_last_run_ms(lbm_batch *b, double *ms);
 int lbm_batch_get_macros(lbm_batch *b, uint32_t domain, double *density, double *x_velocity, double *y_velocity,
                          double *absolute_velocity, size_t count);
 int lbm_batch_fluid_nodes(lbm_batch *b, uint64_t *count);
+/* Tile widths of the four width classes for launches of one step (per domain,
+ * and a persistent run's single steps) and for the residual sums; launches of
+ * several steps have their own partition. */
 int lbm_batch_set_tiles(lbm_batch *b, const uint32_t tile_width[4]);
 int lbm_batch_get_tiles(lbm_batch *b, uint32_t tile_width[4]);
-/* Times the persistent step for every candidate tile width of every width
- * class (coordinate descent, `steps_per_trial` steps each), keeps the fastest
- * and re-initialises the domains (trials advance the state). */
+/* Times the persistent launch of one step for every candidate tile width of
+ * every width class (coordinate descent, `steps_per_trial` launches each),
+ * keeps the fastest and re-initialises the domains (trials advance the state).
+ * best_ms_per_step: that launch's time. */
 int lbm_batch_autotune(lbm_batch *b, uint32_t steps_per_trial, double *best_ms_per_step);
 /* Per-domain steady-state residual ||j^now - j^snap||_2 / ||j^now||_2 over
  * fluid nodes (FP64), then j^snap := j^now; out holds one value per domain.

@@ -415,14 +415,14 @@ int build_parts(lbm_batch *b, int cus)
     return LBM_OK;
 }
 
-// `steps` steps of every domain, several per launch; *cur: the arena read
-// first and, afterwards, the one that holds the last step.
-int run_persistent_steps(lbm_batch *b, uint32_t steps, int *cur)
+// `steps` steps of every domain, several per launch as `plan` says; *cur: the
+// arena read first and, afterwards, the one that holds the last step.
+int run_persistent_steps(lbm_batch *b, uint32_t steps, int *cur, const FusePlan &plan)
 {
     const uint32_t grid = std::max(1u, std::min(b->ntiles, b->persistent_grid));
     for (uint32_t left = steps; left; *cur ^= 1)
     {
-        const uint32_t n = first_chunk(b->fuse, left);
+        const uint32_t n = first_chunk(plan, left);
         left -= n;
         if (n == 1u)
         {
@@ -441,8 +441,8 @@ int run_persistent_steps(lbm_batch *b, uint32_t steps, int *cur)
                            left == 0u ? 1u : 0u,
                            b->nan_protection ? 1u : 0u,
                            b->ones};
-        if (b->fuse.tiles)
-            batch_tile_launch(b->storage, n, b->fuse.steps - 1u, b->fuse.shape, a, b->nparts, b->stream);
+        if (plan.tiles)
+            batch_tile_launch(b->storage, n, plan.steps - 1u, plan.shape, a, b->nparts, b->stream);
         else
             batch_march_launch(b->storage, n, a, b->nparts, b->stream);
         BATCH_TRY(hipGetLastError());
@@ -664,16 +664,9 @@ int lbm_batch_init(lbm_batch *b)
     return LBM_OK;
 }
 
-int lbm_batch_run(lbm_batch *b, uint32_t steps, int32_t mode)
+// `plan`: the persistent launches' (graphs hold the batch's own)
+static int run_steps(lbm_batch *b, uint32_t steps, int32_t mode, const FusePlan &plan)
 {
-    if (!b)
-        return lbm_set_error(LBM_ERR_INVALID_ARGUMENT, "lbm_batch_run: null batch");
-    if (!b->initialized)
-        return lbm_set_error(LBM_ERR_STATE, "lbm_batch_run: call lbm_batch_init first");
-    if (mode < LBM_BATCH_PER_DOMAIN || mode > LBM_BATCH_GRAPH)
-        return lbm_set_error(LBM_ERR_INVALID_ARGUMENT, "lbm_batch_run: unknown mode");
-    if (steps == 0)
-        return LBM_OK;
     const int parity0 = b->cur;
     if (mode == LBM_BATCH_GRAPH && (b->graph_steps != steps || b->graph_parity != parity0))
     {
@@ -682,7 +675,7 @@ int lbm_batch_run(lbm_batch *b, uint32_t steps, int32_t mode)
         hipGraph_t g = nullptr;
         BATCH_TRY(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
         b->graph_end = parity0;
-        int rc = run_persistent_steps(b, steps, &b->graph_end);
+        int rc = run_persistent_steps(b, steps, &b->graph_end, b->fuse);
         hipError_t e = hipStreamEndCapture(b->stream, &g);
         if (rc)
             return rc;
@@ -704,7 +697,7 @@ int lbm_batch_run(lbm_batch *b, uint32_t steps, int32_t mode)
     }
     else if (mode == LBM_BATCH_PERSISTENT)
     {
-        if (int rc = run_persistent_steps(b, steps, &end))
+        if (int rc = run_persistent_steps(b, steps, &end, plan))
             return rc;
     }
     else
@@ -723,6 +716,19 @@ int lbm_batch_run(lbm_batch *b, uint32_t steps, int32_t mode)
     b->last_ms = ms;
     b->cur = end;
     return LBM_OK;
+}
+
+int lbm_batch_run(lbm_batch *b, uint32_t steps, int32_t mode)
+{
+    if (!b)
+        return lbm_set_error(LBM_ERR_INVALID_ARGUMENT, "lbm_batch_run: null batch");
+    if (!b->initialized)
+        return lbm_set_error(LBM_ERR_STATE, "lbm_batch_run: call lbm_batch_init first");
+    if (mode < LBM_BATCH_PER_DOMAIN || mode > LBM_BATCH_GRAPH)
+        return lbm_set_error(LBM_ERR_INVALID_ARGUMENT, "lbm_batch_run: unknown mode");
+    if (steps == 0)
+        return LBM_OK;
+    return run_steps(b, steps, mode, b->fuse);
 }
 
 int lbm_batch_last_run_ms(lbm_batch *b, double *ms)
@@ -788,6 +794,7 @@ int lbm_batch_autotune(lbm_batch *b, uint32_t steps_per_trial, double *best_ms_p
     bool present[4] = {false, false, false, false};
     for (const BatchDom &dm : b->doms)
         present[width_class(dm.H - 2)] = true;
+    const FusePlan single;  // the launches of several steps do not use the tiles
     double best = 1e300;
     for (int c = 0; c < 4; ++c)
     {
@@ -801,9 +808,9 @@ int lbm_batch_autotune(lbm_batch *b, uint32_t steps_per_trial, double *best_ms_p
             widths[c] = w;
             if (int rc = lbm_batch_set_tiles(b, widths))
                 return rc;
-            if (int rc = lbm_batch_run(b, 2, LBM_BATCH_PERSISTENT))  // warm-up
+            if (int rc = run_steps(b, 2, LBM_BATCH_PERSISTENT, single))  // warm-up
                 return rc;
-            if (int rc = lbm_batch_run(b, steps_per_trial, LBM_BATCH_PERSISTENT))
+            if (int rc = run_steps(b, steps_per_trial, LBM_BATCH_PERSISTENT, single))
                 return rc;
             const double per_step = b->last_ms / steps_per_trial;
             if (per_step < best)
