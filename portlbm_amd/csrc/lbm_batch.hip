@@ -524,7 +524,6 @@ void lbm_batch_destroy(lbm_batch *b)
     if (b->stream)
         (void)hipStreamDestroy(b->stream);
     delete b;
-    release_staging();
 }
 
 int lbm_batch_create(const lbm_batch_domain *domains, uint32_t count, int32_t storage, int32_t nan_protection,
@@ -536,7 +535,6 @@ int lbm_batch_create(const lbm_batch_domain *domains, uint32_t count, int32_t st
         return lbm_set_error(LBM_ERR_INVALID_ARGUMENT, "lbm_batch_create: unknown storage type");
     *out = nullptr;
     lbm_batch *b = new lbm_batch();
-    hold_staging();
     b->storage = storage;
     b->nan_protection = nan_protection;
     b->elem = store_bytes(storage);

@@ -2209,7 +2209,6 @@ void lbm_destroy(lbm_ctx *c)
     if (c->stream)
         (void)hipStreamDestroy(c->stream);
     delete c;
-    release_staging();
 }
 
 int lbm_create(const lbm_desc *desc, lbm_ctx **out)
@@ -2220,7 +2219,6 @@ int lbm_create(const lbm_desc *desc, lbm_ctx **out)
     if (int rc = validate_desc(desc))
         return rc;
     lbm_ctx *c = new lbm_ctx();
-    hold_staging();
     c->desc = *desc;
     c->H = desc->horizontal_nodes;
     c->V = desc->vertical_nodes;

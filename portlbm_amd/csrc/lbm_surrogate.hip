@@ -927,7 +927,6 @@ void lbm_surrogate_destroy(lbm_surrogate *s)
     if (s->stream)
         (void)hipStreamDestroy(s->stream);
     delete s;
-    lbm_dev::release_staging();
 }
 
 int lbm_surrogate_create(uint32_t height, uint32_t width, uint32_t max_batch, lbm_surrogate **out)
@@ -941,7 +940,6 @@ int lbm_surrogate_create(uint32_t height, uint32_t width, uint32_t max_batch, lb
                              "lbm_surrogate_create: height and width must be positive multiples of 16 (<= 8192), "
                              "max_batch in 1..4096");
     auto *s = new lbm_surrogate;
-    lbm_dev::hold_staging();
     s->H = int(height);
     s->W = int(width);
     s->Bmax = int(max_batch);

@@ -16,12 +16,8 @@ struct HostPiece
 };
 
 // Copies the pieces once the work enqueued on `stream` is done; returns when
-// they have arrived.  Any thread, any stream.
+// they have arrived.  Any thread, any stream.  Its pinned staging, at most 16
+// MiB, is kept for the process.
 hipError_t download(const HostPiece *pieces, size_t count, hipStream_t stream);
-
-// The objects that may call download() (contexts, batches, networks) hold its
-// staging memory between them: it is given back with the last of them.
-void hold_staging();
-void release_staging();
 
 }  // namespace lbm_dev
