@@ -356,10 +356,10 @@ int step_dispatch(lbm_batch *b, int parity, bool macros, const BatchTile *tiles,
 // or a block's first node.
 int build_parts(lbm_batch *b, int cus)
 {
-    uint64_t nodes = 0;
+    std::vector<FuseExtent> extents;
     for (const BatchDom &dm : b->doms)
-        nodes += dm.D;
-    b->fuse = plan_fusion(b->elem, nodes);
+        extents.push_back(FuseExtent{dm.H - 2u, dm.V - 2u});
+    b->fuse = plan_fusion(b->elem, LBM_LAYOUT_STREAM, extents.data(), extents.size());
     std::vector<BatchPart> parts;
     if (b->fuse.tiles)
     {

@@ -33,6 +33,7 @@
 #include "lbm_march.hpp"
 
 #include <algorithm>
+#include <iterator>
 #include <utility>
 
 namespace lbm_dev
@@ -714,6 +715,80 @@ __global__ __launch_bounds__(MARCH_BLOCK, 2) void k_batch_march(BatchFused a, ui
     const StepParams p = batch_params<S>(a, part.dom);
     constexpr uint32_t sr[kFusedMaxSteps] = {};
     march_wave<LBM_LAYOUT_STREAM, S, T>(p, sr, part.x, int(part.y0), int(part.y1), lds[0]);
+}
+
+// What of the columns that marching waves own, or of the nodes that blocks
+// own, lies in the domains.
+static double march_share(size_t elem, const FuseExtent *domains, size_t count)
+{
+    const uint32_t own = uint32_t(MARCH_OWN) * uint32_t(8u / elem);
+    double in = 0.0, all = 0.0;
+    for (size_t d = 0; d < count; ++d)
+    {
+        in += double(domains[d].w) * domains[d].h;
+        all += double((domains[d].w + own - 1u) / own * own) * domains[d].h;
+    }
+    return in / all;
+}
+static double tile_share(uint32_t w, uint32_t h, uint32_t steps, const FuseExtent *domains, size_t count)
+{
+    const uint32_t ow = w - 2u * (steps - 1u), oh = h - 2u * (steps - 1u);
+    double in = 0.0, all = 0.0;
+    for (size_t d = 0; d < count; ++d)
+    {
+        in += double(domains[d].w) * domains[d].h;
+        all += double((domains[d].w + ow - 1u) / ow * ow) * double((domains[d].h + oh - 1u) / oh * oh);
+    }
+    return in / all;
+}
+
+FusePlan plan_fusion(size_t elem, int layout, const FuseExtent *domains, size_t count)
+{
+    const FusePlan march{kMarchMaxSteps, false, TileShape::k32x32}, one{};
+    uint64_t nodes = 0;
+    for (size_t d = 0; d < count; ++d)
+        nodes += uint64_t(domains[d].w) * domains[d].h;
+    if (count == 1u && domains->h <= 4u && layout == LBM_LAYOUT_STREAM && nodes >= 100000u)
+        return one;
+    if (count == 1u && (domains->h <= 10u ? nodes > 36000u : domains->h <= 12u && nodes >= 300000u))
+        return FusePlan{domains->h <= 10u ? 4u : 3u, true, TileShape::k32x16};
+    // 16-bit tiles and how much of them is used
+    struct
+    {
+        FusePlan plan;
+        double share;
+    } tiles[3] = {{{3u, true, TileShape::k32x16}, tile_share(32, 16, 3, domains, count)},
+                  {{4u, true, TileShape::k32x16}, tile_share(32, 16, 4, domains, count) / 1.15},
+                  {{5u, true, TileShape::k32x32}, tile_share(32, 32, 5, domains, count) / 1.04}};
+    const auto &fit = *std::max_element(std::begin(tiles), std::end(tiles),
+                                        [](const auto &a, const auto &b) { return a.share < b.share; });
+    // whether the stream layout's one-step kernel has full blocks of 256 columns
+    const bool full = count == 1u && layout == LBM_LAYOUT_STREAM &&
+                      domains->w >= 0.85 * ((domains->w + 255u) / 256u * 256u);
+    if (nodes >= (elem == 8 ? 1500000u : (elem == 4 ? 2500000u : 3500000u)))
+    {
+        const double share = march_share(elem, domains, count);
+        if (elem >= 4)
+        {
+            if (share >= 0.5)
+                return march;
+        }
+        else
+        {
+            const double marched = share >= 0.6 ? 5.7 / share + 8e6 / double(nodes) : 1e3, tiled = 9.9 / fit.share;
+            if (full && 8.2 < 0.95 * std::min(marched, tiled))
+                return one;
+            if (marched <= tiled)
+                return march;
+        }
+    }
+    if (nodes <= 36000u)
+        return FusePlan{5u, true, TileShape::k16x16};
+    if (nodes <= (elem == 8 ? 300000u : 500000u))
+        return FusePlan{nodes <= 200000u ? 6u : 5u, true, TileShape::k32x32};
+    if (elem >= 4)
+        return FusePlan{elem == 8 ? 4u : 3u, true, TileShape::k32x16};
+    return full && fit.share < 0.6 ? one : fit.plan;
 }
 
 uint32_t march_strips(int storage, uint32_t inner_width)

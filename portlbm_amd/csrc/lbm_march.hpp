@@ -43,26 +43,51 @@ struct FusePlan
 //   1024 x 256   10.2 / 6.1 / 6.3    32x32 T 5: 4.69 / 3.73 / 3.65    32x16 T 4: 4.38 / 3.82 / 3.90
 //   2048 x 512   29.5 / 16.1 / 16.3  32x16 T 4: 12.6 / 10.7 / 11.1    march:     14.6 / 13.0 / 20.3
 //   4096 x 1024  112 / 55.8 / 48.9   32x16 T 4: 59.0 / 42.9 / 38.7    march:     45.4 / 32.7 / 37.5
-// and at the lines between the shapes (bundle layout, FP64 / FP32 / BF16;
+// and at the lines between the shapes (FP64 / FP32 / BF16, bundle layout;
 // "1.8e5": inner nodes):
 //   1.8e5  32x32 T 6: 3.77 / 3.18 / 3.27   T 5: 4.06 / 3.38 / 3.42
 //   2.6e5  32x32 T 6: 5.06 / 4.20 / 4.16   T 5: 4.52 / 3.59 / 3.74
 //   3.9e5  32x32 T 5: 6.39 / 4.96 / 5.00   32x16 T 4: 5.81 / 4.98 / 5.12 (FP64 collision 7.12, 6.90)
-//   1.0e6  32x16 T 3: 11.7 / 10.1 / 10.4   32x16 T 4: 12.2 / 10.7 / 11.1   march: 14.8 / 13.9 / 18.0
-//   2.0e6  32x16 T 3: 23.2 / 18.5 / 19.1   32x16 T 4: 22.9 / 19.8 / 20.5   march: 24.8 / 19.8 / 24.1
-//   3.0e6  32x16 T 3: 39.0 / 27.2 / 28.0   march: 35.1 / 27.2 / 27.5 (3001 x 997 for nsol, FP32: 31.0, 28.4)
-// FP64 marches from 1.5e6: at 2.0e6 the collision layout takes 24.7 marched
-// and 27.3 in tiles.
-inline FusePlan plan_fusion(size_t elem, uint64_t nodes)
+//   1.05e6 32x16 T 3: 14.7 / 11.5 / 11.6   32x16 T 4: 13.7 / 11.6 / 11.9 (FP64 collision 22.0, 18.7)
+//   1.5e6  32x16 T 3: 19.3 / 15.3 / 15.4   32x16 T 4: 19.0 / 16.2 / 16.4   march: 20.8 / 16.9 / 21.2
+// (FP64 collision at 1.5e6: 29.6, 25.8, march 20.9).  March against the better
+// of T 3 and T 4 (stream, collision, bundle):
+//   FP64   2.0e6  25.4 25.5 25.4 : 29.3 34.8 27.7     3.0e6  33.8 35.7 35.5 : 39.4 51.7 40.1
+//   FP32   2.25e6 21.7 23.3 23.2 : 21.1 27.0 23.1     2.5e6  23.6 24.9 24.9 : 23.4 29.7 24.6
+//          2.75e6 24.7 26.4 25.8 : 26.0 32.5 27.1     3.0e6  26.4 28.1 27.8 : 28.1 35.4 30.0
+//   FP16   2.5e6  23.3 24.7 24.2 : 20.9 24.8 23.7     3.0e6  24.5 25.9 25.9 : 25.0 29.2 28.6
+//          3.5e6  26.8 29.1 28.8 : 29.0 33.3 32.8     4.2e6  32.4 34.0 33.7 : 34.3 39.9 38.0
+//
+// All of that is for lattices of some width and height.  A marching wave owns
+// 56, 112 or 224 columns (FP64, FP32, 16-bit), a block 22 to 28 columns by 10
+// to 26 rows, and what of them lies past the lattice is work for nothing:
+// * FP64 and FP32 march where the lattice takes at least half of the waves'
+//   columns (1.9e6 nodes 64 wide, 0.57: FP64 36.4, tiles 38.0, FP32 at 3.8e6
+//   55.5, 56.8; batches of 16 x 16 domains, 0.14 in FP32).
+// * 16-bit lattices compare the us that 1e6 nodes take: marching, 5.7 over the
+//   share of the columns and 8 / nodes for a launch's ramp, never below a share
+//   of 0.6; tiles, 9.9 over the share of the regions; in the stream layout also
+//   one step per launch, 8.2 where the columns fill that kernel's blocks of 256
+//   to 0.85 (up to 11 where they do not).  58 x 65000: march 94.6, 32x32 T 5
+//   47.7, 32x16 T 3 55.0, one step 58.7; 226 x 65000: 169, 145, 161, 124; 450 x
+//   65000: 264, 269, 286, 228; 280 x 65000: 167, 173, 170, 195; 976 domains of
+//   64 x 64: 90.2, 48.0, 53.6, 94.4.  Their tiles are 32x16 with T 3 unless T
+//   4's rows (65000 x 26: 17.4 : 18.6) or 32x32's columns (113 x 30000: 34.1 :
+//   38.6) fit clearly better; where no shape has a share of 0.6 the stream
+//   layout takes one step per launch (65000 x 13: 9.6, T 4 11.5, T 3 11.7).
+// * Lattices of at most 10 rows take 32x16 tiles with T 4 (10 own rows), of 11
+//   or 12 with T 3: 65000 x 6 5.6 / 5.1 / 5.5 us in the stream layout, with the
+//   shape for 3.9e5 nodes otherwise 5.7 / 9.4 / 8.9; 40000 x 11 6.3 / 5.3 / 5.5
+//   against 7.9 / 6.9 / 7.2.
+//   One or two rows between walls in the stream layout leave a step nothing to
+//   share: one step per launch (65000 x 3: 3.7 / 3.2 / 3.8, T 4 5.1 / 4.7 / 4.8).
+struct FuseExtent
 {
-    if (nodes >= (elem == 8 ? 1500000u : (elem == 4 ? 2500000u : 3500000u)))
-        return FusePlan{kMarchMaxSteps, false, TileShape::k32x32};
-    if (nodes <= 36000u)
-        return FusePlan{5u, true, TileShape::k16x16};
-    if (nodes <= (elem == 8 ? 300000u : 500000u))
-        return FusePlan{nodes <= 200000u ? 6u : 5u, true, TileShape::k32x32};
-    return FusePlan{elem == 8 ? 4u : 3u, true, TileShape::k32x16};
-}
+    uint32_t w, h;  // inner columns and rows
+};
+
+// The plan for one lattice, or for the domains of a batch together.
+FusePlan plan_fusion(size_t elem, int layout, const FuseExtent *domains, size_t count);
 
 // The first launch of n steps: as few launches as there can be, of nearly the same length.
 inline uint32_t first_chunk(const FusePlan &plan, uint32_t n)

@@ -2372,7 +2372,10 @@ int lbm_create(const lbm_desc *desc, lbm_ctx **out)
     }
     c->cus = cus;
     if (c->two_lattice)
-        c->fuse = plan_fusion(c->elem, uint64_t(c->Hx - 2u) * (c->Vx - 2u));
+    {
+        const FuseExtent extent{c->Hx - 2u, c->Vx - 2u};
+        c->fuse = plan_fusion(c->elem, desc->layout, &extent, 1u);
+    }
     CREATE_TRY(hipMalloc(&c->lat[0], lat_bytes + std::max<size_t>(64, side_bytes)));
     if (c->two_lattice)
         CREATE_TRY(hipMalloc(&c->lat[1], lat_bytes + 64));
