@@ -90,9 +90,8 @@ enum lbm_rounding { LBM_ROUND_NEAREST = 0, LBM_ROUND_STOCHASTIC = 1 };
 /* Step kernels of npol/nsol.
  * Auto, first choice: round-to-nearest lattices whose second copy takes at
  * most 1/64 of the device's memory, and gets it, run the unexpanded lattice
- * through lptl's kernels, several steps per launch; lbm_get_populations then
- * returns the rest state at buffer nodes.  Everything else works in place on
- * one lattice, by one of the kernels below.
+ * through lptl's kernels, several steps per launch.  Everything else works in
+ * place on one lattice, by one of the kernels below.
  * The in-place kernels of lattices whose tiles are at most 64 nodes wide.
  * Sweep: one wave walks each tile, the tile-edge copies in side arrays (no
  * refresh launches); block: one work-group per tile with the reference's
@@ -248,10 +247,13 @@ int lbm_get_frame(lbm_ctx *ctx, double *density, double *x_velocity, double *y_v
  * (freed by lbm_destroy).  Fluid and ghost nodes
  * are current.  Solid nodes' populations are never read (half-way
  * bounce-back takes the fluid node's own), and the fused kernels leave them
- * zero or as they were.  npol/nsol with tiles at most 64 nodes wide keep
- * the buffer copies of a step outside the lattice, so the lattice's buffer
- * rows/columns hold what they held when last refreshed (a split step
- * refreshes them). */
+ * zero or as they were.  npol/nsol on the unexpanded lattice, and in place
+ * with tiles at most 64 nodes wide, keep the buffer copies of a step outside
+ * the lattice, so the lattice's buffer rows/columns hold what they were last
+ * set to (lbm_set_populations, lbm_set_state; the rest state before; in place
+ * a split step refreshes them).  On the unexpanded lattice the first call that
+ * sets them takes a second, expanded one to keep them in, until
+ * lbm_init_populations; where there is no memory for it they stay at rest. */
 int lbm_get_populations(lbm_ctx *ctx, double *values, size_t count);
 int lbm_set_populations(lbm_ctx *ctx, const double *values, size_t count);
 

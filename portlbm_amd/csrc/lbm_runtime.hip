@@ -126,7 +126,9 @@ struct lbm_ctx
     double feq_in[9], feq_out[9];
     // npol / nsol that need not stay in place (see plan_compact): the work is
     // done by this context on the unexpanded lattice; the outer one converts
-    // what callers hand over and receive in the expanded order.
+    // what callers hand over and receive in the expanded order.  Its own lat[0]
+    // holds what its buffer nodes were set to, from the first time that a
+    // caller sets them (ensure_expanded).
     lbm_ctx *inner = nullptr;
     std::vector<int8_t> outer_phase;  // the expanded node types, as set
     // 16-bit forms: rho_ref per unexpanded column (Hx + 64 floats, the tail
@@ -2454,6 +2456,8 @@ int lbm_get_phase(lbm_ctx *c, int8_t *phase, size_t n)
 
 // The 16-bit forms' initial rho_ref table: the rest state's 1, the ghost
 // columns at rho_in and rho_out.
+static void drop_expanded(lbm_ctx *c);
+
 static int reset_reference(lbm_ctx *c)
 {
     c->ref_cur = 0;
@@ -2472,7 +2476,10 @@ int lbm_init_populations(lbm_ctx *c)
     if (!c)
         return fail(LBM_ERR_INVALID_ARGUMENT, "lbm_init_populations: null context");
     if (c->inner)
+    {
+        drop_expanded(c);
         return lbm_init_populations(c->inner);
+    }
     if (!c->phase_set)
         return fail(LBM_ERR_STATE, "lbm_init_populations: lbm_set_phase must come first");
     c->cur = 0;
@@ -2893,6 +2900,106 @@ static int set_state_tail(lbm_ctx *c, const char *in, uint32_t ref_len, uint64_t
     return LBM_OK;
 }
 
+// The population accessors convert between the storage and FP64 through a
+// staging buffer of at most kStageDoubles that the context keeps after the
+// first call, one chunk at a time.
+constexpr uint32_t kStageDoubles = 1u << 22;  // 32 MiB
+
+static int ensure_stage(lbm_ctx *c)
+{
+    if (!c->stage)
+        LBM_HIP_TRY(hipMalloc(&c->stage, size_t(std::min(kStageDoubles, 9u * c->N)) * sizeof(double)));
+    return LBM_OK;
+}
+
+// All 9 N populations of c's own lattice, to or from the host.
+static int read_populations(lbm_ctx *c, double *values)
+{
+    if (int rc = ensure_stage(c))
+        return rc;
+    const VTable vt = vtable(c);
+    const size_t count = 9ull * c->N;
+    for (uint32_t i0 = 0; i0 < count; i0 += kStageDoubles)
+    {
+        const uint32_t n = uint32_t(std::min<size_t>(kStageDoubles, count - i0));
+        if (int rc = vt.decode(c, c->stage, i0, n))
+            return rc;
+        const HostPiece piece{values + i0, c->stage, n * sizeof(double)};
+        LBM_HIP_TRY(download(&piece, 1, c->stream));  // the next chunk reuses the staging buffer
+    }
+    return LBM_OK;
+}
+
+static int write_populations(lbm_ctx *c, const double *values)
+{
+    if (int rc = ensure_stage(c))
+        return rc;
+    const VTable vt = vtable(c);
+    const size_t count = 9ull * c->N;
+    for (uint32_t i0 = 0; i0 < count; i0 += kStageDoubles)
+    {
+        const uint32_t n = uint32_t(std::min<size_t>(kStageDoubles, count - i0));
+        LBM_HIP_TRY(hipMemcpyAsync(c->stage, values + i0, n * sizeof(double), hipMemcpyHostToDevice, c->stream));
+        if (int rc = vt.encode(c, c->stage, i0, n))
+            return rc;
+        LBM_HIP_TRY(hipStreamSynchronize(c->stream));
+    }
+    return LBM_OK;
+}
+
+// The expanded lattice of a context that works on an inner one, for its buffer
+// nodes: at rest when it is made.  False where there is no memory for it.
+static void drop_expanded(lbm_ctx *c)
+{
+    if (c->stream)
+        (void)hipStreamSynchronize(c->stream);
+    (void)hipFree(c->lat[0]);
+    (void)hipFree(c->ref[0]);
+    (void)hipFree(c->stage);
+    c->lat[0] = nullptr;
+    c->ref[0] = nullptr;
+    c->stage = nullptr;
+}
+
+static bool ensure_expanded(lbm_ctx *c)
+{
+    if (c->lat[0])
+        return true;
+    auto made = [&]() -> int {
+        if (!c->stream)
+            LBM_HIP_TRY(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
+        LBM_HIP_TRY(hipMalloc(&c->lat[0], c->lattice_elems * c->elem + 64));
+        if (c->ref_len)
+            LBM_HIP_TRY(hipMalloc(&c->ref[0], c->ref_len * sizeof(float)));
+        if (int rc = reset_reference(c))
+            return rc;
+        if (int rc = vtable(c).init(c))
+            return rc;
+        LBM_HIP_TRY(hipStreamSynchronize(c->stream));
+        return ensure_stage(c);
+    };
+    if (made() == LBM_OK)
+        return true;
+    (void)hipGetLastError();
+    drop_expanded(c);
+    return false;
+}
+
+// The same before the lattice is set: at the inner one's column reference.
+// Where this fails the buffer nodes, which no step reads, stay at rest.
+static bool expanded_to_set(lbm_ctx *c)
+{
+    if (!ensure_expanded(c))
+        return false;
+    const lbm_ctx *in = c->inner;
+    if (!c->ref[0] || hipMemcpy(c->ref[0], in->ref[in->ref_cur], std::min(c->ref_len, in->ref_len) * sizeof(float),
+                                hipMemcpyDeviceToDevice) == hipSuccess)
+        return true;
+    (void)hipGetLastError();
+    drop_expanded(c);
+    return false;
+}
+
 static int get_inner_state(lbm_ctx *c, char *out)
 {
     lbm_ctx *in = c->inner;
@@ -2901,8 +3008,14 @@ static int get_inner_state(lbm_ctx *c, char *out)
     std::memcpy(out + 8, &cur, 4);
     std::memcpy(out + 12, &lattices, 4);
     const size_t lat_bytes = c->lattice_elems * c->elem;
-    std::memset(out + 16, 0, lat_bytes);
+    const bool kept = c->lat[0];
     std::vector<char> own(in->lattice_elems * in->elem);
+    if (ensure_expanded(c))
+        LBM_HIP_TRY(hipMemcpy(out + 16, c->lat[0], lat_bytes, hipMemcpyDeviceToHost));
+    else
+        std::memset(out + 16, 0, lat_bytes);
+    if (!kept)
+        drop_expanded(c);
     LBM_HIP_TRY(hipStreamSynchronize(in->stream));
     LBM_HIP_TRY(hipMemcpy(own.data(), in->lat[in->cur], own.size(), hipMemcpyDeviceToHost));
     for_placed_runs(c, [&](size_t o, size_t x, size_t n) { std::memcpy(out + 16 + x, own.data() + o, n); });
@@ -2918,7 +3031,11 @@ static int set_inner_state(lbm_ctx *c, const char *buf, uint64_t iteration)
     for_placed_runs(c, [&](size_t o, size_t x, size_t n) { std::memcpy(own.data() + o, buf + 16 + x, n); });
     for (void *lat : in->lat)
         LBM_HIP_TRY(hipMemcpy(lat, own.data(), own.size(), hipMemcpyHostToDevice));
-    return set_state_tail(in, buf + 16 + c->lattice_elems * c->elem, c->ref_len, iteration, 0);
+    if (int rc = set_state_tail(in, buf + 16 + c->lattice_elems * c->elem, c->ref_len, iteration, 0))
+        return rc;
+    if (expanded_to_set(c))
+        LBM_HIP_TRY(hipMemcpy(c->lat[0], buf + 16, c->lattice_elems * c->elem, hipMemcpyHostToDevice));
+    return LBM_OK;
 }
 
 int lbm_get_state(lbm_ctx *c, void *buf, size_t bytes)
@@ -2975,18 +3092,6 @@ int lbm_set_state(lbm_ctx *c, const void *buf, size_t bytes)
     return set_state_tail(c, in + off, c->ref_len, iteration, int(cur));
 }
 
-// The population accessors convert between the storage and FP64 through a
-// staging buffer of at most kStageDoubles that the context keeps after the
-// first call, one chunk at a time.
-constexpr uint32_t kStageDoubles = 1u << 22;  // 32 MiB
-
-static int ensure_stage(lbm_ctx *c)
-{
-    if (!c->stage)
-        LBM_HIP_TRY(hipMalloc(&c->stage, size_t(std::min(kStageDoubles, 9u * c->N)) * sizeof(double)));
-    return LBM_OK;
-}
-
 int lbm_get_populations(lbm_ctx *c, double *values, size_t count)
 {
     if (!c || !values)
@@ -3000,13 +3105,24 @@ int lbm_get_populations(lbm_ctx *c, double *values, size_t count)
             std::vector<double> own(9 * M);
             if (int rc = lbm_get_populations(c->inner, own.data(), own.size()))
                 return rc;
-            // buffer nodes are not kept: the rest state, as after lbm_init_populations
-            static const double w[9] = {1.0 / 36, 1.0 / 9, 1.0 / 36, 1.0 / 9, 4.0 / 9,
-                                        1.0 / 9,  1.0 / 36, 1.0 / 9, 1.0 / 36};
             const int layout = c->desc.layout;
-            for (uint32_t d = 0; d < 9; ++d)
-                for (size_t e = 0; e < c->N; ++e)
-                    values[flat_index(layout, e, d, c->N)] = w[d];
+            const bool kept = c->lat[0];
+            if (ensure_expanded(c))
+            {
+                const int rc = read_populations(c, values);
+                if (!kept)
+                    drop_expanded(c);
+                if (rc)
+                    return rc;
+            }
+            else
+            {
+                static const double w[9] = {1.0 / 36, 1.0 / 9, 1.0 / 36, 1.0 / 9, 4.0 / 9,
+                                            1.0 / 9,  1.0 / 36, 1.0 / 9, 1.0 / 36};
+                for (uint32_t d = 0; d < 9; ++d)
+                    for (size_t e = 0; e < c->N; ++e)
+                        values[flat_index(layout, e, d, c->N)] = w[d];
+            }
             for (uint32_t d = 0; d < 9; ++d)
                 for_runs(c, [&](size_t u, size_t e, size_t k) {
                     for (size_t i = 0; i < k; ++i)
@@ -3015,18 +3131,7 @@ int lbm_get_populations(lbm_ctx *c, double *values, size_t count)
             return LBM_OK;
         });
     }
-    if (int rc = ensure_stage(c))
-        return rc;
-    const VTable vt = vtable(c);
-    for (uint32_t i0 = 0; i0 < count; i0 += kStageDoubles)
-    {
-        const uint32_t n = uint32_t(std::min<size_t>(kStageDoubles, count - i0));
-        if (int rc = vt.decode(c, c->stage, i0, n))
-            return rc;
-        const HostPiece piece{values + i0, c->stage, n * sizeof(double)};
-        LBM_HIP_TRY(download(&piece, 1, c->stream));  // the next chunk reuses the staging buffer
-    }
-    return LBM_OK;
+    return read_populations(c, values);
 }
 
 int lbm_set_populations(lbm_ctx *c, const double *values, size_t count)
@@ -3048,25 +3153,18 @@ int lbm_set_populations(lbm_ctx *c, const double *values, size_t count)
                     for (size_t i = 0; i < k; ++i)
                         own[flat_index(layout, u + i, d, M)] = values[flat_index(layout, e + i, d, c->N)];
                 });
-            return lbm_set_populations(c->inner, own.data(), own.size());
+            if (int rc = lbm_set_populations(c->inner, own.data(), own.size()))
+                return rc;
+            return expanded_to_set(c) ? write_populations(c, values) : LBM_OK;
         });
     }
     if (!c->initialized)
         return fail(LBM_ERR_STATE, "lbm_set_populations: call lbm_init_populations first");
     if (count != 9ull * c->N)
         return fail(LBM_ERR_INVALID_ARGUMENT, "lbm_set_populations: count must be 9 * expanded node count");
-    if (int rc = ensure_stage(c))
-        return rc;
     c->side_valid = false;
-    const VTable vt = vtable(c);
-    for (uint32_t i0 = 0; i0 < count; i0 += kStageDoubles)
-    {
-        const uint32_t n = uint32_t(std::min<size_t>(kStageDoubles, count - i0));
-        LBM_HIP_TRY(hipMemcpyAsync(c->stage, values + i0, n * sizeof(double), hipMemcpyHostToDevice, c->stream));
-        if (int rc = vt.encode(c, c->stage, i0, n))
-            return rc;
-        LBM_HIP_TRY(hipStreamSynchronize(c->stream));
-    }
+    if (int rc = write_populations(c, values))
+        return rc;
     if (c->two_lattice)
         LBM_HIP_TRY(hipMemcpyAsync(c->lat[1 - c->cur], c->lat[c->cur], c->lattice_elems * c->elem,
                                    hipMemcpyDeviceToDevice, c->stream));

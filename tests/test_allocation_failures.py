@@ -57,3 +57,28 @@ with pa.Lattice.from_settings(doc) as lat:
     lat.run_frames(20, 5)
     assert live()[0] == before and len([k for k in log() if "k_copy_frame" in k]) == 4
 """)
+
+
+@pytest.mark.parametrize("storage", ["f64", "f16-shifted"])
+def test_buffer_nodes_without_memory(runtime, storage):
+    """Where the expanded lattice cannot be had, setting populations or a state
+    succeeds and the buffer nodes stay at rest."""
+    stand_in.run(runtime, f"""
+doc = pa.settings("npol", "stream", inner_h=65, inner_v=40, storage={storage!r}, time_steps=1)
+with pa.Lattice.from_settings(doc) as lat:
+    values, state = lat.populations(), lat.state()
+    before = live()
+    for call in (lambda: lat.set_populations(values), lambda: lat.set_state(state), lat.state, lat.populations):
+        for nth in (1, 2, 3):
+            lat.init()
+            fail("hipMalloc", nth)
+            call()
+            fail("hipMalloc", 0)
+    lat.init()
+    assert live() == before, (before, live())
+    lat.set_populations(values)
+    assert live()[0] > before[0]
+    extra = live()[0] - before[0]
+    assert extra >= 9 * lat.N * {8 if storage == "f64" else 2}
+assert live()[0] == 0, live()
+""")

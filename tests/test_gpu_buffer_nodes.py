@@ -1,0 +1,66 @@
+"""Buffer rows and columns of npol and nsol, which no step reads: under the
+automatic tile kernel, which works on the unexpanded lattice, they hold what
+they hold under the in-place sweep -- the rest state, or what a caller last
+set them to, at the storage's precision."""
+import numpy as np
+import pytest
+
+import portlbm_amd as pa
+from test_gpu_one_lattice import document
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("storage", ["f64", "f32", "f16-shifted", "bf16-shifted"])
+@pytest.mark.parametrize("layout", ["collision", "stream", "bundle"])
+@pytest.mark.parametrize("algorithm", ["npol", "nsol"])
+def test_buffer_nodes_hold_what_they_were_set_to(algorithm, layout, storage):
+    docs = [document(algorithm, layout, storage, 131, 77, 64, kernel) for kernel in ("auto", "sweep")]
+    phase = pa.build_phase(docs[0])
+    auto, place = (pa.Lattice(pa.desc_from_settings(doc), phase) for doc in docs)
+    N = auto.N
+    n, d = np.nonzero(phase != 1)[0].astype(np.int64), np.arange(9)[:, None]  # solid populations are never read
+    slots = (9 * n + d if layout == "collision" else N * d + n if layout == "stream"
+             else 3 * (d // 3) * N + d % 3 + 3 * n).ravel()
+
+    def same():
+        np.testing.assert_array_equal(auto.populations()[slots], place.populations()[slots])
+
+    with auto, place:
+        same()
+        rest = auto.populations()
+        values = rest * np.random.default_rng(3).uniform(0.99, 1.01, rest.size)
+        for lattice in (auto, place):
+            lattice.set_populations(values)
+        same()
+        for lattice in (auto, place):
+            lattice.run(7)
+        same()
+        auto.set_state(place.state())
+        same()
+        place.set_state(auto.state())
+        for lattice in (auto, place):
+            lattice.run(5)
+        same()
+        for lattice in (auto, place):
+            lattice.init()
+        same()
+        np.testing.assert_array_equal(auto.populations()[slots], rest[slots])
+
+
+@pytest.mark.parametrize("layout", ["collision", "stream", "bundle"])
+@pytest.mark.parametrize("storage", ["f16-shifted", "bf16-shifted"])
+@pytest.mark.parametrize("algorithm", ["npol", "nsol"])
+def test_fields_past_the_changes_of_the_column_reference(algorithm, storage, layout):
+    """16-bit storage changes its column reference at steps 128 and 256."""
+    for shape in ((131, 77, 64), (300, 100, 1024)):
+        lattices = [pa.Lattice.from_settings(document(algorithm, layout, storage, *shape, kernel))
+                    for kernel in ("auto", "block", "sweep")]
+        for steps in (128, 1, 140):
+            for lattice in lattices:
+                lattice.run(steps)
+            for lattice in lattices[1:]:
+                for a, b in zip(lattices[0].macros(), lattice.macros()):
+                    np.testing.assert_array_equal(a, b)
+        for lattice in lattices:
+            lattice.close()
