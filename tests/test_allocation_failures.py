@@ -59,6 +59,46 @@ with pa.Lattice.from_settings(doc) as lat:
 """)
 
 
+IN_PLACE = """
+def kernels(algorithm, layout, h, v, storage="f64", limit=None, nth=0, group=1024):
+    memory(288 << 30)
+    if limit:
+        memory(limit)
+    fail("hipMalloc", nth)
+    doc = pa.settings(algorithm, layout, inner_h=h, inner_v=v, work_group_size=group, storage=storage, time_steps=1)
+    with pa.Lattice.from_settings(doc) as lat:
+        fail("hipMalloc", 0)
+        log()
+        lat.run(6)
+        return sorted({k.split("k_")[1].split("<")[0] for k in log() if "k_step" in k or "k_tile_s" in k or "k_march" in k})
+"""
+
+
+def test_one_lattice_schemes_stay_in_place_without_memory(runtime):
+    """npol and nsol take a second, unexpanded lattice where it is at most 1/64
+    of the device's memory and can be had; otherwise the in-place kernel of
+    their layout, storage and size."""
+    stand_in.run(runtime, IN_PLACE + """
+size = 9 * (256 + 2 + 127) * (64 + 2) * 8  # as plan_compact counts it
+assert kernels("npol", "stream", 256, 64) == ["tile_steps"]
+assert kernels("npol", "stream", 256, 64, limit=64 * size) == ["tile_steps"]
+assert kernels("npol", "stream", 256, 64, limit=64 * size - 1) == ["step_npol"]
+assert kernels("nsol", "bundle", 256, 64, limit=64 * size - 1) == ["step_nsol"]
+for nth in range(1, 9):  # any allocation of the second context
+    assert kernels("npol", "stream", 256, 64, nth=nth) == ["step_npol"], nth
+# in place, by size, layout and storage
+G = 1 << 30
+assert kernels("npol", "stream", 2048, 512, limit=G) == ["step_tile_sweep"]
+assert kernels("nsol", "bundle", 2048, 512, "f32", limit=G) == ["step_tile_sweep"]
+assert kernels("npol", "collision", 2048, 512, limit=G) == ["step_tile_staged"]
+assert kernels("nsol", "collision", 2048, 512, "f32", limit=G) == ["step_tile_staged"]
+assert kernels("npol", "collision", 512, 128, limit=G // 8) == ["step_npol"]
+assert kernels("npol", "collision", 2048, 512, "f16-shifted", limit=G) == ["step_tile_sweep"]
+memory(288 << 30)
+assert live()[0] == 0 and live()[2] == 0, live()
+""")
+
+
 @pytest.mark.parametrize("storage", ["f64", "f16-shifted"])
 def test_buffer_nodes_without_memory(runtime, storage):
     """Where the expanded lattice cannot be had, setting populations or a state
