@@ -2032,7 +2032,10 @@ static bool plan_compact(const lbm_ctx *c)
         return false;
     size_t free_bytes = 0, total = 0;
     if (hipMemGetInfo(&free_bytes, &total) != hipSuccess)
+    {
+        (void)hipGetLastError();
         return false;
+    }
     return 9ull * (c->H + 127u) * c->V * c->elem <= total / 64u;
 }
 

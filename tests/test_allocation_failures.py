@@ -86,6 +86,8 @@ assert kernels("npol", "stream", 256, 64, limit=64 * size - 1) == ["step_npol"]
 assert kernels("nsol", "bundle", 256, 64, limit=64 * size - 1) == ["step_nsol"]
 for nth in range(1, 9):  # any allocation of the second context
     assert kernels("npol", "stream", 256, 64, nth=nth) == ["step_npol"], nth
+fail("hipMemGetInfo", 1)
+assert kernels("npol", "stream", 256, 64) == ["step_npol"]
 # in place, by size, layout and storage
 G = 1 << 30
 assert kernels("npol", "stream", 2048, 512, limit=G) == ["step_tile_sweep"]
