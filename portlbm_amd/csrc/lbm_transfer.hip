@@ -25,48 +25,43 @@ constexpr size_t kSlots = 16;
 constexpr size_t kBytesPerThread = size_t(3) << 20;  // a thread costs 16 us to start: about 0.1 ms of copying
 constexpr size_t kMaxThreads = 8;
 
-// One ring for the process, used by one call at a time; a call that finds it
-// taken copies through the runtime.  It has as many slots as the largest call
-// so far could fill, 16 at most, and stays: a program that creates, runs, reads
-// and destroys one lattice after another took 250 us per 64 x 32 lattice and
-// 5.1 ms per 2048 x 512 one with a ring given back with the last object, 205 us
-// and 3.2 ms so.
+// One ring for the process, made by the first call that uses it and used by one
+// at a time; a call that finds it taken copies through the runtime.  It stays: a
+// program that creates, runs, reads and destroys one lattice after another took
+// 250 us per 64 x 32 lattice and 5.1 ms per 2048 x 512 one with a ring given
+// back with the last object, 205 us and 3.2 ms so.
 struct Ring
 {
     std::mutex use;
     int device = -1;  // whose events these are
     char *slots = nullptr;
-    size_t made = 0;  // slots, and events
     hipEvent_t ready[kSlots] = {};
 
-    // at least `want` (<= kSlots) slots
-    hipError_t create(size_t want)
+    hipError_t create()
     {
         int dev = 0;
         if (hipError_t err = hipGetDevice(&dev))
             return err;
-        if (made && dev != device)
-            return hipErrorInvalidDevice;
-        if (made >= want)
-            return hipSuccess;
-        destroy();
+        if (slots)
+            return dev == device ? hipSuccess : hipErrorInvalidDevice;
         device = dev;
-        if (hipError_t err = hipHostMalloc(reinterpret_cast<void **>(&slots), want * kSlotBytes, hipHostMallocPortable))
-        {
-            slots = nullptr;
-            return err;
-        }
-        for (size_t i = 0; i < want; ++i)
-            if (hipError_t err = hipEventCreateWithFlags(&ready[i], hipEventDisableTiming))
+        for (hipEvent_t &e : ready)
+            if (hipError_t err = hipEventCreateWithFlags(&e, hipEventDisableTiming))
             {
-                ready[i] = nullptr;
-                destroy();
+                e = nullptr;
+                drop_events();
                 return err;
             }
-        made = want;
+        if (hipError_t err = hipHostMalloc(reinterpret_cast<void **>(&slots), kSlots * kSlotBytes,
+                                           hipHostMallocPortable))
+        {
+            slots = nullptr;
+            drop_events();
+            return err;
+        }
         return hipSuccess;
     }
-    void destroy()
+    void drop_events()
     {
         for (hipEvent_t &e : ready)
         {
@@ -74,10 +69,6 @@ struct Ring
                 (void)hipEventDestroy(e);
             e = nullptr;
         }
-        if (slots)
-            (void)hipHostFree(slots);
-        slots = nullptr;
-        made = 0;
     }
 };
 
@@ -130,6 +121,11 @@ hipError_t download(const HostPiece *pieces, size_t count, hipStream_t stream)
     std::unique_lock<std::mutex> lock(r.use, std::try_to_lock);
     if (!lock.owns_lock())
         return through_runtime(pieces, count, stream);
+    if (r.create() != hipSuccess)
+    {
+        (void)hipGetLastError();
+        return through_runtime(pieces, count, stream);
+    }
     // chunks of at most a slot, over pieces that adjoin on the device
     std::vector<Chunk> chunks;
     size_t total = 0;
@@ -158,11 +154,6 @@ hipError_t download(const HostPiece *pieces, size_t count, hipStream_t stream)
         }
     }
     const size_t nc = chunks.size();
-    if (r.create(std::min(kSlots, nc)) != hipSuccess)
-    {
-        (void)hipGetLastError();
-        return through_runtime(pieces, count, stream);
-    }
     std::atomic<size_t> issued{0}, next{0};
     std::atomic<int> error{hipSuccess};
     const std::unique_ptr<std::atomic<bool>[]> emptied(new (std::nothrow) std::atomic<bool>[nc]);

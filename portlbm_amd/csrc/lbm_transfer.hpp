@@ -16,8 +16,8 @@ struct HostPiece
 };
 
 // Copies the pieces once the work enqueued on `stream` is done; returns when
-// they have arrived.  Any thread, any stream.  Its pinned staging, at most 16
-// MiB, is kept for the process.
+// they have arrived.  Any thread, any stream.  Its pinned staging, 16 MiB, is
+// made at the first call and kept for the process.
 hipError_t download(const HostPiece *pieces, size_t count, hipStream_t stream);
 
 }  // namespace lbm_dev
