@@ -321,6 +321,7 @@ hipError_t hipEventDestroy(hipEvent_t e)
 }
 hipError_t hipEventRecord(hipEvent_t e, hipStream_t) { return done(e ? hipSuccess : hipErrorInvalidHandle); }
 hipError_t hipEventSynchronize(hipEvent_t e) { return done(e ? hipSuccess : hipErrorInvalidHandle); }
+hipError_t hipEventQuery(hipEvent_t e) { return done(e ? hipSuccess : hipErrorInvalidHandle); }
 hipError_t hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t)
 {
     *ms = 1.f;
