@@ -397,11 +397,12 @@ __device__ __forceinline__ void march_wave(const StepParams &p, const uint32_t (
             }
         }
         E t[N][9];
+        C rhos[N], jxs[N], jys[N], usqs[N];
+        collide_nodes<C, Storage<S>::kPromote, Storage<S>::kFull, N>(f, C(p.omega), rhos, jxs, jys, usqs);
 #pragma unroll
         for (int i = 0; i < N; ++i)
         {
-            C rho, jx, jy, usq;
-            collide_node<C, Storage<S>::kPromote, Storage<S>::kFull>(f[i], C(p.omega), rho, jx, jy, usq);
+            const C rho = rhos[i], jx = jxs[i], jy = jys[i], usq = usqs[i];
             if constexpr (k < T)
                 uy[k][i] = N == 4 ? clamp_output(jy, p.nan_protection) : jy;
             else if ((p.write_macros || bit(i, LBM_CODE_UY_SOURCE)) && owned && bit(i, LBM_CODE_FLUID))

@@ -51,7 +51,8 @@ __device__ __forceinline__ void tile_block(const StepParams &p, const uint32_t (
         for (int d = 0; d < 9; ++d)
             pop[0][d][tid] = pop[1][d][tid] = src[at<L>(pn, uint32_t(d), p.S)];
     }
-    C f[9];
+    C fs[1][9];
+    C(&f)[9] = fs[0];
     if (fluid)
         pull<L, S>(src, pn, code, p.P, p.S, f, r3);
     for (uint32_t k = 1;; ++k)
@@ -78,8 +79,9 @@ __device__ __forceinline__ void tile_block(const StepParams &p, const uint32_t (
                 else
                     zou_he_outlet<C, Storage<S>::kPromote>(f, C(p.rho_out), u);
             }
-            C rho, jx, jy, usq;
-            collide_node<C, Storage<S>::kPromote, Storage<S>::kFull>(f, C(p.omega), rho, jx, jy, usq);
+            C rhos[1], jxs[1], jys[1], usqs[1];
+            collide_nodes<C, Storage<S>::kPromote, Storage<S>::kFull, 1>(fs, C(p.omega), rhos, jxs, jys, usqs);
+            const C rho = rhos[0], jx = jxs[0], jy = jys[0], usq = usqs[0];
             E t[9];
             node_bits<S>(f, pn, sr[k - 1u], t, 0.f);
             if (k < steps)
