@@ -26,9 +26,12 @@
 //   FP32     204 -> 104      235 -> 115      242 -> 116
 //   FP16     128 -> 106      177 -> 113      184 -> 113
 // (FP16 with stochastic rounding, cylinder channel: 160 -> 122.)
-// What bounds it at T = 4: vector instructions, 62 % of the cycles in FP64
-// (rocprofv3: 2.06e8 per launch of 557 us) with two waves per SIMD, next to
-// 2.65 GB moved per launch (4.8 TB/s).
+// What bounds it at T = 4 (rocprofv3; stream FP64 / collision FP64 / stream FP32
+// / stream FP16): vector instructions take 0.68 / 0.70 / 0.83 / 0.91 of the
+// SIMDs' cycles; 1.60 / 1.64 / 1.48 / 1.45 of the two waves that a SIMD's
+// registers hold are there, for the last round of waves is ragged; they wait
+// 0.22 / 0.26 / 0.17 / 0.11 of their time.  FP64 stream moves 2.65 GB per launch
+// (4.7 TB/s).
 
 #include "lbm_march.hpp"
 
@@ -277,9 +280,10 @@ __device__ __forceinline__ void march_wave(const StepParams &p, const uint32_t (
         else
         {
             // The copies of row j into LDS are older than the stores of the row
-            // emitted since (STORES on every row), and vector memory
-            // operations complete in order: they have landed once at most
-            // that many are in flight.
+            // emitted since (at least STORES on every row: one per 64 vectors
+            // of an array, as many again where the lattice ends inside a
+            // vector), and vector memory operations complete in order: they
+            // have landed once at most that many are in flight.
             constexpr int STORES = L == LBM_LAYOUT_COLLISION ? 4 : 6;
             asm volatile("s_waitcnt vmcnt(%0)" ::"n"(STORES) : "memory");
             const u32x4 *stage_lds = lds_of(j);
@@ -462,10 +466,11 @@ __device__ __forceinline__ void march_wave(const StepParams &p, const uint32_t (
                 last_row[d] = out[d];
     };
 
-    // The nine stores of stage T's row.  They are issued on every row, lanes
-    // with nothing to store at an offset past the row (the hardware drops
-    // them): a wait for the next row's loads can then leave exactly nine
-    // stores in flight; stores behind a branch would have to be waited for.
+    // The stores of stage T's row.  They are issued on every row, lanes with
+    // nothing to store at an offset past the row (the hardware drops them): a
+    // wait for the next row's loads can then leave them in flight (nine in the
+    // stream layout, at least STORES in the others); stores behind a branch
+    // would have to be waited for.
     auto emit = [&](auto ph, int j) {
         constexpr int P0 = decltype(ph)::value;
         const int r = j - T;

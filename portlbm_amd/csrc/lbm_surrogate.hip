@@ -61,7 +61,8 @@ inline int conv_level(int k) { return k < 8 ? k / 2 : k == 8 ? 4 : k == 13 ? 0 :
 // rows share the weights, the tiles the pixels; four waves have 4 R rows, whose
 // input with its 1-node halo is staged in LDS.
 //
-// The order of the sums is that of k.  Another order moves activations across
+// The chunks are summed in the order of k (within a chunk, FP32 sums kc + s, kc +
+// 4 + s, kc + 8 + s, kc + 12 + s for s = 0..3).  Another order moves activations across
 // BF16 rounding bounds and across the zero of a ReLU, where the gradient jumps
 // (taps before channels, with 16-byte LDS reads: no faster in FP32, and a
 // gradient up to six times as far from FP64).  A lane's four pixels of a chunk
@@ -688,10 +689,11 @@ int pack_all(lbm_surrogate *s)
 // of a convolution.  Rows of a wave share the weights and most of the halo,
 // channel tiles share the staged input: four rows and all channel tiles where
 // that leaves two blocks per compute unit (512), two rows, then one row below
-// that (two at most for more than 32 input channels, whose tile would leave one
-// block per compute unit in LDS); the channel tiles of a layer too small for
-// 512 blocks of one row get blocks of their own.  16 -> 16 channels at 256 x
-// 256, 16 samples in FP32: 136 us with one row, 74 us with four.
+// that (two at most for more than 32 input channels, in either type: 48 in FP32
+// would take 65.7 KB, above the 64 KB that a launch gets unasked); the channel
+// tiles of a layer too small for 512 blocks of one row get blocks of their own.
+// 16 -> 16 channels at 256 x 256, 16 samples in FP32: 136 us with one row, 74 us
+// with four.
 template <class F>
 void conv_shape(int Cin, int Cout, int H, int W, int B, F f)
 {
@@ -1133,7 +1135,7 @@ static int host_batch(lbm_surrogate *s, const float *inputs, const float *target
     S_TRY(hipStreamSynchronize(s->stream));
     if (!(m > 0.0))
         return lbm_set_error(LBM_ERR_INVALID_ARGUMENT, std::string(what) + ": the batch has no fluid node");
-    *norm = 1.0 / (LBM_SURROGATE_OUTPUTS * m);
+    *norm = 1.0 / (double(LBM_SURROGATE_OUTPUTS) * m);
     return LBM_OK;
 }
 
@@ -1275,7 +1277,7 @@ int lbm_surrogate_train(lbm_surrogate *s, uint32_t steps, uint32_t schedule_step
             lr = lr_min + 0.5 * (lr_max - lr_min) * (1.0 + std::cos(kPi * t));
         }
         forward(s, int(batch));
-        loss_backward(s, int(batch), 1.0 / (LBM_SURROGATE_OUTPUTS * m), s->history, int(step));
+        loss_backward(s, int(batch), 1.0 / (double(LBM_SURROGATE_OUTPUTS) * m), s->history, int(step));
         S_TRY(hipGetLastError());
         if (int rc = adam_step(s, float(lr)))
             return rc;

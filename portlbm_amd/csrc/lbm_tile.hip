@@ -13,8 +13,13 @@
 // compute unit, and a step then takes the latency of one node's pulls and
 // collision.  Measured us per step, one step per launch -> here: 256 x 64
 // FP64 stream 3.82 -> 1.25, collision 5.24 -> 1.30; 512 x 128 4.53 -> 2.12;
-// 1024 x 256 10.2 -> 4.7, collision 9.3 -> 4.9; 2048 x 512 29.5 -> 12.6.  The
+// 1024 x 256 10.2 -> 4.7, collision 9.3 -> 5.0; 2048 x 512 29.5 -> 12.6.  The
 // marching kernel takes over where HBM bounds a step (plan_fusion).
+//
+// What bounds it (rocprofv3): at 1024 x 256 in FP64 the 473 blocks of 147 KB of
+// LDS, one per compute unit, go in two rounds; compute units are busy 0.60 of
+// the time, vector instructions take 0.27 of the SIMDs' cycles, waves wait 0.47
+// of theirs.  At 1999 x 501 in BF16 vector instructions take 0.69.
 
 #include "lbm_march.hpp"
 
