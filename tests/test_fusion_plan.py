@@ -74,6 +74,17 @@ assert not wrong, wrong
 """)
 
 
+def test_two_steps_take_smaller_regions(runtime):
+    stand_in.run(runtime, """
+with pa.Lattice.from_settings(pa.settings("nptl", "collision", inner_h=1024, inner_v=256, time_steps=1)) as lat:
+    for steps, shape in ((2, "32, 16"), (3, "32, 32"), (7, "32, 32"), (2, "32, 16")):
+        log()
+        lat.run(steps)
+        launches = [k for k in log() if "k_tile_steps" in k]
+        assert launches and all(shape in k for k in launches), (steps, launches)
+""")
+
+
 @pytest.mark.parametrize("count,h,v,storage,expect", [
     (976, 64, 64, "f16-shifted", "k_batch_tiles"), (40, 700, 150, "f16-shifted", "k_batch_march"),
     (61, 256, 256, "bf16-shifted", "k_batch_tiles"), (40, 500, 150, "f32", "k_batch_march"),
