@@ -422,7 +422,11 @@ int run_persistent_steps(lbm_batch *b, uint32_t steps, int *cur, const FusePlan 
     const uint32_t grid = std::max(1u, std::min(b->ntiles, b->persistent_grid));
     for (uint32_t left = steps; left; *cur ^= 1)
     {
-        const uint32_t n = first_chunk(plan, left);
+        // Two FP64 steps leave most of a 32 x 32 region, cut for five or six of
+        // them, to its halo: one by one (300 domains of 30 x 30: 37.0 us, at once
+        // 41.6; 10 of 100 x 60 12.5, 12.6).
+        const bool pair = left == 2u && b->elem == 8 && plan.tiles && plan.shape == TileShape::k32x32;
+        const uint32_t n = pair ? 1u : first_chunk(plan, left);
         left -= n;
         if (n == 1u)
         {

@@ -98,3 +98,16 @@ with pa.Batch(docs, storage={storage!r}) as b:
     steps = [k for k in log() if "k_batch" in k]
     assert steps and all({expect!r} in k for k in steps), steps
 """)
+
+
+def test_two_steps_of_a_batch(runtime):
+    stand_in.run(runtime, """
+docs = [pa.settings("lptl", "stream", inner_h=30, inner_v=30, time_steps=1)] * 300
+for storage, steps, launches in (("f64", 2, ["k_batch_step"] * 2), ("f64", 3, ["k_batch_tiles"]),
+                                 ("f32", 2, ["k_batch_tiles"]), ("f64", 7, ["k_batch_tiles"] * 2)):
+    with pa.Batch(docs, storage=storage) as b:
+        log()
+        b.run(steps, "persistent")
+        names = [k for k in log() if "k_batch" in k]
+        assert len(names) == len(launches) and all(n in k for n, k in zip(launches, names)), (storage, steps, names)
+""")
