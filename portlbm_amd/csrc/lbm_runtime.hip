@@ -1265,6 +1265,27 @@ __global__ void k_prime_side_cols(const T *lat, T *out0, T *out1, uint32_t Vx, u
     }
 }
 
+// The nodes of an unexpanded lattice `in` to their places in the expanded
+// lattice `ex`, or back.
+template <int L, class T>
+__global__ void k_expand(T *in, T *ex, Geom gi, Geom ge, uint32_t V, uint32_t sub_v, int back)
+{
+    const uint32_t n = blockIdx.x * blockDim.x + threadIdx.x, H = gi.H;
+    if (n >= H * V)
+        return;
+    const uint32_t x = n % H, y = n / H;
+    const uint32_t p = place(x, y, gi.P, gi.X0);
+    const uint32_t e = place(map_axis(x, H - 1u, ge.sub_h, 1), map_axis(y, V - 1u, sub_v, 1), ge.P, ge.X0);
+#pragma unroll
+    for (uint32_t d = 0; d < 9; ++d)
+    {
+        if (back)
+            in[at<L>(p, d, gi.Sd)] = ex[at<L>(e, d, ge.Sd)];
+        else
+            ex[at<L>(e, d, ge.Sd)] = in[at<L>(p, d, gi.Sd)];
+    }
+}
+
 // Buffer rows: directions 0..2 from the row above, 6..8 from the row below
 // (general/buffered.hpp:74-93).  Covers the full expanded width, ghost
 // columns included.
@@ -1835,6 +1856,23 @@ struct Impl
         return LBM_OK;
     }
 
+    // The inner context's lattice into c's expanded one, or (back) both of the
+    // inner context's lattices from it.
+    static int expand(lbm_ctx *c, bool back)
+    {
+        lbm_ctx *in = c->inner;
+        LBM_HIP_TRY(hipStreamSynchronize(in->stream));
+        hipLaunchKernelGGL((k_expand<L, T>), dim3((in->N + 255u) / 256u), dim3(256), 0, c->stream,
+                           static_cast<T *>(in->lat[in->cur]), static_cast<T *>(c->lat[0]), geom(in), geom(c), c->V,
+                           c->sub_v, back ? 1 : 0);
+        LBM_HIP_TRY(hipGetLastError());
+        if (back)
+            LBM_HIP_TRY(hipMemcpyAsync(in->lat[1 - in->cur], in->lat[in->cur], in->lattice_elems * sizeof(T),
+                                       hipMemcpyDeviceToDevice, c->stream));
+        LBM_HIP_TRY(hipStreamSynchronize(c->stream));
+        return LBM_OK;
+    }
+
     // One pass of a split step (pass = enum lbm_pass); the collide pass ends
     // the step (lattice swap, iteration count).
     static int split(lbm_ctx *c, int pass, double *buf)
@@ -1980,6 +2018,7 @@ struct VTable
     int (*reduce)(lbm_ctx *, int, double *);
     int (*split)(lbm_ctx *, int, double *);
     int (*fused)(lbm_ctx *, uint32_t, bool);
+    int (*expand)(lbm_ctx *, bool);
 };
 
 template <int L, int S>
@@ -1987,7 +2026,7 @@ static VTable make_vtable()
 {
     return VTable{&Impl<L, S>::step, &Impl<L, S>::init, &Impl<L, S>::decode, &Impl<L, S>::encode,
                   &Impl<L, S>::equilibrium, &Impl<L, S>::reduce, &Impl<L, S>::split,
-                  &Impl<L, S>::fused};
+                  &Impl<L, S>::fused, &Impl<L, S>::expand};
 }
 
 template <int L>
@@ -3012,9 +3051,8 @@ static bool ensure_expanded(lbm_ctx *c)
     return false;
 }
 
-// The same before the lattice is set: at the inner one's column reference.
-// Where this fails the buffer nodes, which no step reads, stay at rest.
-static bool expanded_to_set(lbm_ctx *c)
+// The same, at the inner one's column reference.
+static bool expanded_ready(lbm_ctx *c)
 {
     if (!ensure_expanded(c))
         return false;
@@ -3036,33 +3074,47 @@ static int get_inner_state(lbm_ctx *c, char *out)
     std::memcpy(out + 12, &lattices, 4);
     const size_t lat_bytes = c->lattice_elems * c->elem;
     const bool kept = c->lat[0];
-    std::vector<char> own(in->lattice_elems * in->elem);
-    if (ensure_expanded(c))
-        LBM_HIP_TRY(hipMemcpy(out + 16, c->lat[0], lat_bytes, hipMemcpyDeviceToHost));
+    if (expanded_ready(c))
+    {
+        int rc = vtable(c).expand(c, false);
+        const hipError_t e = rc ? hipSuccess : hipMemcpy(out + 16, c->lat[0], lat_bytes, hipMemcpyDeviceToHost);
+        if (!kept)
+            drop_expanded(c);
+        if (rc)
+            return rc;
+        LBM_HIP_TRY(e);
+    }
     else
+    {
         std::memset(out + 16, 0, lat_bytes);
-    if (!kept)
-        drop_expanded(c);
-    LBM_HIP_TRY(hipStreamSynchronize(in->stream));
-    LBM_HIP_TRY(hipMemcpy(own.data(), in->lat[in->cur], own.size(), hipMemcpyDeviceToHost));
-    for_placed_runs(c, [&](size_t o, size_t x, size_t n) { std::memcpy(out + 16 + x, own.data() + o, n); });
+        std::vector<char> own(in->lattice_elems * in->elem);
+        LBM_HIP_TRY(hipStreamSynchronize(in->stream));
+        LBM_HIP_TRY(hipMemcpy(own.data(), in->lat[in->cur], own.size(), hipMemcpyDeviceToHost));
+        for_placed_runs(c, [&](size_t o, size_t x, size_t n) { std::memcpy(out + 16 + x, own.data() + o, n); });
+    }
     return get_state_tail(in, out + 16 + lat_bytes, c->ref_len);
 }
 
 static int set_inner_state(lbm_ctx *c, const char *buf, uint64_t iteration)
 {
     lbm_ctx *in = c->inner;
-    std::vector<char> own(in->lattice_elems * in->elem);
-    LBM_HIP_TRY(hipStreamSynchronize(in->stream));
-    LBM_HIP_TRY(hipMemcpy(own.data(), in->lat[0], own.size(), hipMemcpyDeviceToHost));  // padding as it is
-    for_placed_runs(c, [&](size_t o, size_t x, size_t n) { std::memcpy(own.data() + o, buf + 16 + x, n); });
-    for (void *lat : in->lat)
-        LBM_HIP_TRY(hipMemcpy(lat, own.data(), own.size(), hipMemcpyHostToDevice));
-    if (int rc = set_state_tail(in, buf + 16 + c->lattice_elems * c->elem, c->ref_len, iteration, 0))
-        return rc;
-    if (expanded_to_set(c))
-        LBM_HIP_TRY(hipMemcpy(c->lat[0], buf + 16, c->lattice_elems * c->elem, hipMemcpyHostToDevice));
-    return LBM_OK;
+    const size_t lat_bytes = c->lattice_elems * c->elem;
+    if (expanded_ready(c))
+    {
+        LBM_HIP_TRY(hipMemcpy(c->lat[0], buf + 16, lat_bytes, hipMemcpyHostToDevice));
+        if (int rc = vtable(c).expand(c, true))
+            return rc;
+    }
+    else
+    {
+        std::vector<char> own(in->lattice_elems * in->elem);
+        LBM_HIP_TRY(hipStreamSynchronize(in->stream));
+        LBM_HIP_TRY(hipMemcpy(own.data(), in->lat[0], own.size(), hipMemcpyDeviceToHost));  // padding as it is
+        for_placed_runs(c, [&](size_t o, size_t x, size_t n) { std::memcpy(own.data() + o, buf + 16 + x, n); });
+        for (void *lat : in->lat)
+            LBM_HIP_TRY(hipMemcpy(lat, own.data(), own.size(), hipMemcpyHostToDevice));
+    }
+    return set_state_tail(in, buf + 16 + lat_bytes, c->ref_len, iteration, 0);
 }
 
 int lbm_get_state(lbm_ctx *c, void *buf, size_t bytes)
@@ -3128,28 +3180,26 @@ int lbm_get_populations(lbm_ctx *c, double *values, size_t count)
     if (c->inner)
     {
         return with_host_memory("lbm_get_populations", [&]() -> int {
+            const bool kept = c->lat[0];
+            if (expanded_ready(c))
+            {
+                int rc = vtable(c).expand(c, false);
+                if (!rc)
+                    rc = read_populations(c, values);
+                if (!kept)
+                    drop_expanded(c);
+                return rc;
+            }
             const size_t M = size_t(c->H) * c->V;
             std::vector<double> own(9 * M);
             if (int rc = lbm_get_populations(c->inner, own.data(), own.size()))
                 return rc;
+            static const double w[9] = {1.0 / 36, 1.0 / 9, 1.0 / 36, 1.0 / 9, 4.0 / 9,
+                                        1.0 / 9,  1.0 / 36, 1.0 / 9, 1.0 / 36};
             const int layout = c->desc.layout;
-            const bool kept = c->lat[0];
-            if (ensure_expanded(c))
-            {
-                const int rc = read_populations(c, values);
-                if (!kept)
-                    drop_expanded(c);
-                if (rc)
-                    return rc;
-            }
-            else
-            {
-                static const double w[9] = {1.0 / 36, 1.0 / 9, 1.0 / 36, 1.0 / 9, 4.0 / 9,
-                                            1.0 / 9,  1.0 / 36, 1.0 / 9, 1.0 / 36};
-                for (uint32_t d = 0; d < 9; ++d)
-                    for (size_t e = 0; e < c->N; ++e)
-                        values[flat_index(layout, e, d, c->N)] = w[d];
-            }
+            for (uint32_t d = 0; d < 9; ++d)
+                for (size_t e = 0; e < c->N; ++e)
+                    values[flat_index(layout, e, d, c->N)] = w[d];
             for (uint32_t d = 0; d < 9; ++d)
                 for_runs(c, [&](size_t u, size_t e, size_t k) {
                     for (size_t i = 0; i < k; ++i)
@@ -3167,11 +3217,16 @@ int lbm_set_populations(lbm_ctx *c, const double *values, size_t count)
         return fail(LBM_ERR_INVALID_ARGUMENT, "lbm_set_populations: null argument");
     if (c->inner)
     {
+        if (!c->inner->initialized)
+            return fail(LBM_ERR_STATE, "lbm_set_populations: call lbm_init_populations first");
+        if (count != 9ull * c->N)
+            return fail(LBM_ERR_INVALID_ARGUMENT, "lbm_set_populations: count must be 9 * expanded node count");
         return with_host_memory("lbm_set_populations", [&]() -> int {
-            if (!c->inner->initialized)
-                return fail(LBM_ERR_STATE, "lbm_set_populations: call lbm_init_populations first");
-            if (count != 9ull * c->N)
-                return fail(LBM_ERR_INVALID_ARGUMENT, "lbm_set_populations: count must be 9 * expanded node count");
+            if (expanded_ready(c))
+            {
+                const int rc = write_populations(c, values);
+                return rc ? rc : vtable(c).expand(c, true);
+            }
             const size_t M = size_t(c->H) * c->V;
             const int layout = c->desc.layout;
             std::vector<double> own(9 * M);
@@ -3180,9 +3235,7 @@ int lbm_set_populations(lbm_ctx *c, const double *values, size_t count)
                     for (size_t i = 0; i < k; ++i)
                         own[flat_index(layout, u + i, d, M)] = values[flat_index(layout, e + i, d, c->N)];
                 });
-            if (int rc = lbm_set_populations(c->inner, own.data(), own.size()))
-                return rc;
-            return expanded_to_set(c) ? write_populations(c, values) : LBM_OK;
+            return lbm_set_populations(c->inner, own.data(), own.size());
         });
     }
     if (!c->initialized)

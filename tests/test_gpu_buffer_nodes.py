@@ -64,3 +64,21 @@ def test_fields_past_the_changes_of_the_column_reference(algorithm, storage, lay
                     np.testing.assert_array_equal(a, b)
         for lattice in lattices:
             lattice.close()
+
+
+@pytest.mark.parametrize("storage", ["f16-shifted", "bf16-shifted"])
+@pytest.mark.parametrize("algorithm", ["npol", "nsol"])
+def test_buffer_nodes_past_the_changes_of_the_column_reference(algorithm, storage):
+    """Nodes that no step writes are read at the reference of the time."""
+    docs = [document(algorithm, "stream", storage, 131, 77, 64, kernel) for kernel in ("auto", "sweep")]
+    phase = pa.build_phase(docs[0])
+    auto, place = (pa.Lattice(pa.desc_from_settings(doc), phase) for doc in docs)
+    slots = (auto.N * np.arange(9)[:, None] + np.nonzero(phase != 1)[0]).ravel()
+    with auto, place:
+        values = auto.populations() * np.random.default_rng(3).uniform(0.99, 1.01, 9 * auto.N)
+        for lattice in (auto, place):
+            lattice.set_populations(values)
+        for steps in (100, 200):
+            for lattice in (auto, place):
+                lattice.run(steps)
+            np.testing.assert_array_equal(auto.populations()[slots], place.populations()[slots])
