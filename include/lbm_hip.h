@@ -253,7 +253,8 @@ int lbm_get_frame(lbm_ctx *ctx, double *density, double *x_velocity, double *y_v
  * set to (lbm_set_populations, lbm_set_state; the rest state before; in place
  * a split step refreshes them).  On the unexpanded lattice the first call that
  * sets them takes a second, expanded one to keep them in, until
- * lbm_init_populations; where there is no memory for it they stay at rest. */
+ * lbm_init_populations; where there is no memory for it they stay at rest.
+ * Reading the lattice or its state before that takes one for the call. */
 int lbm_get_populations(lbm_ctx *ctx, double *values, size_t count);
 int lbm_set_populations(lbm_ctx *ctx, const double *values, size_t count);
 

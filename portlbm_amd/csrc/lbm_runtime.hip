@@ -129,7 +129,8 @@ struct lbm_ctx
     // done by this context on the unexpanded lattice; the outer one converts
     // what callers hand over and receive in the expanded order.  Its own lat[0]
     // holds what its buffer nodes were set to, from the first time that a
-    // caller sets them (ensure_expanded).
+    // caller sets them (ensure_expanded); a read takes and frees one where
+    // there is none.
     lbm_ctx *inner = nullptr;
     std::vector<int8_t> outer_phase;  // the expanded node types, as set
     // 16-bit forms: rho_ref per unexpanded column (Hx + 64 floats, the tail
@@ -1266,7 +1267,8 @@ __global__ void k_prime_side_cols(const T *lat, T *out0, T *out1, uint32_t Vx, u
 }
 
 // The nodes of an unexpanded lattice `in` to their places in the expanded
-// lattice `ex`, or back.
+// lattice `ex`, or back.  Bound by the link to the host around it: at 4096 x
+// 1024 FP64 lbm_get_populations takes 23 ms, converted on the host 246.
 template <int L, class T>
 __global__ void k_expand(T *in, T *ex, Geom gi, Geom ge, uint32_t V, uint32_t sub_v, int back)
 {
